@@ -17,8 +17,8 @@
 //   vgemm            one workgroup per (function-block pair I <= J, split):
 //                    acc += Phi_I Z_J^T + Z_I Phi_J^T over the batches where
 //                    both blocks are live (MFMA-bound).
-// and once per build: vreduce (split sum + un-permute + mirror) and the FP64
-// energy / electron-count reduction.
+// and once per build: finish (split sum + un-permute + mirror, and the FP64
+// energy / electron-count sums).
 #include <algorithm>
 
 #include "nkx_internal.hpp"
@@ -327,11 +327,13 @@ constexpr int HP = 32;      // points per LDS stage
 constexpr int LDP = HP + 1; // padded row
 
 // blockIdx.x = (zs * nsplit + split) * npairs + pair; Z is tile array
-// zbase + zs, and the partials go to vpart + zs * nsplit * npairs * FB * FB.
+// zbase + zs, and the partials go to vpart + zs * nsplit * npairs * FB * FB:
+// written by the first chunk of a build, added to by the later ones.
 __global__ void __launch_bounds__(256) vgemm_f64(
     int npairs, int nsplit, const int *__restrict__ pair_I, const int *__restrict__ pair_J,
     const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1, int64_t s0,
-    int narr, int zbase, const double *__restrict__ tiles, double *__restrict__ vpart) {
+    int narr, int zbase, int first, const double *__restrict__ tiles,
+    double *__restrict__ vpart) {
   const int p = blockIdx.x % npairs;
   const int split = (blockIdx.x / npairs) % nsplit;
   const int zs = blockIdx.x / (npairs * nsplit);
@@ -394,46 +396,43 @@ __global__ void __launch_bounds__(256) vgemm_f64(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int mu = 16 * wv + 4 * r + q, nu = 16 * j + l16;
-      out[mu * FB + nu] += acc[j][r];
+      out[mu * FB + nu] = first ? acc[j][r] : out[mu * FB + nu] + acc[j][r];
     }
 }
 
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) vreduce_kernel(int npairs, int nsplit,
-                                                      const int *__restrict__ pair_I,
-                                                      const int *__restrict__ pair_J,
-                                                      const int *__restrict__ fperm, MolTab mt,
-                                                      const int *__restrict__ mol_nbf,
-                                                      const double *__restrict__ vpart,
-                                                      double *const *__restrict__ Vmol) {
-  const int p = blockIdx.x;
-  const int I = pair_I[p], J = pair_J[p];
-  const int mol = mt.blk_mol[I];
-  const int nbf = mol_nbf[mol];
-  double *V = Vmol[mol];
-  const int lI = mt.blk_local[I], lJ = mt.blk_local[J];
-  for (int e = threadIdx.x; e < FB * FB; e += 256) {
-    const int mu = e / FB, nu = e % FB;
-    if (I == J && mu > nu) continue;
-    const int i = lI * FB + mu, j = lJ * FB + nu;
-    if (i >= nbf || j >= nbf) continue;
-    double v = 0.0;
-    for (int s = 0; s < nsplit; ++s) v += vpart[((int64_t)s * npairs + p) * (FB * FB) + e];
-    const int oi = fperm[I * FB + mu], oj = fperm[J * FB + nu];
-    V[(int64_t)oi * nbf + oj] = v;
-    V[(int64_t)oj * nbf + oi] = v;
-  }
-}
+// End of a build, one launch: the V tiles (sum of the split partials,
+// un-permutation, mirror image) and the per-molecule E and N sums.
+//
+// Bound by reading the partials once.  Workgroup (pair p, row mu) of the first
+// 64 npairs nz ones: wave k sums splits [k ns / 4, (k + 1) ns / 4) of the row's
+// 64 elements with 16 loads in flight, and the four sums are added in wave
+// order.  One workgroup per whole pair, a serial sum per thread, left the chip
+// empty and took 1302 us on benzene (3 pairs, 335 splits, 33 MB) and 1835 us
+// on 32 waters (91 pairs, 293 splits, 0.87 GB); now 11.5 us and 179 us (4.9
+// TB/s).  The last nmol workgroups sum the per-batch (E, N_alpha, N_beta)
+// triples of a molecule in a fixed order, eight loads ahead (60 us on 32
+// waters as a launch of its own, 22 us on benzene).
+constexpr int RSEG = 4;  // split segments (waves) per row
 
-// Fixed-order sum of the per-batch (E, N_alpha, N_beta) triples, one
-// workgroup per molecule over its batches.
-__global__ void __launch_bounds__(256) en_reduce_kernel(MolTab mt, const double *__restrict__ en,
-                                                        double *__restrict__ out) {
-  __shared__ double sv[3][256];
-  const int mol = blockIdx.x;
+// sum over batches b0 + thread, + 256, ..., then a fixed tree
+__device__ __forceinline__ void en_reduce(MolTab mt, int mol, const double *__restrict__ en,
+                                          double *__restrict__ out, double (*sv)[256]) {
   const int64_t b0 = mt.b0[mol], b1 = b0 + mt.nb[mol];
   double v[3] = {0.0, 0.0, 0.0};
-  for (int64_t b = b0 + threadIdx.x; b < b1; b += 256)
+  int64_t b = b0 + threadIdx.x;
+  for (; b + 7 * 256 < b1; b += 8 * 256) {
+    double t[8][3];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) t[u][c] = en[3 * (b + 256 * u) + c];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[c] += t[u][c];
+  }
+  for (; b < b1; b += 256)
     for (int c = 0; c < 3; ++c) v[c] += en[3 * b + c];
   for (int c = 0; c < 3; ++c) sv[c][threadIdx.x] = v[c];
   __syncthreads();
@@ -444,6 +443,49 @@ __global__ void __launch_bounds__(256) en_reduce_kernel(MolTab mt, const double 
   }
   if (threadIdx.x == 0)
     for (int c = 0; c < 3; ++c) out[3 * mol + c] = sv[c][0];
+}
+
+__global__ void __launch_bounds__(256) finish_kernel(
+    int npairs, int nsplit, int nz, const int *__restrict__ pair_I,
+    const int *__restrict__ pair_J, const int *__restrict__ fperm, MolTab mt, int nmol,
+    const int *__restrict__ mol_nbf, const double *__restrict__ vpart,
+    double *const *__restrict__ Vmol, const double *__restrict__ en, double *__restrict__ enout) {
+  __shared__ double sv[3][256];
+  const int64_t nv = (int64_t)npairs * nz * FB;
+  if ((int64_t)blockIdx.x >= nv) {
+    en_reduce(mt, (int)(blockIdx.x - nv), en, enout, sv);
+    return;
+  }
+  const int mu = blockIdx.x & (FB - 1);
+  const int p = (int)(blockIdx.x / FB) % npairs, zs = (int)(blockIdx.x / FB) / npairs;
+  const int I = pair_I[p], J = pair_J[p];
+  const int mol = mt.blk_mol[I];
+  const int nbf = mol_nbf[mol];
+  const int i = mt.blk_local[I] * FB + mu;
+  if (i >= nbf) return;  // uniform: a padding row
+  const int nu = threadIdx.x & (FB - 1), seg = threadIdx.x / FB;
+  const int64_t st = (int64_t)npairs * (FB * FB);
+  const double *src = vpart + ((int64_t)zs * nsplit * npairs + p) * (FB * FB) + mu * FB + nu;
+  int s = (int)((int64_t)seg * nsplit / RSEG);
+  const int s1 = (int)((int64_t)(seg + 1) * nsplit / RSEG);
+  double v = 0.0;
+  for (; s + 16 <= s1; s += 16) {
+    double t[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) t[u] = src[(s + u) * st];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v += t[u];
+  }
+  for (; s < s1; ++s) v += src[s * st];
+  sv[0][threadIdx.x] = v;
+  __syncthreads();
+  const int j = mt.blk_local[J] * FB + nu;
+  if (seg || j >= nbf || (I == J && mu > nu)) return;
+  v = ((sv[0][nu] + sv[0][FB + nu]) + sv[0][2 * FB + nu]) + sv[0][3 * FB + nu];
+  const int oi = fperm[I * FB + mu], oj = fperm[J * FB + nu];
+  double *V = Vmol[(int64_t)zs * nmol + mol];
+  V[(int64_t)oi * nbf + oj] = v;
+  V[(int64_t)oj * nbf + oi] = v;
 }
 
 // Zero fill (stream-ordered kernel, also valid inside a captured graph).
@@ -534,25 +576,29 @@ void vk_zoverlap(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr
 }
 
 void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
-              int narr, int nz, const double *tiles, double *vpart) {
+              int narr, int nz, bool first, const double *tiles, double *vpart) {
   if (b1 <= b0 || pl.npairs == 0) return;
   hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)(pl.npairs * nsplit * nz)), dim3(256), 0, s,
                      pl.npairs, nsplit, pl.pair_I.p, pl.pair_J.p, pl.tile_slot.p, pl.tab(), b0, b1,
-                     s0, narr, narr - nz, tiles, vpart);
+                     s0, narr, narr - nz, first ? 1 : 0, tiles, vpart);
   NKX_HIP_CHECK(hipGetLastError());
 }
 
-void vk_vreduce(hipStream_t s, const Plan &pl, int nsplit, const double *vpart,
-                double *const *Vmol_dev, const int *mol_nbf_dev) {
-  if (pl.npairs == 0) return;
-  hipLaunchKernelGGL(vreduce_kernel, dim3(pl.npairs), dim3(256), 0, s, pl.npairs, nsplit,
-                     pl.pair_I.p, pl.pair_J.p, pl.fperm_d.p, pl.tab(), mol_nbf_dev, vpart,
-                     Vmol_dev);
+void vk_finish(hipStream_t s, const Plan &pl, int nsplit, int nz, const double *vpart,
+               double *const *Vmol_dev, const double *en, double *enout) {
+  const int64_t nv = (int64_t)pl.npairs * nz * FB;
+  const int64_t nwg = nv + (en ? pl.nmol : 0);
+  if (nwg == 0) return;
+  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "reduction grid too large");
+  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)nwg), dim3(256), 0, s, pl.npairs, nsplit, nz,
+                     pl.pair_I.p, pl.pair_J.p, pl.fperm_d.p, pl.tab(), pl.nmol, pl.mol_nbf.p,
+                     vpart, Vmol_dev, en, enout);
   NKX_HIP_CHECK(hipGetLastError());
 }
 
 void vk_en_reduce(hipStream_t s, const Plan &pl, const double *en, double *out) {
-  hipLaunchKernelGGL(en_reduce_kernel, dim3(pl.nmol), dim3(256), 0, s, pl.tab(), en, out);
+  hipLaunchKernelGGL(finish_kernel, dim3(pl.nmol), dim3(256), 0, s, 0, 0, 0, nullptr, nullptr,
+                     nullptr, pl.tab(), pl.nmol, nullptr, nullptr, nullptr, en, out);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -359,7 +359,8 @@ template <int NPROD>
 __global__ void __launch_bounds__(256) vgemm_mixed(
     int npairs, int nsplit, const int *__restrict__ pair_I, const int *__restrict__ pair_J,
     const int *__restrict__ tile_slot, int64_t nb, int64_t b0, int64_t b1, int64_t s0,
-    int gga, const unsigned short *__restrict__ store, double *__restrict__ vpart) {
+    int gga, int first, const unsigned short *__restrict__ store,
+    double *__restrict__ vpart) {
   const int p = blockIdx.x % npairs;
   const int split = blockIdx.x / npairs;
   const int I = pair_I[p], J = pair_J[p];
@@ -413,7 +414,7 @@ __global__ void __launch_bounds__(256) vgemm_mixed(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int mu = 16 * wv + 4 * q + r, nu = 16 * j + l16;
-      out[mu * FB + nu] += acc64[j][r];
+      out[mu * FB + nu] = first ? acc64[j][r] : out[mu * FB + nu] + acc64[j][r];
     }
 }
 
@@ -451,16 +452,16 @@ void vkb_density(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, c
 }
 
 void vkb_vgemm(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
-               int nsplit, int gga, const uint16_t *store, double *vpart) {
+               int nsplit, int gga, bool first, const uint16_t *store, double *vpart) {
   if (b1 <= b0 || pl.npairs == 0) return;
   if (nprod == 3)
     hipLaunchKernelGGL(vgemm_mixed<3>, dim3((unsigned)(pl.npairs * nsplit)), dim3(256), 0, s,
                        pl.npairs, nsplit, pl.pair_I.p, pl.pair_J.p, pl.tile_slot.p, pl.nb, b0,
-                       b1, s0, gga, store, vpart);
+                       b1, s0, gga, first ? 1 : 0, store, vpart);
   else
     hipLaunchKernelGGL(vgemm_mixed<6>, dim3((unsigned)(pl.npairs * nsplit)), dim3(256), 0, s,
                        pl.npairs, nsplit, pl.pair_I.p, pl.pair_J.p, pl.tile_slot.p, pl.nb, b0,
-                       b1, s0, gga, store, vpart);
+                       b1, s0, gga, first ? 1 : 0, store, vpart);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -851,12 +851,14 @@ __global__ void __launch_bounds__(256) z_slots_i8(int64_t s0, const int *__restr
 // batch starts (used in the second phase) and F_I of the next batch between
 // the phases (F_I is dead by then).  Each element sums its batches in
 // ascending order, F_I Z_J^T before Z_I F_J^T within a batch, as in the
-// one-pair kernel.  Each tile is added into vpart at its pair index.
+// one-pair kernel.  Each tile goes to vpart at its pair index (written by
+// the first chunk of a build, added by the later ones).
 __global__ void __launch_bounds__(512) vgemm_i8(
     int nsp, int nsplit, const int4 *__restrict__ sp_blk, const int4 *__restrict__ sp_pidx,
     int npairs, const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1,
     int64_t s0, int gga, const signed char *__restrict__ store,
-    const signed char *__restrict__ zbase, int64_t zstride, double *__restrict__ vpart) {
+    const signed char *__restrict__ zbase, int64_t zstride, int first,
+    double *__restrict__ vpart) {
   // split-major: the super-pairs of one split run together and walk the same
   // batches, sharing each batch's slots in the caches
   const int sp = blockIdx.x % nsp;
@@ -1045,7 +1047,7 @@ __global__ void __launch_bounds__(512) vgemm_i8(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int mu = 32 * wh + 16 * g + 4 * q + r, nu = 16 * j + l16;
-        out[mu * FB + nu] += v64[g][j][r];
+        out[mu * FB + nu] = first ? v64[g][j][r] : out[mu * FB + nu] + v64[g][j][r];
       }
 }
 
@@ -1179,7 +1181,8 @@ void vkm_density_functional(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, c
 }
 
 void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
-               int gga, const signed char *store, double *vpart, const signed char *zstore_b) {
+               int gga, bool first, const signed char *store, double *vpart,
+               const signed char *zstore_b) {
   if (b1 <= b0 || pl.nspairs == 0) return;
   // Z sections: each slot's own, or (second spin) SEC-strided in zstore_b
   const signed char *zbase = zstore_b ? zstore_b : store + OFF_Z;
@@ -1187,7 +1190,8 @@ void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
   hipLaunchKernelGGL(vgemm_i8, dim3((unsigned)(pl.nspairs * nsplit)), dim3(512), 0, s,
                      pl.nspairs, nsplit, reinterpret_cast<const int4 *>(pl.sp_blk.p),
                      reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.npairs, pl.tile_slot.p,
-                     pl.tab(), b0, b1, s0, gga, store, zbase, zstride, vpart);
+                     pl.tab(), b0, b1, s0, gga, store, zbase, zstride, first ? 1 : 0,
+                     vpart);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -126,6 +126,7 @@ struct Plan {
   DevBuf<int> b_off, b_fbl, slot_b;  // slot s = CSR position; slot_b[s] = its batch
   // function-block pairs (I <= J, same molecule) with a common live batch
   int npairs = 0;
+  bool pairs_full = false;        // every block pair of every molecule is kept
   std::vector<int> pair_I_h, pair_J_h;
   DevBuf<int> pair_I, pair_J;
   // 2 x 2 super-pairs of blocks (one molecule) for the int8 V contraction:

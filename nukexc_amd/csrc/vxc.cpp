@@ -377,6 +377,9 @@ void upload_plan(Plan &pl, const std::vector<PlanPart> &parts, hipStream_t s) {
   pl.nslots = nslots;
   pl.pairs_kept = nslots;
   pl.npairs = (int)pl.pair_I_h.size();
+  int64_t all_pairs = 0;
+  for (const PlanPart &pt : parts) all_pairs += (int64_t)pt.nfb * (pt.nfb + 1) / 2;
+  pl.pairs_full = pl.npairs == all_pairs;
   pl.work_nb2g = nb2g;
   pl.work_nbg = nbg;
   pl.P_total = poff;
@@ -600,12 +603,13 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
       else
         vk_gather_p(s, nbf, pl.mol_ld_h[m], fp, Pm,
                     ws.Pd.p + (size_t)sp * pl.P_total + pl.mol_P_off_h[m]);
-      vk_fill0(s, V[(size_t)sp * nmol + m], (int64_t)nbf * nbf);
+      // the elements of block pairs without a common batch are never written
+      if (!pl.pairs_full) vk_fill0(s, V[(size_t)sp * nmol + m], (int64_t)nbf * nbf);
     }
-  vk_fill0(s, ws.vpart.p, (int64_t)(nspin * vsz));
   tm.end(t, s);
   for_each_chunk(pl, b.slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
     const int ig = b.gga ? 1 : 0;
+    const bool first = b0 == 0;  // the V partials are written, then added to
     int tt = tm.begin(kStageColloc, s);
     if (bf16)
       vkb_colloc(s, s0, s1, pl, ig, bstore);
@@ -640,20 +644,19 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
     }
     tt = tm.begin(kStageVgemm, s);
     if (bf16)
-      vkb_vgemm(s, 6, b0, b1, s0, pl, nsplit, ig, bstore, ws.vpart.p);
+      vkb_vgemm(s, 6, b0, b1, s0, pl, nsplit, ig, first, bstore, ws.vpart.p);
     else if (mixed) {
-      vkm_vgemm(s, b0, b1, s0, pl, nsplit, ig, ws.mstore.p, ws.vpart.p);
+      vkm_vgemm(s, b0, b1, s0, pl, nsplit, ig, first, ws.mstore.p, ws.vpart.p);
       if (nspin == 2)
-        vkm_vgemm(s, b0, b1, s0, pl, nsplit, ig, ws.mstore.p, ws.vpart.p + vsz, ws.zstore_b.p);
+        vkm_vgemm(s, b0, b1, s0, pl, nsplit, ig, first, ws.mstore.p, ws.vpart.p + vsz,
+                  ws.zstore_b.p);
     }
     else
-      vk_vgemm(s, b0, b1, s0, pl, nsplit, narr, nspin, ws.tiles64.p, ws.vpart.p);
+      vk_vgemm(s, b0, b1, s0, pl, nsplit, narr, nspin, first, ws.tiles64.p, ws.vpart.p);
     tm.end(tt, s);
   });
   t = tm.begin(kStageFinal, s);
-  for (int sp = 0; sp < nspin; ++sp)
-    vk_vreduce(s, pl, nsplit, ws.vpart.p + sp * vsz, Vtab + (size_t)sp * nmol, pl.mol_nbf.p);
-  vk_en_reduce(s, pl, ws.blockEN.p, ws.red.p);
+  vk_finish(s, pl, nsplit, nspin, ws.vpart.p, Vtab, ws.blockEN.p, ws.red.p);
   tm.end(t, s);
   tm.end(t_build, s);
   NKX_HIP_CHECK(hipMemcpyAsync(en_dst, ws.red.p, (size_t)3 * nmol * sizeof(double),
@@ -1126,15 +1129,14 @@ void overlap_build(Ctx &c, double *S) {
   ws.tiles64.reserve((size_t)slots_alloc * narr * FB * PT);
   const size_t vsz = (size_t)nsplit * std::max(pl.npairs, 1) * FB * FB;
   ws.vpart.reserve(vsz);
-  vk_fill0(s, ws.vpart.p, (int64_t)vsz);
   vk_fill0(s, S, (int64_t)pl.nbf * pl.nbf);
   double *const *Stab = upload_ptrs(c, std::vector<double *>{S});
   for_each_chunk(pl, slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
     vk_colloc(s, s0, s1, pl, narr, 0, ws.tiles64.p);
     vk_zoverlap(s, s0, s1, pl, narr, ws.tiles64.p);
-    vk_vgemm(s, b0, b1, s0, pl, nsplit, narr, 1, ws.tiles64.p, ws.vpart.p);
+    vk_vgemm(s, b0, b1, s0, pl, nsplit, narr, 1, b0 == 0, ws.tiles64.p, ws.vpart.p);
   });
-  vk_vreduce(s, pl, nsplit, ws.vpart.p, Stab, pl.mol_nbf.p);
+  vk_finish(s, pl, nsplit, 1, ws.vpart.p, Stab, nullptr, nullptr);
   NKX_HIP_CHECK(hipStreamSynchronize(s));
 }
 

@@ -34,13 +34,15 @@ void vk_scatter_density(hipStream_t s, const Plan &pl, const double *r4, double 
 void vk_zoverlap(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr,
                  double *tiles);
 // nz Z arrays (the last nz of the narr per slot), partials for Z array k at
-// vpart + k * nsplit * npairs * 64 * 64
+// vpart + k * nsplit * npairs * 64 * 64; first: the build's first chunk, which
+// writes the partials (the later ones add to them)
 void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
-              int narr, int nz, const double *tiles, double *vpart);
-// V of molecule m is Vmol_dev[m] (device array of device pointers), its
-// function count mol_nbf_dev[m]
-void vk_vreduce(hipStream_t s, const Plan &pl, int nsplit, const double *vpart,
-                double *const *Vmol_dev, const int *mol_nbf_dev);
+              int narr, int nz, bool first, const double *tiles, double *vpart);
+// V of spin z and molecule m is Vmol_dev[z * nmol + m] (device array of device
+// pointers), from the nz sets of partials; en (may be NULL): per-batch
+// triples summed per molecule into enout as vk_en_reduce
+void vk_finish(hipStream_t s, const Plan &pl, int nsplit, int nz, const double *vpart,
+               double *const *Vmol_dev, const double *en, double *enout);
 // out[3 m + c] = (E, N_alpha, N_beta) of molecule m
 void vk_en_reduce(hipStream_t s, const Plan &pl, const double *en, double *out);
 void vk_fill0(hipStream_t s, double *x, int64_t n);
@@ -73,7 +75,7 @@ void vkm_density_functional(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, c
 // zstore_b (may be NULL): Z sections of the second spin, mixed_zsection_bytes()
 // per slot, instead of the slots' own
 void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
-               int gga, const signed char *store, double *vpart,
+               int gga, bool first, const signed char *store, double *vpart,
                const signed char *zstore_b = nullptr);
 // spin-polarised functional and Z slices of both spins (split density form):
 // Z_alpha into the slots, Z_beta into zstore_b
@@ -95,7 +97,7 @@ void vkb_density(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, c
                  const uint16_t *Ps, int gga, uint16_t *store, const XcList &xl, double *coef,
                  double *blockEN);
 void vkb_vgemm(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
-               int nsplit, int gga, const uint16_t *store, double *vpart);
+               int nsplit, int gga, bool first, const uint16_t *store, double *vpart);
 
 // nuclear gradient (kernels_grad.hip)
 // grad_basis: per batch, per-function partial sums of the basis-centre
