@@ -1,4 +1,4 @@
-// Grid partition, compaction, reference-shaped collocation / density / XC.
+// Grid partition, compaction, reference-shaped collocation, functionals.
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -412,314 +412,6 @@ void launch_functional_eval_pol(hipStream_t s, XcList xl, int64_t npts, const do
   hipLaunchKernelGGL(functional_pol_kernel, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0,
                      s, xl, npts, rho, sigma, exc, vrho, vsigma);
   NKX_HIP_CHECK(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
-// Reference-shaped density (density.hpp:150-255): psi_i = sum_mu C(mu,i)
-// Phi(mu,g), rho = sum_i f_i psi_i^2, grad rho = 2 sum_i f_i psi_i grad psi_i.
-// One thread per point; C and f staged through LDS in chunks.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) density_ref_kernel(
-    int nbf, int64_t npts, const double *__restrict__ phi, const double *__restrict__ gx,
-    const double *__restrict__ gy, const double *__restrict__ gz, int nocc,
-    const double *__restrict__ C, const double *__restrict__ f, double *rho, double *grx,
-    double *gry, double *grz, double *sigma) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = g < npts;
-  double r = 0, a = 0, b = 0, c = 0;
-  for (int i = 0; i < nocc; ++i) {
-    double p0 = 0, p1 = 0, p2 = 0, p3 = 0;
-    if (live) {
-      const double *col = C + (size_t)i * nbf;  // LayoutLeft (N_bf, N_occ)
-      const size_t base = (size_t)g * nbf;
-      for (int mu = 0; mu < nbf; ++mu) {
-        const double cm = col[mu];
-        p0 += cm * phi[base + mu];
-        if (gx) {
-          p1 += cm * gx[base + mu];
-          p2 += cm * gy[base + mu];
-          p3 += cm * gz[base + mu];
-        }
-      }
-    }
-    const double fi = f[i];
-    r += fi * p0 * p0;
-    a += fi * p1 * p0;
-    b += fi * p2 * p0;
-    c += fi * p3 * p0;
-  }
-  if (!live) return;
-  rho[g] = r;
-  if (grx) {
-    grx[g] = 2.0 * a;
-    gry[g] = 2.0 * b;
-    grz[g] = 2.0 * c;
-  }
-  if (sigma) sigma[g] = 4.0 * (a * a + b * b + c * c);
-}
-
-void launch_density_ref(hipStream_t s, int nbf, int64_t npts, const double *phi,
-                        const double *gx, const double *gy, const double *gz, int nocc,
-                        const double *C, const double *f, double *rho, double *grx,
-                        double *gry, double *grz, double *sigma) {
-  if (npts == 0) return;
-  hipLaunchKernelGGL(density_ref_kernel, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, s,
-                     nbf, npts, phi, gx, gy, gz, nocc, C, f, rho, grx, gry, grz, sigma);
-  NKX_HIP_CHECK(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
-// Reference-shaped XC assembly (compute_lda xc_integrals.hpp:73-166,
-// compute_gga :424-541): Z_mu,g = w_g (1/2 Phi v_rho + 2 (grad rho . grad Phi)
-// v_sigma) written over Phi's storage pattern, then V = Phi Z^T + (Phi Z^T)^T
-// by a split-K LDS-tiled FP64 kernel, and E = sum_g w rho eps.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) zmat_ref_kernel(int nbf, int64_t npts,
-                                                       const double *__restrict__ phi,
-                                                       const double *__restrict__ gx,
-                                                       const double *__restrict__ gy,
-                                                       const double *__restrict__ gz,
-                                                       const double *__restrict__ w,
-                                                       const double *__restrict__ rho,
-                                                       const double *__restrict__ grx,
-                                                       const double *__restrict__ gry,
-                                                       const double *__restrict__ grz,
-                                                       const double *__restrict__ vrho,
-                                                       const double *__restrict__ vsig,
-                                                       const double *__restrict__ exc,
-                                                       double *Z, double *EN) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  double econ = 0.0;
-  if (e < (int64_t)nbf * npts) {
-    const int mu = (int)(e % nbf);
-    const int64_t g = e / nbf;
-    double z = 0.5 * phi[e] * vrho[g];
-    if (gx) z += 2.0 * vsig[g] * (grx[g] * gx[e] + gry[g] * gy[e] + grz[g] * gz[e]);
-    Z[e] = w[g] * z;
-    if (mu == 0) econ = w[g] * rho[g] * exc[g];
-  }
-  // block reduction of the energy terms
-  for (int o = 32; o > 0; o >>= 1) econ += __shfl_down(econ, o);
-  __shared__ double part[4];
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = econ;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(EN, part[0] + part[1] + part[2] + part[3]);
-}
-
-// V(mu, nu) += sum_g A(mu, g) B(nu, g) with A, B LayoutLeft (nbf, npts):
-// 64 x 64 output tile per block, 16 x 16 threads with 4 x 4 micro-tiles,
-// K split over blockIdx.z, partial tiles added with FP64 atomics.
-__global__ void __launch_bounds__(256) gemm_nt_ref_kernel(int nbf, int64_t npts,
-                                                          const double *__restrict__ A,
-                                                          const double *__restrict__ B,
-                                                          double *V, int64_t kchunk) {
-  __shared__ double As[16][65];
-  __shared__ double Bs[16][65];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-  const int64_t k0 = (int64_t)blockIdx.z * kchunk;
-  const int64_t k1 = k0 + kchunk < npts ? k0 + kchunk : npts;
-  double acc[4][4] = {};
-  for (int64_t kk = k0; kk < k1; kk += 16) {
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      const int kr = e / 64, mc = e % 64;
-      const int64_t g = kk + kr;
-      const bool ok = g < k1;
-      As[kr][mc] = (ok && m0 + mc < nbf) ? A[g * nbf + m0 + mc] : 0.0;
-      Bs[kr][mc] = (ok && n0 + mc < nbf) ? B[g * nbf + n0 + mc] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      double a[4], b[4];
-      for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
-      for (int j = 0; j < 4; ++j) b[j] = Bs[k][tx * 4 + j];
-      for (int i = 0; i < 4; ++i)
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-    }
-    __syncthreads();
-  }
-  for (int i = 0; i < 4; ++i)
-    for (int j = 0; j < 4; ++j) {
-      const int mu = m0 + ty * 4 + i, nu = n0 + tx * 4 + j;
-      if (mu < nbf && nu < nbf) atomicAdd(&V[(size_t)mu * nbf + nu], acc[i][j]);
-    }
-}
-
-__global__ void symmetrize_kernel(int nbf, const double *__restrict__ Vb, double *V) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)nbf * nbf) return;
-  const int i = (int)(e / nbf), j = (int)(e % nbf);
-  V[e] = Vb[(size_t)i * nbf + j] + Vb[(size_t)j * nbf + i];
-}
-
-// Spin-polarised Z for spin s (compute_lsda xc_integrals.hpp:218-240,
-// compute_gga_lsda :653-712): Z = w (1/2 Phi vrho_s + vec_s . grad Phi) with
-// vec_a = 2 vsigma_aa grad rho_a + vsigma_ab grad rho_b (and a <-> b).
-// gr holds grad rho_a (x, y, z) then grad rho_b (x, y, z), npts each.
-__global__ void __launch_bounds__(256) zmat_pol_kernel(int nbf, int64_t npts, int spin,
-                                                       const double *__restrict__ phi,
-                                                       const double *__restrict__ gx,
-                                                       const double *__restrict__ gy,
-                                                       const double *__restrict__ gz,
-                                                       const double *__restrict__ w,
-                                                       const double *__restrict__ gr,
-                                                       const double *__restrict__ vrho,
-                                                       const double *__restrict__ vsig,
-                                                       double *Z) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)nbf * npts) return;
-  const int64_t g = e / nbf;
-  double z = 0.5 * phi[e] * vrho[2 * g + spin];
-  if (gx) {
-    const double *gs = gr + (int64_t)(3 * spin) * npts, *go = gr + (int64_t)(3 - 3 * spin) * npts;
-    const double vss = 2.0 * vsig[3 * g + 2 * spin], vab = vsig[3 * g + 1];
-    const double vx = vss * gs[g] + vab * go[g];
-    const double vy = vss * gs[npts + g] + vab * go[npts + g];
-    const double vz = vss * gs[2 * npts + g] + vab * go[2 * npts + g];
-    z += vx * gx[e] + vy * gy[e] + vz * gz[e];
-  }
-  Z[e] = w[g] * z;
-}
-
-// rho (2g + s) and sigma (3g + k) interleaved from per-spin densities and
-// gradients; energy sum_g w (rho_a + rho_b) exc accumulated by a later pass.
-__global__ void __launch_bounds__(256) pack_pol_kernel(int64_t npts, const double *__restrict__ ra,
-                                                       const double *__restrict__ rb,
-                                                       const double *__restrict__ gr,
-                                                       double *rho2, double *sig3) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= npts) return;
-  rho2[2 * g] = ra[g];
-  rho2[2 * g + 1] = rb[g];
-  if (sig3) {
-    const double ax = gr[g], ay = gr[npts + g], az = gr[2 * npts + g];
-    const double bx = gr[3 * npts + g], by = gr[4 * npts + g], bz = gr[5 * npts + g];
-    sig3[3 * g] = ax * ax + ay * ay + az * az;
-    sig3[3 * g + 1] = ax * bx + ay * by + az * bz;
-    sig3[3 * g + 2] = bx * bx + by * by + bz * bz;
-  }
-}
-
-__global__ void __launch_bounds__(256) energy_pol_kernel(int64_t npts, const double *__restrict__ w,
-                                                         const double *__restrict__ rho2,
-                                                         const double *__restrict__ exc,
-                                                         double *EN) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  double e = 0.0;
-  if (g < npts) e = w[g] * (rho2[2 * g] + rho2[2 * g + 1]) * exc[g];
-  for (int o = 32; o > 0; o >>= 1) e += __shfl_down(e, o);
-  __shared__ double part[4];
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = e;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(EN, part[0] + part[1] + part[2] + part[3]);
-}
-
-// V = Phi Z^T + (Phi Z^T)^T for one spin channel.
-static void assemble_v(hipStream_t s, int nbf, int64_t npts, const double *phi, const double *Z,
-                       double *Vb, double *V) {
-  NKX_HIP_CHECK(hipMemsetAsync(Vb, 0, (size_t)nbf * nbf * sizeof(double), s));
-  if (npts > 0) {
-    const int tiles = (nbf + 63) / 64;
-    int64_t nsplit = std::max<int64_t>(1, std::min<int64_t>(512 / (tiles * tiles) + 1,
-                                                            (npts + 1023) / 1024));
-    const int64_t kchunk = ((npts + nsplit - 1) / nsplit + 15) / 16 * 16;
-    nsplit = (npts + kchunk - 1) / kchunk;
-    hipLaunchKernelGGL(gemm_nt_ref_kernel, dim3(tiles, tiles, (unsigned)nsplit), dim3(256), 0, s,
-                       nbf, npts, phi, Z, Vb, kchunk);
-    NKX_HIP_CHECK(hipGetLastError());
-  }
-  const int64_t nn = (int64_t)nbf * nbf;
-  hipLaunchKernelGGL(symmetrize_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, nbf,
-                     Vb, V);
-  NKX_HIP_CHECK(hipGetLastError());
-}
-
-void xc_from_collocation_pol(Ctx &c, int nbf, int64_t npts, const double *phi, const double *gx,
-                             const double *gy, const double *gz, const double *w, int nocca,
-                             const double *Ca, const double *fa, int noccb, const double *Cb,
-                             const double *fb, const XcList &xl, bool gga, double *E,
-                             double *Va, double *Vb) {
-  hipStream_t s = c.stream;
-  const bool grad = gga && gx;
-  // per-point scratch: ra, rb, grad (6), rho2 (2), sig3 (3), exc, vrho (2),
-  // vsig (3) = 19 npts; Z; Vbar; E
-  const size_t per = 19 * (size_t)npts;
-  c.ws.scratch.reserve(per + (size_t)nbf * npts + (size_t)nbf * nbf + 1);
-  double *ra = c.ws.scratch.p, *rb = ra + npts, *gr = rb + npts, *rho2 = gr + 6 * npts,
-         *sig3 = rho2 + 2 * npts, *exc = sig3 + 3 * npts, *vr = exc + npts, *vs = vr + 2 * npts;
-  double *Z = c.ws.scratch.p + per;
-  double *Vbar = Z + (size_t)nbf * npts;
-  double *EN = Vbar + (size_t)nbf * nbf;
-  launch_density_ref(s, nbf, npts, phi, grad ? gx : nullptr, gy, gz, nocca, Ca, fa, ra,
-                     grad ? gr : nullptr, gr + npts, gr + 2 * npts, nullptr);
-  launch_density_ref(s, nbf, npts, phi, grad ? gx : nullptr, gy, gz, noccb, Cb, fb, rb,
-                     grad ? gr + 3 * npts : nullptr, gr + 4 * npts, gr + 5 * npts, nullptr);
-  const unsigned nblk = (unsigned)((npts + 255) / 256);
-  NKX_HIP_CHECK(hipMemsetAsync(EN, 0, sizeof(double), s));
-  if (npts > 0) {
-    hipLaunchKernelGGL(pack_pol_kernel, dim3(nblk), dim3(256), 0, s, npts, ra, rb, gr, rho2,
-                       grad ? sig3 : nullptr);
-    NKX_HIP_CHECK(hipGetLastError());
-    launch_functional_eval_pol(s, xl, npts, rho2, grad ? sig3 : nullptr, exc, vr,
-                               grad ? vs : nullptr);
-    hipLaunchKernelGGL(energy_pol_kernel, dim3(nblk), dim3(256), 0, s, npts, w, rho2, exc, EN);
-    NKX_HIP_CHECK(hipGetLastError());
-  }
-  const int64_t ne = (int64_t)nbf * npts;
-  for (int spin = 0; spin < 2; ++spin) {
-    if (ne > 0) {
-      hipLaunchKernelGGL(zmat_pol_kernel, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s,
-                         nbf, npts, spin, phi, grad ? gx : nullptr, gy, gz, w, gr, vr, vs, Z);
-      NKX_HIP_CHECK(hipGetLastError());
-    }
-    assemble_v(s, nbf, npts, phi, Z, Vbar, spin ? Vb : Va);
-  }
-  NKX_HIP_CHECK(hipMemcpyAsync(E, EN, sizeof(double), hipMemcpyDeviceToHost, s));
-  NKX_HIP_CHECK(hipStreamSynchronize(s));
-}
-
-void xc_from_collocation(Ctx &c, int nbf, int64_t npts, const double *phi, const double *gx,
-                         const double *gy, const double *gz, const double *w, int nocc,
-                         const double *C, const double *f, const XcList &xl, bool gga,
-                         double *E, double *V) {
-  hipStream_t s = c.stream;
-  const bool grad = gga && gx;
-  // per-point scratch: rho, grx, gry, grz, sigma, exc, vrho, vsigma; Z; Vbar; E
-  const size_t per = 8 * (size_t)npts;
-  c.ws.scratch.reserve(per + (size_t)nbf * npts + (size_t)nbf * nbf + 1);
-  double *rho = c.ws.scratch.p, *grx = rho + npts, *gry = grx + npts, *grz = gry + npts,
-         *sig = grz + npts, *exc = sig + npts, *vr = exc + npts, *vs = vr + npts;
-  double *Z = c.ws.scratch.p + per;
-  double *Vb = Z + (size_t)nbf * npts;
-  double *EN = Vb + (size_t)nbf * nbf;
-  launch_density_ref(s, nbf, npts, phi, grad ? gx : nullptr, gy, gz, nocc, C, f, rho,
-                     grad ? grx : nullptr, gry, grz, grad ? sig : nullptr);
-  launch_functional_eval(s, xl, npts, rho, grad ? sig : nullptr, exc, vr, grad ? vs : nullptr);
-  NKX_HIP_CHECK(hipMemsetAsync(Vb, 0, ((size_t)nbf * nbf + 1) * sizeof(double), s));
-  const int64_t ne = (int64_t)nbf * npts;
-  if (ne > 0) {
-    hipLaunchKernelGGL(zmat_ref_kernel, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s, nbf,
-                       npts, phi, grad ? gx : nullptr, gy, gz, w, rho, grx, gry, grz, vr, vs,
-                       exc, Z, EN);
-    NKX_HIP_CHECK(hipGetLastError());
-    const int tiles = (nbf + 63) / 64;
-    int64_t nsplit = std::max<int64_t>(1, std::min<int64_t>(512 / (tiles * tiles) + 1,
-                                                            (npts + 1023) / 1024));
-    const int64_t kchunk = ((npts + nsplit - 1) / nsplit + 15) / 16 * 16;
-    nsplit = (npts + kchunk - 1) / kchunk;
-    hipLaunchKernelGGL(gemm_nt_ref_kernel, dim3(tiles, tiles, (unsigned)nsplit), dim3(256), 0, s,
-                       nbf, npts, phi, Z, Vb, kchunk);
-    NKX_HIP_CHECK(hipGetLastError());
-  }
-  const int64_t nn = (int64_t)nbf * nbf;
-  if (nn > 0) {
-    hipLaunchKernelGGL(symmetrize_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s,
-                       nbf, Vb, V);
-    NKX_HIP_CHECK(hipGetLastError());
-  }
-  NKX_HIP_CHECK(hipMemcpyAsync(E, EN, sizeof(double), hipMemcpyDeviceToHost, s));
-  NKX_HIP_CHECK(hipStreamSynchronize(s));
 }
 
 }  // namespace nkx
