@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(256) pm_group_i8(int64_t s0, int64_t b0,
 
 // ---------------------------------------------------------------------------
 // Density stage, three kernels: the contraction (density_x2_i8), per batch
-// the reduction and the functional (density_f_i8), the Z slices (z_slots_i8).
+// the reduction and the functional (density_f), the Z slices (z_slots_i8).
 //
 // density_x2_i8: X = P Phi for a pair of function blocks of a batch group.
 // One workgroup of four waves per (batch group of GBT batches, pair of
@@ -651,10 +651,11 @@ __global__ void __launch_bounds__(256) density_x2_i8(
 
 // Per batch: column sums of the live slots in ascending block order,
 // functional, Z coefficients, (E, N) partial sums.
-__global__ void __launch_bounds__(256) density_f_i8(
+__global__ void __launch_bounds__(256) density_f(
     int64_t s0, int64_t b0, const int *__restrict__ b_off, int gga,
     const double *__restrict__ part, const double *__restrict__ pw, XcList xl,
-    double *__restrict__ coef, double *__restrict__ blockEN, double *__restrict__ epoint) {
+    double *__restrict__ coef, double *__restrict__ blockEN, double *__restrict__ epoint,
+    double *__restrict__ rhopt) {
   const int64_t b = b0 + blockIdx.x;
   __shared__ double cs[4][PT];
   const int c = threadIdx.x / PT, g = threadIdx.x % PT;
@@ -678,6 +679,12 @@ __global__ void __launch_bounds__(256) density_f_i8(
     coef[4 * gp + 3] = bs * gzr;
     double e = w * o.e, n = w * rho;
     if (epoint) epoint[gp] = e;  // w e_xc of this point
+    if (rhopt) {                 // rho and grad rho of this point
+      rhopt[4 * gp] = rho;
+      rhopt[4 * gp + 1] = gxr;
+      rhopt[4 * gp + 2] = gyr;
+      rhopt[4 * gp + 3] = gzr;
+    }
     for (int o2 = 32; o2 > 0; o2 >>= 1) {
       e += __shfl_down(e, o2);
       n += __shfl_down(n, o2);
@@ -690,13 +697,13 @@ __global__ void __launch_bounds__(256) density_f_i8(
   }
 }
 
-// Spin-polarised form of density_f_i8: the slot sums of the two spin
+// Spin-polarised form of density_f: the slot sums of the two spin
 // contractions (part_a, part_b) give rho_s and grad rho_s per point; the
 // polarised functional gives the Z coefficients of each spin,
 //   a_s = w v_rho_s / 2,  b_s = w (2 v_sigma_ss grad rho_s + v_sigma_ab grad rho_s'),
 // (xc_integrals.hpp:655-664) into coef_a, coef_b ([point][4] each), and
 // (E, N_alpha, N_beta) per batch.
-__global__ void __launch_bounds__(256) density_fp_i8(
+__global__ void __launch_bounds__(256) density_fp(
     int64_t s0, int64_t b0, const int *__restrict__ b_off, int gga,
     const double *__restrict__ part_a, const double *__restrict__ part_b,
     const double *__restrict__ pw, XcList xl, double *__restrict__ coef_a,
@@ -1137,8 +1144,8 @@ void vkm_density_finish(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_
                         double *coef, double *blockEN, const double *part) {
   if (b1 <= b0) return;
   (void)shape;
-  hipLaunchKernelGGL(density_f_i8, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
-                     pl.b_off.p, gga, part, pl.pw.p, xl, coef, blockEN, nullptr);
+  hipLaunchKernelGGL(density_f, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
+                     pl.b_off.p, gga, part, pl.pw.p, xl, coef, blockEN, nullptr, nullptr);
   NKX_HIP_CHECK(hipGetLastError());
   const int64_t s1 = pl.b_off_h[b1];
   if (s1 > s0)
@@ -1153,7 +1160,7 @@ void vkm_density_finish_pol(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, c
                             double *blockEN, const double *part_a, const double *part_b,
                             double *epoint) {
   if (b1 <= b0) return;
-  hipLaunchKernelGGL(density_fp_i8, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
+  hipLaunchKernelGGL(density_fp, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
                      pl.b_off.p, gga, part_a, part_b, pl.pw.p, xl, coef_a, coef_b, blockEN,
                      epoint);
   NKX_HIP_CHECK(hipGetLastError());
@@ -1173,10 +1180,10 @@ int64_t mixed_zsection_bytes() { return SEC; }
 
 void vkm_density_functional(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
                             int gga, const XcList &xl, double *coef, double *blockEN,
-                            const double *part, double *epoint) {
+                            const double *part, double *epoint, double *rhopt) {
   if (b1 <= b0) return;
-  hipLaunchKernelGGL(density_f_i8, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
-                     pl.b_off.p, gga, part, pl.pw.p, xl, coef, blockEN, epoint);
+  hipLaunchKernelGGL(density_f, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
+                     pl.b_off.p, gga, part, pl.pw.p, xl, coef, blockEN, epoint, rhopt);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -169,7 +169,7 @@ struct Workspace {
   DevBuf<double> coef;             // per padded point and spin: a, bx, by, bz
   DevBuf<double> blockEN;          // per batch: E, N_alpha, N_beta partial sums
   DevBuf<double> vpart;            // split-K partial V tiles
-  DevBuf<double> dpart;            // per spin and slot: column sums of the density contraction (int8 split form)
+  DevBuf<double> dpart;            // per spin and slot: column sums of the density contraction
   DevBuf<signed char> zstore_b;    // int8 form, second spin: Z sections per slot
   DevBuf<double> red;              // small reduction outputs
   DevBuf<double> scratch;

@@ -542,13 +542,12 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   const size_t slot_bytes = b.bf16    ? (size_t)bf16_slot_bytes(gga ? 1 : 0)
                             : b.mixed ? (size_t)mixed_slot_bytes(gga ? 1 : 0)
                                       : (size_t)b.narr * FB * PT * sizeof(double);
-  // per slot beyond the tile store: density partials per spin and the second
-  // spin's Z section (int8 form)
+  // per slot beyond the tile store: density partials per spin and (int8 form)
+  // the second spin's Z section
   const size_t slot_extra =
-      b.mixed && !b.bf16
-          ? (size_t)nspin * 4 * PT * sizeof(double) +
-                (nspin == 2 ? (size_t)mixed_zsection_bytes() : 0)
-          : 0;
+      b.bf16 ? 0
+             : (size_t)nspin * 4 * PT * sizeof(double) +
+                   (b.mixed && nspin == 2 ? (size_t)mixed_zsection_bytes() : 0);
   int64_t max_slots = chunk_slot_budget(slot_bytes + slot_extra, mem_cap);
   // at least the largest single batch
   for (int64_t bb = 0; bb < pl.nb; ++bb)
@@ -556,7 +555,6 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   b.slots_alloc = std::min<int64_t>(max_slots, std::max<int64_t>(pl.nslots, 1));
   if (b.mixed) {
     ws.mstore.reserve((size_t)b.slots_alloc * slot_bytes);
-    if (!b.bf16) ws.dpart.reserve((size_t)nspin * b.slots_alloc * 4 * PT);
     if (!b.bf16 && nspin == 2)
       ws.zstore_b.reserve((size_t)b.slots_alloc * mixed_zsection_bytes());
     int64_t psb = 0;
@@ -567,12 +565,26 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
     ws.tiles64.reserve((size_t)b.slots_alloc * b.narr * FB * PT);
     ws.Pd.reserve((size_t)nspin * pl.P_total);
   }
+  if (!b.bf16) ws.dpart.reserve((size_t)nspin * b.slots_alloc * 4 * PT);
   ws.coef.reserve((size_t)4 * nspin * pl.npts_pad);
   ws.blockEN.reserve((size_t)3 * pl.nb);
   b.vsz = (size_t)b.nsplit * std::max(pl.npairs, 1) * FB * FB;
   ws.vpart.reserve(nspin * b.vsz);
   ws.red.reserve((size_t)3 * pl.nmol);
   return b;
+}
+
+// The functional of the FP64 form from the density partials of one chunk.
+static void fp64_functional(hipStream_t s, int nspin, int64_t b0, int64_t b1, int64_t s0,
+                            const Plan &pl, int gga, const XcList &xl, Workspace &ws,
+                            int64_t slots_alloc, double *epoint) {
+  if (nspin == 2)
+    vkm_density_finish_pol(s, b0, b1, s0, pl, gga, nullptr, nullptr, xl, ws.coef.p,
+                           ws.coef.p + (size_t)4 * pl.npts_pad, ws.blockEN.p, ws.dpart.p,
+                           ws.dpart.p + (size_t)slots_alloc * 4 * PT, epoint);
+  else
+    vkm_density_functional(s, b0, b1, s0, pl, gga, xl, ws.coef.p, ws.blockEN.p, ws.dpart.p,
+                           epoint);
 }
 
 // Every launch of one build, stream-ordered, ending with the copy of the
@@ -601,7 +613,7 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
         vkm_gather_p(s, nbf, pl.mol_nfb_h[m], fp, Pm,
                      ws.Ps.p + (size_t)sp * b.psb + pl.mol_Ps_off_h[m]);
       else
-        vk_gather_p(s, nbf, pl.mol_ld_h[m], fp, Pm,
+        vk_gather_p(s, nbf, pl.mol_ld_h[m], fp, true, Pm,
                     ws.Pd.p + (size_t)sp * pl.P_total + pl.mol_P_off_h[m]);
       // the elements of block pairs without a common batch are never written
       if (!pl.pairs_full) vk_fill0(s, V[(size_t)sp * nmol + m], (int64_t)nbf * nbf);
@@ -628,12 +640,15 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
                     ws.mstore.p, xl, ws.coef.p, ws.blockEN.p,
                     ws.dpart.p + (size_t)sp * b.slots_alloc * 4 * PT);
     else
-      vk_density(s, nspin, b.group, b0, b1, s0, pl, ws.Pd.p, narr, ig, ws.tiles64.p, xl,
-                 ws.coef.p, ws.blockEN.p, nullptr);
+      vk_density(s, nspin, b.group, b0, b1, s0, pl, ws.Pd.p, narr, ig, ws.tiles64.p, ws.dpart.p,
+                 b.slots_alloc * 4 * PT);
     tm.end(tt, s);
-    if (mixed && !bf16) {
+    if (!bf16) {
       tt = tm.begin(kStageZ, s);
-      if (nspin == 2)
+      if (!mixed) {
+        fp64_functional(s, nspin, b0, b1, s0, pl, ig, xl, ws, b.slots_alloc, nullptr);
+        vk_z_slots(s, s0, s1, pl, narr, nspin, ig, ws.coef.p, ws.tiles64.p);
+      } else if (nspin == 2)
         vkm_density_finish_pol(s, b0, b1, s0, pl, ig, ws.mstore.p, ws.zstore_b.p, xl,
                                ws.coef.p, ws.coef.p + (size_t)4 * pl.npts_pad, ws.blockEN.p,
                                ws.dpart.p, ws.dpart.p + (size_t)b.slots_alloc * 4 * PT);
@@ -937,7 +952,7 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
   const size_t slot_bytes =
       mixed ? (size_t)mixed_slot_bytes(gga ? 1 : 0) + (size_t)nspin * 4 * PT * sizeof(double) +
                   (nspin == 2 ? (size_t)mixed_zsection_bytes() : 0)
-            : (size_t)narr * FB * PT * sizeof(double);
+            : ((size_t)narr * FB * PT + (size_t)nspin * 4 * PT) * sizeof(double);
   int64_t max_slots =
       chunk_slot_budget(slot_bytes + 3 * FB * sizeof(double), c.opt.mem_budget);
   for (int64_t b = 0; b < pl.nb; ++b)
@@ -956,13 +971,13 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
   const size_t dsz = (size_t)slots_alloc * 4 * PT;
   if (mixed) {
     ws.mstore.reserve((size_t)slots_alloc * mixed_slot_bytes(gga ? 1 : 0));
-    ws.dpart.reserve(nspin * dsz);
     ws.Ps.reserve(nspin * psb);
     if (nspin == 2) ws.zstore_b.reserve((size_t)slots_alloc * mixed_zsection_bytes());
   } else {
     ws.tiles64.reserve((size_t)slots_alloc * narr * FB * PT);
-    ws.Pd.reserve((size_t)nspin * pl.P_total);
+    ws.Pd.reserve((size_t)2 * nspin * pl.P_total);  // P, then its transpose
   }
+  ws.dpart.reserve(nspin * dsz);
   ws.coef.reserve((size_t)4 * nspin * pl.npts_pad);
   ws.blockEN.reserve((size_t)3 * pl.nb);
   ws.red.reserve(3);
@@ -982,8 +997,9 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
     if (mixed)
       vkm_gather_p(s, pl.nbf, pl.mol_nfb_h[0], pl.fperm_d.p, P[sp], ws.Ps.p + sp * psb);
     else
-      vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, P[sp],
-                  ws.Pd.p + (size_t)sp * pl.P_total);
+      for (int tr = 0; tr < 2; ++tr)
+        vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, tr == 1, P[sp],
+                    ws.Pd.p + (size_t)(tr * nspin + sp) * pl.P_total);
   }
   vk_fill0(s, gacc, (int64_t)n_ga);
   const int ig = gga ? 1 : 0;
@@ -1016,13 +1032,13 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
         vkg_fold(s, b0, b1, s0, pl, nseg, cpart, gacc);
       }
     } else {
-      // the density kernel writes coef per point as [spin][4]
       vk_colloc(s, s0, s1, pl, narr, 1, ws.tiles64.p);
-      vk_density(s, nspin, 4, b0, b1, s0, pl, ws.Pd.p, narr, ig, ws.tiles64.p, xl, ws.coef.p,
-                 ws.blockEN.p, epoint);
+      vk_density(s, nspin, 2, b0, b1, s0, pl, ws.Pd.p + (size_t)nspin * pl.P_total, narr, ig,
+                 ws.tiles64.p, ws.dpart.p, (int64_t)dsz);
+      fp64_functional(s, nspin, b0, b1, s0, pl, ig, xl, ws, slots_alloc, epoint);
       for (int sp = 0; sp < nspin; ++sp) {
         vkg_basis(s, b0, b1, s0, pl, ws.Pd.p + (size_t)sp * pl.P_total, narr, ig, ws.tiles64.p,
-                  ws.coef.p + 4 * sp, 4 * nspin, sp > 0, cpart, tpt);
+                  ws.coef.p + (size_t)4 * sp * pl.npts_pad, 4, sp > 0, cpart, tpt);
         vkg_fold(s, b0, b1, s0, pl, nseg, cpart, gacc);
       }
     }
@@ -1056,22 +1072,25 @@ void density_points(Ctx &c, const double *P, double *rho, double *gx, double *gy
   Workspace &ws = c.ws;
   hipStream_t s = c.stream;
   const int narr = 5;
-  int64_t max_slots = chunk_slot_budget((size_t)narr * FB * PT * sizeof(double), c.opt.mem_budget);
+  int64_t max_slots =
+      chunk_slot_budget(((size_t)narr * FB * PT + 4 * PT) * sizeof(double), c.opt.mem_budget);
   for (int64_t b = 0; b < pl.nb; ++b)
     max_slots = std::max<int64_t>(max_slots, pl.b_off_h[b + 1] - pl.b_off_h[b]);
   const int64_t slots_alloc = std::min<int64_t>(max_slots, std::max<int64_t>(pl.nslots, 1));
   ws.tiles64.reserve((size_t)slots_alloc * narr * FB * PT);
+  ws.dpart.reserve((size_t)slots_alloc * 4 * PT);
   ws.Pd.reserve((size_t)pl.P_total);
   ws.coef.reserve((size_t)4 * pl.npts_pad);
   ws.blockEN.reserve((size_t)3 * pl.nb);
   ws.gbuf.reserve((size_t)4 * pl.npts_pad);
   XcList none{};
   none.n = 0;
-  vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, P, ws.Pd.p);
+  vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, true, P, ws.Pd.p);
   for_each_chunk(pl, slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
     vk_colloc(s, s0, s1, pl, narr, 1, ws.tiles64.p);
-    vk_density(s, 1, 4, b0, b1, s0, pl, ws.Pd.p, narr, 1, ws.tiles64.p, none, ws.coef.p,
-               ws.blockEN.p, nullptr, ws.gbuf.p);
+    vk_density(s, 1, 2, b0, b1, s0, pl, ws.Pd.p, narr, 1, ws.tiles64.p, ws.dpart.p, 0);
+    vkm_density_functional(s, b0, b1, s0, pl, 1, none, ws.coef.p, ws.blockEN.p, ws.dpart.p,
+                           nullptr, ws.gbuf.p);
   });
   vk_scatter_density(s, pl, ws.gbuf.p, rho, gx, gy, gz, sigma);
 }

@@ -5,17 +5,22 @@
 
 namespace nkx {
 
-void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, const double *P,
-                 double *Pd);
+// Pd = P permuted and zero-padded, or its transpose
+void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, bool transpose,
+                 const double *P, double *Pd);
 void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int gga,
                double *tiles);
-// group: batches per workgroup (1, 2 or 4); epoint (may be NULL): w e_xc
-// per sorted point; rhopt (may be NULL, nspin 1): rho and grad rho per sorted
-// point
+// FP64 density contraction (kernels_density.hip): column sums of Phi X and grad
+// Phi X, X = P Phi, per live slot (4 x 64 doubles), spin s at part + s pstride.
+// Pt: the gathered transposes of nspin density matrices; group: consecutive
+// batches per workgroup (1, 2 or 4).  The functional is vkm_density_functional
+// or vkm_density_finish_pol (coef per spin 4 npts_pad apart), then vk_z_slots
+// forms the Z arrays.
 void vk_density(hipStream_t s, int nspin, int group, int64_t b0, int64_t b1, int64_t s0,
-                const Plan &pl, const double *Pd, int narr, int gga, double *tiles,
-                const XcList &xl, double *coef, double *blockEN, double *epoint,
-                double *rhopt = nullptr);
+                const Plan &pl, const double *Pt, int narr, int gga, const double *tiles,
+                double *part, int64_t pstride);
+void vk_z_slots(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int nspin,
+                int gga, const double *coef, double *tiles);
 // screened-grid set-up (kernels_sparse.hip): Morton order of the points
 // (AoS; w, owner may be NULL) in place and the box of each run of per points
 // (6 doubles per box); the CSR list of functions (host centres and radii)
@@ -67,11 +72,12 @@ void vkm_density(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_t s0, c
 void vkm_density_finish(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_t s0,
                         const Plan &pl, int gga, signed char *store, const XcList &xl,
                         double *coef, double *blockEN, const double *part);
-// per-batch reduction of part and the functional only (no Z slices);
-// epoint (may be NULL): w e_xc per sorted point
+// per-batch reduction of part and the functional only (no Z slices), both
+// forms; epoint, rhopt (may be NULL): w e_xc, and rho and grad rho (4), per
+// sorted point
 void vkm_density_functional(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
                             int gga, const XcList &xl, double *coef, double *blockEN,
-                            const double *part, double *epoint);
+                            const double *part, double *epoint, double *rhopt = nullptr);
 // zstore_b (may be NULL): Z sections of the second spin, mixed_zsection_bytes()
 // per slot, instead of the slots' own
 void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
