@@ -15,7 +15,7 @@
 //                    (kernels_density.hip); density_f: the functional per
 //                    batch; z_slots: Z = w (v_rho/2 Phi + 2 v_sigma grad rho .
 //                    grad Phi) written back to the tile store.
-//   vgemm            one workgroup per (function-block pair I <= J, split):
+//   vgemm            one workgroup per (2 x 2 super-pair of blocks, split):
 //                    acc += Phi_I Z_J^T + Z_I Phi_J^T over the batches where
 //                    both blocks are live (MFMA-bound).
 // and once per build: finish (split sum + un-permute + mirror, and the FP64
@@ -73,82 +73,267 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
 }
 
 // ---------------------------------------------------------------------------
-// acc(I, J) += Phi_I Z_J^T + Z_I Phi_J^T over batches where I and J are live.
-constexpr int HP = 32;      // points per LDS stage
-constexpr int LDP = HP + 1; // padded row
+// V contraction on 2 x 2 block super-tiles: V(I, J) = Phi_I Z_J^T + Z_I Phi_J^T
+// over the batches where I and J are live, for the four tiles (I_a, J_b) of a
+// super-pair (blocks I_0 < I_1, J_0 < J_1 of one molecule, -1: missing).  On
+// the diagonal (I = J) only Vbar = Phi Z^T of the four tiles is formed and
+// added to its transpose at the end, half the products.  blockIdx.x = (zs
+// nsplit + split) nsp + super-pair; Z is tile array zbase + zs, and the
+// partials go to vpart + zs nsplit npairs 64^2, written by the first chunk of a
+// build, added to by the later ones.
+//
+// One workgroup of eight waves per (super-pair, split); its batches b = lo +
+// split + nsplit i are taken in windows of 512 candidates, compacted in
+// ascending order into an LDS list of the four slots.  A batch runs in four
+// stages of 16 points: Phi and Z of the J blocks are copied straight into LDS
+// one stage ahead (two buffers), each wave loads its own rows of Phi_I and Z_I
+// into registers one stage ahead, one wait and one barrier per stage.  A wave
+// owns 32 rows of I_a and the 64 columns of J_b; with one J block 16 rows
+// each; with one block in all, the four row groups twice, each with half of a
+// stage's products.  The contraction index (points) is dealt to lanes in runs
+// of four, so that a lane reads 32 contiguous bytes of a row; the 16-byte
+// pieces of an LDS row are exchanged by bits 1 .. 3 of the row, so that sixteen
+// rows fall on sixteen different bank groups.
+//
+// Bound by the FP64 MFMA rate (busy 70 % of the cycles; the rest is the wait at
+// a stage's start, one workgroup per CU): 16 waters take 8.7 ms, 48 TFLOP/s,
+// a 12-atom molecule with two spins 402 us, water 26 us.  One workgroup per
+// block pair, both products on the diagonal too, read four tiles for every two
+// products of them (58 GB on 16 waters): 9.9 ms, 737 us and 245 us.
+constexpr int VS = 16;             // points of a stage
+constexpr int VSEC = FB * VS;      // doubles of one block's stage
 
-// blockIdx.x = (zs * nsplit + split) * npairs + pair; Z is tile array
-// zbase + zs, and the partials go to vpart + zs * nsplit * npairs * FB * FB:
-// written by the first chunk of a build, added to by the later ones.
-__global__ void __launch_bounds__(256) vgemm_f64(
-    int npairs, int nsplit, const int *__restrict__ pair_I, const int *__restrict__ pair_J,
-    const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1, int64_t s0,
+// four doubles 32-byte aligned
+__device__ __forceinline__ v4d ld4(const double *p) { return *reinterpret_cast<const v4d *>(p); }
+
+// s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima)
+__device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+__global__ void __launch_bounds__(512) vgemm_f64(
+    int nsp, int nsplit, const int4 *__restrict__ sp_blk, const int4 *__restrict__ sp_pidx,
+    int npairs, const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1, int64_t s0,
     int narr, int zbase, int first, const double *__restrict__ tiles,
     double *__restrict__ vpart) {
-  const int p = blockIdx.x % npairs;
-  const int split = (blockIdx.x / npairs) % nsplit;
-  const int zs = blockIdx.x / (npairs * nsplit);
-  const int zarr = zbase + zs;
+  // Z_J0, Z_J1, Phi_J0, Phi_J1 of a stage; two buffers, declared apart so that
+  // a copy into one is known not to touch the other
+  __shared__ __attribute__((aligned(16))) double bufA[4][VSEC];
+  __shared__ __attribute__((aligned(16))) double bufB[4][VSEC];
+  __shared__ int ls[4][512];  // slots of I_0, I_1, J_0, J_1 per listed batch
+  __shared__ int wcnt[8];
+  // workgroups are dealt to the eight XCDs in turn: the super-pairs of a split
+  // run on one XCD and share its L2 for the batches' tiles
+  const int xcd = blockIdx.x & 7, rr = blockIdx.x >> 3, nsg = (nsplit + 7) / 8;
+  const int sp = rr % nsp, split = (rr / nsp) % nsg * 8 + xcd, zs = rr / (nsp * nsg);
+  if (split >= nsplit) return;
+  const int64_t zoff = (int64_t)(zbase + zs) * TILE;
   vpart += (int64_t)zs * nsplit * npairs * (FB * FB);
-  const int I = pair_I[p], J = pair_J[p];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int4 blk = sp_blk[sp], pix = sp_pidx[sp];
+  const bool diag = blk.x == blk.z;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, q = lane >> 4;
-  __shared__ double A0[FB][LDP], A1[FB][LDP], B0[FB][LDP], B1[FB][LDP];
-  v4d acc[4];
-  for (int j = 0; j < 4; ++j) acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
-  // batches of the pair's molecule inside [b0, b1)
-  const int mol = mt.blk_mol[I];
+  // this wave's tile (wa, wb), rows row0 .. of I_wa, one or two groups of 16;
+  // half: the half of a stage's products it forms (-1: all)
+  const bool two = blk.w >= 0;           // two J blocks (then two I blocks)
+  const bool one = !two && blk.y < 0;    // one block in all
+  const int wa = one ? 0 : wv >> 2, wb = two ? wv & 1 : 0;
+  const int row0 = two ? 32 * ((wv >> 1) & 1) : 16 * (wv & 3);
+  const int half = one ? wv >> 2 : -1;
+  v4d acc[2][4];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[g][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  // batches of the super-pair's molecule inside [b0, b1)
+  const int mol = mt.blk_mol[blk.x];
   const int64_t mb0 = mt.b0[mol], mnb = mt.nb[mol];
-  const int *tsI = tile_slot + mt.ts_off[mol] + (int64_t)mt.blk_local[I] * mnb - mb0;
-  const int *tsJ = tile_slot + mt.ts_off[mol] + (int64_t)mt.blk_local[J] * mnb - mb0;
+  const int *ts0 = tile_slot + mt.ts_off[mol] - mb0;
+  const int bl[4] = {blk.x, blk.y, blk.z, blk.w};
+  int64_t tso[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) tso[u] = bl[u] >= 0 ? (int64_t)mt.blk_local[bl[u]] * mnb : -1;
   const int64_t lo = b0 > mb0 ? b0 : mb0, hi = b1 < mb0 + mnb ? b1 : mb0 + mnb;
-  for (int64_t b = lo + split; b < hi; b += nsplit) {
-    const int sI = tsI[b], sJ = tsJ[b];
-    if (sI < 0 || sJ < 0) continue;
-    const double *tI = tiles + (sI - s0) * narr * TILE;
-    const double *tJ = tiles + (sJ - s0) * narr * TILE;
-    for (int h = 0; h < PT; h += HP) {
-      {
-        const double *zI = tI + zarr * TILE, *zJ = tJ + zarr * TILE;
+
+  struct AFrag {
+    v4d f[2], z[2];  // rows of Phi_I, Z_I per row group
+  };
+  auto slot = [&](int u, int i) { return __builtin_amdgcn_readfirstlane(ls[u][i]); };
+  // operands of stage st (point group) of listed batch i: this wave's rows to
+  // registers (those of slot s0 where its tile is idle: never used), the J
+  // blocks to LDS
+  auto issue = [&](int i, int st, double (*dst)[VSEC], AFrag &a) {
+    const int sI = slot(wa, i);
+    const double *pI = tiles + (int64_t)(sI >= 0 ? sI - s0 : 0) * narr * TILE +
+                       (row0 + l16) * PT + VS * st + 4 * q;
+    a.f[0] = ld4(pI);
+    if (two) a.f[1] = ld4(pI + 16 * PT);
+    if (!diag) {
+      a.z[0] = ld4(pI + zoff);
+      if (two) a.z[1] = ld4(pI + zoff + 16 * PT);
+    }
+    // 8 rows x 128 bytes per copy, the waves in turn
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int e = 2 * (u * 256 + (int)threadIdx.x);
-          const int r = e / HP, c = e % HP;
-          const int off = r * PT + h + c;
-          const double2 a0 = *reinterpret_cast<const double2 *>(tI + off);
-          const double2 a1 = *reinterpret_cast<const double2 *>(zI + off);
-          const double2 b0v = *reinterpret_cast<const double2 *>(tJ + off);
-          const double2 b1v = *reinterpret_cast<const double2 *>(zJ + off);
-          A0[r][c] = a0.x;  A0[r][c + 1] = a0.y;
-          A1[r][c] = a1.x;  A1[r][c + 1] = a1.y;
-          B0[r][c] = b0v.x; B0[r][c + 1] = b0v.y;
-          B1[r][c] = b1v.x; B1[r][c + 1] = b1v.y;
-        }
-      }
-      __syncthreads();
-#pragma unroll 2
-      for (int k0 = 0; k0 < HP; k0 += 4) {
-        const double aphi = A0[16 * wv + l16][k0 + q];
-        const double az = A1[16 * wv + l16][k0 + q];
+    for (int jb = 0; jb < 2; ++jb) {
+      if (jb && !two) continue;
+      const int sJ = slot(2 + jb, i);
+      if (sJ < 0) continue;
+      const int r = 8 * wv + (lane >> 3);
+      const int c = (lane & 7) ^ ((r >> 1) & 7);
+      const double *src = tiles + (int64_t)(sJ - s0) * narr * TILE + r * PT + VS * st + 2 * c;
+      __builtin_amdgcn_global_load_lds(src + zoff, &dst[jb][8 * wv * VS], 16, 0, 0);
+      if (!diag) __builtin_amdgcn_global_load_lds(src, &dst[2 + jb][8 * wv * VS], 16, 0, 0);
+    }
+  };
+  // A (rows of I) x the section's 64 columns, four steps of four points
+  auto phase = [&](const double *sec, const v4d (&a)[2]) {
+    v4d bv[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const double bz = B1[16 * j + l16][k0 + q];
-          const double bphi = B0[16 * j + l16][k0 + q];
-          acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(aphi, bz, acc[j], 0, 0, 0);
-          acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(az, bphi, acc[j], 0, 0, 0);
-        }
+    for (int j = 0; j < 4; ++j) {
+      const int r = 16 * j + l16, x = (r >> 1) & 7;
+      const double2 u = *reinterpret_cast<const double2 *>(sec + r * VS + 2 * ((2 * q) ^ x));
+      const double2 v = *reinterpret_cast<const double2 *>(sec + r * VS + 2 * ((2 * q + 1) ^ x));
+      bv[j] = v4d{u.x, u.y, v.x, v.y};
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (half >= 0 && (e >> 1) != half) continue;  // uniform
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[0][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0][e], bv[j][e], acc[0][j], 0, 0, 0);
+      if (two) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[1][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1][e], bv[j][e], acc[1][j], 0, 0, 0);
       }
-      __syncthreads();
+    }
+  };
+  AFrag a0, a1;
+  // stage t of a window of n batches: wait for its operands, start the next
+  // stage's, form its products
+  auto step = [&](int t, int n, double (*cur)[VSEC], double (*nxt)[VSEC], const AFrag &a,
+                  AFrag &an) {
+    wait_vm0();
+    __syncthreads();  // cur complete, nxt free
+    if (t + 1 < 4 * n) issue((t + 1) >> 2, (t + 1) & 3, nxt, an);
+    const int i = t >> 2;
+    if (slot(wa, i) >= 0 && slot(2 + wb, i) >= 0) {
+      phase(&cur[wb][0], a.f);
+      if (!diag) phase(&cur[2 + wb][0], a.z);
+    }
+  };
+
+  for (int64_t c0 = lo + split; c0 < hi; c0 += 512 * (int64_t)nsplit) {
+    const int64_t b = c0 + (int64_t)nsplit * threadIdx.x;
+    int sl[4] = {-1, -1, -1, -1};
+    if (b < hi) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (tso[u] >= 0) sl[u] = ts0[tso[u] + b];
+    }
+    const bool act = (sl[0] >= 0 || sl[1] >= 0) && (sl[2] >= 0 || sl[3] >= 0);
+    const unsigned long long m = __ballot(act);
+    __syncthreads();  // the previous window is done with the list and buffers
+    if (lane == 0) wcnt[wv] = __popcll(m);
+    __syncthreads();
+    int off = 0, n = 0;
+    for (int w = 0; w < 8; ++w) {
+      if (w < wv) off += wcnt[w];
+      n += wcnt[w];
+    }
+    n = __builtin_amdgcn_readfirstlane(n);
+    if (act) {
+      const int i = off + __popcll(m & ((1ull << lane) - 1ull));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ls[u][i] = sl[u];
+    }
+    __syncthreads();
+    if (n == 0) continue;
+    issue(0, 0, bufA, a0);
+    for (int t = 0; t < 4 * n; t += 2) {  // an even number of stages
+      step(t, n, bufA, bufB, a0, a1);
+      step(t + 1, n, bufB, bufA, a1, a0);
     }
   }
-  double *out = vpart + ((int64_t)split * npairs + p) * (FB * FB);
+
+  if (diag) {
+    // through LDS, tile by tile: with one block the second halves' sums, then
+    // V(a, b) = Vbar(a, b) + Vbar(b, a)^T for (0, 0), (0, 1), (1, 1)
+    double(*t)[FB + 1] = reinterpret_cast<double(*)[FB + 1]>(&bufA[0][0]);
+    static_assert(sizeof(bufA) >= 32 * (FB + 1) * sizeof(double), "half a tile in a buffer");
+    const int ng = two ? 2 : 1;
+    if (one) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+      for (int h = 0; h < 2; ++h) {  // 32 rows at a time
+        __syncthreads();
+        if (half == 1 && (row0 >> 5) == h) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int mu = 16 * wv + 4 * r + q, nu = 16 * j + l16;
-      out[mu * FB + nu] = first ? acc[j][r] : out[mu * FB + nu] + acc[j][r];
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) t[(row0 & 31) + 4 * r + q][16 * j + l16] = acc[0][j][r];
+        }
+        __syncthreads();
+        if (half == 0 && (row0 >> 5) == h) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[0][j][r] += t[(row0 & 31) + 4 * r + q][16 * j + l16];
+        }
+      }
     }
+    const int ntile = two ? 3 : (one ? 1 : 2);
+    for (int k = 0; k < ntile; ++k) {
+      // target tile (ta, tb), from tile (tb, ta)
+      const int ta = k == 2 ? 1 : 0, tb = k == 0 ? 0 : 1;
+      v4d add[2][4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {  // rows 32 h .. of the source = columns of the target
+        __syncthreads();
+        if (wa == tb && wb == ta && half != 1) {
+#pragma unroll
+          for (int g = 0; g < 2; ++g)
+            if (g < ng && ((row0 + 16 * g) >> 5) == h) {
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  t[((row0 + 16 * g) & 31) + 4 * r + q][16 * j + l16] = acc[g][j][r];
+            }
+        }
+        __syncthreads();
+        if (wa == ta && wb == tb) {
+#pragma unroll
+          for (int g = 0; g < 2; ++g)
+            if (g < ng) {
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  add[g][2 * h + j][r] = t[16 * j + l16][row0 + 16 * g + 4 * r + q];
+            }
+        }
+      }
+      if (wa == ta && wb == tb) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          if (g < ng)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[g][j] += add[g][j];
+      }
+    }
+  }
+  const int pp = wa ? (wb ? pix.w : pix.z) : (wb ? pix.y : pix.x);
+  if (pp < 0 || half == 1) return;
+  double *out = vpart + ((int64_t)split * npairs + pp) * (FB * FB);
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    if (g && !two) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int mu = row0 + 16 * g + 4 * r + q, nu = 16 * j + l16;
+        out[mu * FB + nu] = first ? acc[g][j][r] : out[mu * FB + nu] + acc[g][j][r];
+      }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -299,10 +484,13 @@ void vk_zoverlap(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr
 
 void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
               int narr, int nz, bool first, const double *tiles, double *vpart) {
-  if (b1 <= b0 || pl.npairs == 0) return;
-  hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)(pl.npairs * nsplit * nz)), dim3(256), 0, s,
-                     pl.npairs, nsplit, pl.pair_I.p, pl.pair_J.p, pl.tile_slot.p, pl.tab(), b0, b1,
-                     s0, narr, narr - nz, first ? 1 : 0, tiles, vpart);
+  if (b1 <= b0 || pl.nspairs == 0) return;
+  const int64_t nwg = (int64_t)pl.nspairs * ((nsplit + 7) / 8 * 8) * nz;
+  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "V contraction grid too large");
+  hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)nwg), dim3(512), 0, s, pl.nspairs, nsplit,
+                     reinterpret_cast<const int4 *>(pl.sp_blk.p),
+                     reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.npairs, pl.tile_slot.p,
+                     pl.tab(), b0, b1, s0, narr, narr - nz, first ? 1 : 0, tiles, vpart);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -474,18 +474,20 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
   return (int64_t)(budget / slot_bytes);
 }
 
-// Split count of the V contraction over batches: about 8192 workgroups of
-// the FP64 kernel's pair tiles or of the int8 kernel's super-pair tiles
-// (a few per CU at a time, the rest balancing the tail), or the autotuned
-// value.
-int choose_nsplit(const Plan &pl, int tuned = 0, bool super = false) {
-  const int64_t units = super ? pl.nspairs : pl.npairs;
+// Split count of the V contraction over batches, or the tuned value.  FP64:
+// about 4096 workgroups of a super-pair tile (one per CU at a time, the rest
+// balancing the tail: with 2048 the CUs of 16 waters were busy 84 % of the
+// time; every split costs a tile of partials per pair), at least four batches
+// each (31 splits of 32 batches left water on 31 CUs: 245 us, now 26).  int8 and bf16: about 8192 workgroups of a super-pair tile
+// or a pair, at least 32 batches each (on small molecules one batch per
+// workgroup is mostly set-up there).
+int choose_nsplit(const Plan &pl, int precision, int tuned = 0) {
+  const bool f64 = precision == NKX_PREC_FP64;
+  const int64_t units = precision == NKX_PREC_MIXED_BF16 ? pl.npairs : pl.nspairs;
   if (units == 0) return 1;
-  // about 8192 workgroups, and (automatic choice) at least 32 batches per
-  // split: on small molecules one batch per workgroup is mostly set-up
-  const int64_t target = 8192;
+  const int64_t target = f64 ? 4096 : 8192;
   int64_t ns = tuned > 0 ? tuned : (target + units - 1) / units;
-  if (tuned <= 0) ns = std::min<int64_t>(ns, pl.nb / 32);
+  if (tuned <= 0) ns = std::min<int64_t>(ns, pl.nb / (f64 ? 4 : 32));
   ns = std::max<int64_t>(1, std::min<int64_t>(ns, pl.nb));
   return (int)ns;
 }
@@ -532,7 +534,7 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   b.gga = gga;
   const int nmol = pl.nmol;
   b.narr = (gga ? 4 : 1) + nspin;
-  b.nsplit = choose_nsplit(pl, tuned_split, precision == NKX_PREC_MIXED);
+  b.nsplit = choose_nsplit(pl, precision, tuned_split);
   b.bf16 = precision == NKX_PREC_MIXED_BF16;
   b.mixed = precision == NKX_PREC_MIXED || b.bf16;
   NKX_REQUIRE(!b.bf16 || nspin == 1, NKX_ERR_UNSUPPORTED,
@@ -711,7 +713,7 @@ namespace {
 // fastest pair in the ctx options and returns its build time.
 double autotune_on(Ctx &c, const Plan &pl, int precision, const std::function<void()> &build,
                    int *best_split, int *best_group) {
-  const int base = choose_nsplit(pl, 0, precision == NKX_PREC_MIXED);
+  const int base = choose_nsplit(pl, precision);
   std::vector<int> splits;
   for (int k : {base / 4, base / 2, base, 2 * base, 4 * base}) {
     const int v = std::max(1, std::min<int>(k, (int)std::max<int64_t>(pl.nb, 1)));
@@ -1139,7 +1141,7 @@ void overlap_build(Ctx &c, double *S) {
   Workspace &ws = c.ws;
   hipStream_t s = c.stream;
   const int narr = 2;
-  const int nsplit = choose_nsplit(pl);
+  const int nsplit = choose_nsplit(pl, NKX_PREC_FP64);
   int64_t max_slots =
       chunk_slot_budget((size_t)narr * FB * PT * sizeof(double), c.opt.mem_budget);
   for (int64_t b = 0; b < pl.nb; ++b)
