@@ -407,28 +407,23 @@ int nkx_molset_create(nkx_ctx *ctx, int nmol, const int *natoms, const double *x
     nkx::Ctx &c = ctx->c;
     NKX_REQUIRE(nmol > 0 && natoms && xyz && Z && nbf, NKX_ERR_INVALID_ARGUMENT,
                 "molset_create: bad arguments");
-    std::vector<std::vector<double>> pts(nmol), wts(nmol);
+    std::vector<nkx::GridState> grids(nmol);
+    std::vector<nkx::MolPoints> mols;
     std::vector<nkx::BasisHost> bases;
     size_t aoff = 0, foff = 0;
     for (int k = 0; k < nmol; ++k) {
-      nkx::GridState g;
+      nkx::GridState &g = grids[k];
       build_grid(c, natoms[k], xyz + 3 * aoff, Z + aoff, nrad, nang_order, radial_scheme,
                  ta_alpha, w_thr, radial_sizing, g);
-      pts[k].resize(3 * (size_t)g.npts);
-      wts[k].resize(g.npts);
-      NKX_HIP_CHECK(hipMemcpyAsync(pts[k].data(), g.pts.p, pts[k].size() * sizeof(double),
-                                   hipMemcpyDeviceToHost, c.stream));
-      NKX_HIP_CHECK(hipMemcpyAsync(wts[k].data(), g.w.p, wts[k].size() * sizeof(double),
-                                   hipMemcpyDeviceToHost, c.stream));
-      NKX_HIP_CHECK(hipStreamSynchronize(c.stream));
       NKX_REQUIRE(g.npts > 0, NKX_ERR_INVALID_ARGUMENT, "molset_create: a molecule has no points");
       if (npts_out) npts_out[k] = g.npts;
+      mols.push_back(nkx::MolPoints{g.npts, g.pts.p, g.w.p});
       bases.push_back(make_basis(nbf[k], n + foff, l + foff, m + foff, zeta + foff, norm + foff,
                                  centers + 3 * foff, nullptr));
       aoff += natoms[k];
       foff += nbf[k];
     }
-    nkx::build_molset_plan(c, pts, wts, bases);
+    nkx::build_molset_plan(c, mols, bases);
   });
 }
 

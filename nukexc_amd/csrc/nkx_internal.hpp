@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -57,6 +58,61 @@ struct DevBuf {
     reserve(count);
     if (count) NKX_HIP_CHECK(hipMemcpyAsync(p, host, count * sizeof(T), hipMemcpyHostToDevice, s));
   }
+};
+
+// Page-locked host memory; grows on demand and never shrinks.  What the GPU
+// reads or writes in it is reused only after the stream was waited for.
+struct PinBuf {
+  char *p = nullptr;
+  size_t n = 0;
+  PinBuf() = default;
+  PinBuf(const PinBuf &) = delete;
+  PinBuf &operator=(const PinBuf &) = delete;
+  ~PinBuf() { release(); }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+  }
+  void reserve(size_t bytes) {
+    if (bytes <= n) return;
+    release();
+    NKX_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&p), bytes, hipHostMallocDefault));
+    n = bytes;
+  }
+};
+
+// Host tables gathered into one page-locked buffer and copied to the device at
+// once; each table's device pointer is set by the upload.
+struct TablePack {
+  struct Item {
+    const void *src;
+    size_t bytes, off;
+    void **dst;
+  };
+  std::vector<Item> items;
+  size_t total = 0;
+  template <typename T>
+  void add(T *&dst, const T *src, size_t count) {
+    items.push_back({src, count * sizeof(T), total, reinterpret_cast<void **>(&dst)});
+    total += (count * sizeof(T) + 255) & ~(size_t)255;
+  }
+  void upload(PinBuf &pin, DevBuf<char> &dev, hipStream_t s) {
+    if (total == 0) return;
+    pin.reserve(total);
+    dev.reserve(total);
+    for (const Item &it : items) {
+      if (it.bytes) std::memcpy(pin.p + it.off, it.src, it.bytes);
+      *it.dst = dev.p + it.off;
+    }
+    NKX_HIP_CHECK(hipMemcpyAsync(dev.p, pin.p, total, hipMemcpyHostToDevice, s));
+  }
+};
+
+// A table inside a packed device buffer.
+template <typename T>
+struct DevView {
+  T *p = nullptr;
 };
 
 // STO basis on the device, one record per function.
@@ -116,9 +172,10 @@ struct Plan {
   int nbf = 0, nbf_pad = 0, nfb = 0;       // totals over molecules
   int64_t npts = 0, npts_pad = 0, nb = 0;  // nb = number of point batches
   std::vector<int> fperm;     // global sorted position -> original function index in its molecule
-  DevBuf<int> fperm_d;
-  DevBuf<FuncRec> funcs;      // nbf_pad records in sorted order (padding: norm 0)
-  DevBuf<HarmTerm> terms;
+  DevBuf<char> tables;        // the packed small tables (DevView members)
+  DevView<int> fperm_d;
+  DevView<FuncRec> funcs;     // nbf_pad records in sorted order (padding: norm 0)
+  DevView<HarmTerm> terms;
   DevBuf<double> px, py, pz, pw;  // sorted, padded point SoA
   DevBuf<int> pidx;               // sorted position -> original point in its molecule (-1: pad)
   // batch -> active function blocks (CSR)
@@ -128,13 +185,13 @@ struct Plan {
   int npairs = 0;
   bool pairs_full = false;        // every block pair of every molecule is kept
   std::vector<int> pair_I_h, pair_J_h;
-  DevBuf<int> pair_I, pair_J;
+  DevView<int> pair_I, pair_J;
   // 2 x 2 super-pairs of blocks (one molecule) for the int8 V contraction:
   // 4 ints each, blocks I0 I1 J0 J1 (-1: none) and the pair indices of the
   // tiles (I0,J0) (I0,J1) (I1,J0) (I1,J1) (-1: not a kept pair, or redundant)
   int nspairs = 0;
   int max_mol_nfb = 0;            // largest function-block count of one molecule
-  DevBuf<int> sp_blk, sp_pidx;
+  DevView<int> sp_blk, sp_pidx;
   DevBuf<int> tile_slot;          // per molecule [block][batch] -> slot in the tile store or -1
   int64_t nslots = 0;
   int64_t pairs_kept = 0;
@@ -144,12 +201,23 @@ struct Plan {
   std::vector<int> mol_nbf_h, mol_ld_h, mol_nfb_h, mol_blk0_h;
   std::vector<int64_t> mol_b0_h, mol_nb_h, mol_npts_h, mol_P_off_h, mol_Ps_off_h;
   int64_t P_total = 0;            // sum of ld^2 (one spin of gathered FP64 P)
-  DevBuf<int> blk_mol, blk_local, mol_ld, mol_nfb, mol_nbf;
-  DevBuf<int64_t> mol_b0, mol_nb, mol_ts_off, mol_P_off, mol_Ps_off;
+  DevView<int> blk_mol, blk_local, mol_ld, mol_nfb, mol_nbf;
+  DevView<int64_t> mol_b0, mol_nb, mol_ts_off, mol_P_off, mol_Ps_off;
   MolTab tab() const {
     return MolTab{blk_mol.p, blk_local.p, mol_ld.p, mol_nfb.p, mol_b0.p,
                   mol_nb.p,  mol_ts_off.p, mol_P_off.p, mol_Ps_off.p};
   }
+};
+
+// Scratch of a plan's construction, kept by the ctx.
+struct PlanScratch {
+  DevBuf<double> part, boxes;      // box of the points; box per batch
+  DevBuf<uint64_t> key;            // Morton codes, unsorted and sorted
+  DevBuf<int> idx, count, pairs;   // point indices (twice); per batch counts; pair flags
+  DevBuf<char> tmp;                // of the radix sort
+  DevBuf<unsigned char> live;      // per molecule [batch][block]
+  DevBuf<char> fn;                 // screening centres and radii
+  PinBuf pin_fn, pin_tab, pin_cnt;
 };
 
 struct Options {
@@ -247,6 +315,7 @@ struct Ctx {
   Plan plan;
   Plan mplan;                    // plan of the molecule set (nkx_molset_create)
   uint64_t mplan_version = 0;    // bumped by every nkx_molset_create
+  PlanScratch plan_ws;
   Workspace ws;
   GraphState graph;
   DevBuf<double> becke_rtab;     // inter-atomic distances of the last partition
@@ -339,8 +408,12 @@ double autotune(Ctx &c, const double *P, const XcList &xl, bool gga, int precisi
                 int *best_split, int *best_group);
 double molset_autotune(Ctx &c, const double *const *P, const XcList &xl, bool gga,
                        int precision, double *const *V, int *best_split, int *best_group);
-void build_molset_plan(Ctx &c, const std::vector<std::vector<double>> &mol_pts,
-                       const std::vector<std::vector<double>> &mol_w,
+// points and weights of each molecule on the device
+struct MolPoints {
+  int64_t npts;
+  const double *pts, *w;
+};
+void build_molset_plan(Ctx &c, const std::vector<MolPoints> &mols,
                        const std::vector<BasisHost> &bases);
 void overlap_build(Ctx &c, double *S);
 // nuclear gradient of E_xc at fixed P (nspin spin density matrices, or the

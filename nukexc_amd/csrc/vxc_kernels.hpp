@@ -5,6 +5,20 @@
 
 namespace nkx {
 
+// launch plan (kernels_plan.hip): a molecule's points in Morton order, padded
+// to batches of 64, and the batches' boxes (6 doubles)
+void vk_plan_points(hipStream_t s, PlanScratch &sc, int64_t npts, const double *pts,
+                    const double *w, double *px, double *py, double *pz, double *pw, int *pidx,
+                    double *boxes);
+// live[batch][block] and per batch (live blocks, functions in them); fn:
+// centre and screening radius per sorted function
+void vk_plan_screen(hipStream_t s, int64_t nb, int nbf, int nfb, const double *boxes,
+                    const double *fn, unsigned char *live, int *count);
+// slots of the molecule's batches b0 .. b0 + nb - 1 (b_off over all batches),
+// its [block][batch] table and pairs[nfb][nfb] of blocks with a common batch
+void vk_plan_fill(hipStream_t s, int64_t nb, int nfb, int blk0, int64_t b0,
+                  const unsigned char *live, const int *b_off, int *b_fbl, int *slot_b,
+                  int *tile_slot, int *pairs);
 // Pd = P permuted and zero-padded, or its transpose
 void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, bool transpose,
                  const double *P, double *Pd);
