@@ -609,7 +609,8 @@ int nkx_collocation(nkx_ctx *ctx, int64_t npts, const double *pts, double *phi, 
     for (int i = 0; i < B.nbf; ++i) {
       const auto &t = nkx::solid_harmonic_terms(B.l[i], B.m[i]);
       fr[i] = nkx::FuncRec{B.cx[i], B.cy[i], B.cz[i], B.zeta[i], B.norm[i],
-                           B.n[i] - B.l[i] - 1, (int)terms.size(), (int)t.size(), 0};
+                           B.n[i] - B.l[i] - 1, (int)terms.size(), (int)t.size(),
+                           nkx::func_type(B.l[i], B.m[i])};
       terms.insert(terms.end(), t.begin(), t.end());
     }
     nkx::DevBuf<nkx::FuncRec> fd;

@@ -186,14 +186,15 @@ __global__ void __launch_bounds__(256, 2) density_x_f64(
   }
 }
 
-// Z_s = a_s Phi + b_s . grad Phi per live slot, array narr - nspin + s of the
-// slot; coef[s] + 4 point.  Two points per thread, both spins from one read.
+// Z_s = ascale a_s Phi + b_s . grad Phi per live slot, array narr - nspin + s of
+// the slot; coef[s] + 4 point.  Two points per thread, both spins from one read.
 // Bound by its bytes: 128 KB read and 32 KB written per slot and spin (GGA),
 // 5.3 TB/s on 16 waters.
 __global__ void __launch_bounds__(256) z_slots_f64(int64_t s0, const int *__restrict__ slot_b,
                                                    int narr, int nspin, int gga,
                                                    const double *__restrict__ coef,
-                                                   int64_t cspin, double *__restrict__ tiles) {
+                                                   int64_t cspin, double ascale,
+                                                   double *__restrict__ tiles) {
   const int64_t b = slot_b[s0 + blockIdx.x];
   double *tb = tiles + (int64_t)blockIdx.x * narr * TILE;
   const int c = 2 * (threadIdx.x & 31), r0 = threadIdx.x >> 5;
@@ -204,6 +205,8 @@ __global__ void __launch_bounds__(256) z_slots_f64(int64_t s0, const int *__rest
       const double *p = coef + s * cspin + 4 * (b * PT + c);
 #pragma unroll
       for (int a = 0; a < 4; ++a) k[s][a] = make_double2(p[a], p[4 + a]);
+      k[s][0].x *= ascale;
+      k[s][0].y *= ascale;
     }
 #pragma unroll 4
   for (int r = r0; r < FB; r += 8) {
@@ -251,10 +254,10 @@ void vk_density(hipStream_t s, int nspin, int group, int64_t b0, int64_t b1, int
 }
 
 void vk_z_slots(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int nspin,
-                int gga, const double *coef, double *tiles) {
+                int gga, double ascale, const double *coef, double *tiles) {
   if (s1 <= s0) return;
   hipLaunchKernelGGL(z_slots_f64, dim3((unsigned)(s1 - s0)), dim3(256), 0, s, s0, pl.slot_b.p,
-                     narr, nspin, gga, coef, (int64_t)4 * pl.npts_pad, tiles);
+                     narr, nspin, gga, coef, (int64_t)4 * pl.npts_pad, ascale, tiles);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -17,8 +17,9 @@
 //   dmu_ij/dR_i = -u_i/R~ - [R~ = R_ij] mu (R_i - R_j)/R_ij^2,
 //   dmu_ij/dR_j = +u_j/R~ + [R~ = R_ij] mu (R_i - R_j)/R_ij^2,
 //   u_i = (r - R_i)/r_i; s' = 0 where mu is clamped at +-1.
+#include "grad_rows.hpp"
+#include "lane_sums.hpp"
 #include "nkx_internal.hpp"
-#include "sto_eval.hpp"
 #include "vxc_kernels.hpp"
 
 namespace nkx {
@@ -33,147 +34,157 @@ constexpr int GC = FB * 3;  // per-slot partial: 64 functions x 3 components
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// One workgroup per batch.  Tile store arrays: Phi, dPhi/dx, dPhi/dy, dPhi/dz
-// (narr >= 4).  coef per point (stride cstride doubles): (w v_rho / 2, b_x,
-// b_y, b_z) of the spin whose P is Pd; accum adds the point sums to tpt (the
-// second spin of an open shell) instead of writing them.
-__global__ void __launch_bounds__(256) grad_basis_f64(
-    int nbf_pad, const double *__restrict__ Pd, const int *__restrict__ b_off,
-    const int *__restrict__ b_fbl, int64_t s0, int64_t b0, int narr, int gga,
-    const double *__restrict__ tiles, const double *__restrict__ coef,
+// Basis-centre term: X = P Phi and W = P Y (Y in tile array yarr) for one pair
+// of a batch's live blocks, then grad_rows.  One workgroup of four waves per
+// (batch, pair of list blocks); a wave holds 32 rows of its block x 64 points
+// of both products (16 rows of the only block where the pair has one).  The
+// contraction is that of density_x_f64 (kernels_density.hip) in stages of 16
+// functions: Phi and Y of the next stage go straight into the other LDS
+// buffer and the next P fragments into the other register set while the
+// current stage's products run.  The epilogue passes X and W of a wave through
+// its own part of the buffers, eight rows at a time, to a point per lane.
+// cpart[(slot - s0) 192 + 3 mu + k]: per function; tpart[(slot - s0) 256 + 64 k +
+// point], slot the pair's first: per point, over the pair's functions.
+//
+// Bound by the FP64 MFMA rate and FP64 VALU issue (grad_rows) in turn; see
+// there for what the epilogue took before.
+constexpr int GS = 16;           // functions of a stage
+constexpr int GSTG = GS * PT;    // doubles of one array's stage
+
+// s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima)
+__device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+__global__ void __launch_bounds__(256, 2) grad_basis_f64(
+    MolTab mt, const double *__restrict__ Pt, const int *__restrict__ b_off,
+    const int *__restrict__ b_fbl, int64_t s0, int64_t b0, int64_t b1, int nmg, int narr,
+    int yarr, int gga, const double *__restrict__ tiles, const double *__restrict__ coef,
     const FuncRec *__restrict__ F, const HarmTerm *__restrict__ T,
     const double *__restrict__ px, const double *__restrict__ py,
-    const double *__restrict__ pz, int cstride, int accum, double *__restrict__ cpart,
-    double *__restrict__ tpt) {
-  const int b = (int)(b0 + blockIdx.x);
-  const int lo = b_off[b], hi = b_off[b + 1];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const double *__restrict__ pz, double *__restrict__ cpart, double *__restrict__ tpart) {
+  // the pairs of a batch run on one XCD (workgroups are dealt to the eight
+  // XCDs in turn) and share its L2 for the tiles
+  const int xcd = blockIdx.x & 7, rr = blockIdx.x >> 3;
+  const int mgi = rr % nmg;
+  const int64_t b = b0 + (int64_t)(rr / nmg) * 8 + xcd;
+  if (b >= b1) return;
+  const int lo = b_off[b], n = b_off[b + 1] - lo;
+  if (2 * mgi >= n) return;  // uniform
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, q = lane >> 4;
-
-  __shared__ double Pk[FB][FB];   // Pk[k][i] = P(mu = i, nu = k)
-  __shared__ double Ph[FB][PT];   // Phi of the K block
-  __shared__ double Yh[FB][PT];   // Y of the K block
-  __shared__ double cfs[4][PT];
+  // Phi, Y of a stage; two buffers, declared apart so that a copy into one is
+  // known not to touch the other
+  __shared__ __attribute__((aligned(16))) double bufA[2][GSTG];
+  __shared__ __attribute__((aligned(16))) double bufB[2][GSTG];
   __shared__ double red[4][3][PT];
-  __shared__ double tsum[3][PT];
-
-  for (int e = threadIdx.x; e < 4 * PT; e += 256) {
-    const int c = e / PT, g = e % PT;
-    cfs[c][g] = coef[cstride * ((int64_t)b * PT + g) + c];
-  }
-  for (int e = threadIdx.x; e < 3 * PT; e += 256) (&tsum[0][0])[e] = 0.0;
-  __syncthreads();
-
-  for (int mi = lo; mi < hi; ++mi) {
-    const int fm = b_fbl[mi];
-    v4d accX[4], accW[4];
-    for (int j = 0; j < 4; ++j) accX[j] = accW[j] = v4d{0.0, 0.0, 0.0, 0.0};
-    for (int ki = lo; ki < hi; ++ki) {
-      const int fk = b_fbl[ki];
-      const double *psrc = Pd + (int64_t)(fk * FB) * nbf_pad + fm * FB;
-      const double *tsrc = tiles + (ki - s0) * narr * TILE;
+  const bool two = 2 * mgi + 1 < n;
+  const int im = lo + 2 * mgi + (two ? wv >> 1 : 0);
+  const int fm = __builtin_amdgcn_readfirstlane(b_fbl[im]);
+  const int mol = mt.blk_mol[fm], ld = mt.ld[mol];
+  const int row0 = two ? 32 * (wv & 1) : 16 * wv;  // of the block
+  const int mbase = fm - mt.blk_local[fm];
+  const double *prow =
+      Pt + mt.P_off[mol] + (int64_t)(mt.blk_local[fm] * FB + row0 + l16) * ld + 4 * q;
+  v4d accX[2][4], accW[2][4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = 2 * (u * 256 + (int)threadIdx.x);
-        const int r = e >> 6, c = e & 63;
-        *reinterpret_cast<double2 *>(&Pk[r][c]) =
-            *reinterpret_cast<const double2 *>(psrc + (int64_t)r * nbf_pad + c);
-        const double2 ph = *reinterpret_cast<const double2 *>(tsrc + e);
-        *reinterpret_cast<double2 *>(&Ph[r][c]) = ph;
-        double2 y;
-        y.x = 2.0 * cfs[0][c] * ph.x;
-        y.y = 2.0 * cfs[0][c + 1] * ph.y;
-        if (gga) {
+  for (int g = 0; g < 2; ++g)
 #pragma unroll
-          for (int d = 1; d <= 3; ++d) {
-            const double2 gd = *reinterpret_cast<const double2 *>(tsrc + d * TILE + e);
-            y.x += cfs[d][c] * gd.x;
-            y.y += cfs[d][c + 1] * gd.y;
+    for (int j = 0; j < 4; ++j) accX[g][j] = accW[g][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  auto issue = [&](int s, double (*dst)[GSTG], v4d (&a)[2]) {
+    const int ki = lo + (s >> 2), h = s & 3;
+    const int fk = __builtin_amdgcn_readfirstlane(b_fbl[ki]);
+    const double *p = prow + (fk - mbase) * FB + GS * h;
+    a[0] = *reinterpret_cast<const v4d *>(p);
+    if (two) a[1] = *reinterpret_cast<const v4d *>(p + (int64_t)16 * ld);
+    const double *src = tiles + (int64_t)(ki - s0) * narr * TILE + GSTG * h;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      // rows 2 rp, 2 rp + 1: 16 bytes per lane, halves exchanged in rows with
+      // bit 2 set (density_x_f64)
+      const int rp = 2 * wv + u, r = 2 * rp + (lane >> 5);
+      const int c = (lane & 31) ^ (((rp >> 1) & 1) << 3);
+      const double *g = src + r * PT + 2 * c;
+      __builtin_amdgcn_global_load_lds(g, &dst[0][rp * 2 * PT], 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(g + (int64_t)yarr * TILE, &dst[1][rp * 2 * PT], 16, 0, 0);
+    }
+  };
+  auto products = [&](const double (*cur)[GSTG], const v4d (&a)[2]) {
+    const int col = l16 ^ ((q & 1) << 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int op = 0; op < 2; ++op) {
+        double bv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bv[j] = cur[op][(4 * q + e) * PT + ((16 * j) ^ col)];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          if (g && !two) continue;  // uniform
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            v4d &acc = op ? accW[g][j] : accX[g][j];
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[g][e], bv[j], acc, 0, 0, 0);
           }
         }
-        *reinterpret_cast<double2 *>(&Yh[r][c]) = y;
       }
-      __syncthreads();
-#pragma unroll 4
-      for (int k0 = 0; k0 < FB; k0 += 4) {
-        const double a = Pk[k0 + q][16 * wv + l16];
+  };
+  v4d a0[2], a1[2];
+  issue(0, bufA, a0);
+  for (int s = 0; s < 4 * n; s += 2) {
+    wait_vm0();
+    __syncthreads();  // bufA complete, bufB free
+    issue(s + 1, bufB, a1);
+    products(bufA, a0);
+    wait_vm0();
+    __syncthreads();
+    if (s + 2 < 4 * n) issue(s + 2, bufA, a0);
+    products(bufB, a1);
+  }
+  // epilogue: wave w's part of the buffers holds eight rows of X, then of W
+  const int64_t gp = b * PT + lane;
+  const GradPoint pt{px[gp], py[gp], pz[gp], coef[4 * gp + 1], coef[4 * gp + 2], coef[4 * gp + 3]};
+  double tp[3] = {0.0, 0.0, 0.0};
+  double *Xs = (wv & 2 ? &bufB[0][0] : &bufA[0][0]) + (wv & 1) * GSTG, *Ws = Xs + 8 * GR_LD;
+  static_assert(2 * 8 * GR_LD <= GSTG, "eight rows of X and W per wave");
+  __syncthreads();  // the buffers' readers are done
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    if (g && !two) continue;
+    GradFuncs gf;
+    gf.load(F + (int64_t)fm * FB + row0 + 16 * g, lane);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          accX[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Ph[k0 + q][16 * j + l16], accX[j], 0,
-                                                          0, 0);
-          accW[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Yh[k0 + q][16 * j + l16], accW[j], 0,
-                                                          0, 0);
+          Xs[(4 * r + q) * GR_LD + 16 * j + l16] = accX[g][j][2 * h + r];
+          Ws[(4 * r + q) * GR_LD + 16 * j + l16] = accW[g][j][2 * h + r];
         }
-      }
-      __syncthreads();
+      grad_rows<8>(gf, 8 * h, T, pt, gga, Xs, Ws, lane,
+                   cpart + (im - s0) * GC + 3 * (row0 + 16 * g + 8 * h), tp);
     }
-    // Epilogue: c_mu(g) for the 16 (mu, g) pairs of this lane.
-    const double *tb = tiles + (mi - s0) * narr * TILE;
-    double cm[4][3], tp[4][3];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      for (int k = 0; k < 3; ++k) cm[r][k] = 0.0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      for (int k = 0; k < 3; ++k) tp[j][k] = 0.0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int mu = 16 * wv + 4 * r + q;
-      const FuncRec rec = F[fm * FB + mu];
-      if (rec.norm == 0.0) continue;  // padding function
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int g = 16 * j + l16;
-        const double X = accX[j][r], W = accW[j][r];
-        double c[3];
-        for (int k = 0; k < 3; ++k) c[k] = -2.0 * tb[(1 + k) * TILE + mu * PT + g] * W;
-        if (gga) {
-          const int64_t gp = (int64_t)b * PT + g;
-          double v, gr[3], h[6];
-          sto_value_grad_hess(rec, T, px[gp], py[gp], pz[gp], v, gr, h);
-          const double bx = cfs[1][g], by = cfs[2][g], bz = cfs[3][g];
-          c[0] -= 2.0 * (h[0] * bx + h[1] * by + h[2] * bz) * X;
-          c[1] -= 2.0 * (h[1] * bx + h[3] * by + h[4] * bz) * X;
-          c[2] -= 2.0 * (h[2] * bx + h[4] * by + h[5] * bz) * X;
-        }
-        for (int k = 0; k < 3; ++k) {
-          cm[r][k] += c[k];
-          tp[j][k] += c[k];
-        }
-      }
-    }
-    // per function: sum over the batch's points (j in registers, l16 lanes)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      for (int k = 0; k < 3; ++k) {
-        double v = cm[r][k];
-        v += __shfl_xor(v, 1);
-        v += __shfl_xor(v, 2);
-        v += __shfl_xor(v, 4);
-        v += __shfl_xor(v, 8);
-        if (l16 == 0) cpart[(mi - s0) * GC + (16 * wv + 4 * r + q) * 3 + k] = v;
-      }
-    // per point: sum over this block's functions (q lanes, then waves)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      for (int k = 0; k < 3; ++k) {
-        double v = tp[j][k];
-        v += __shfl_xor(v, 16);
-        v += __shfl_xor(v, 32);
-        if (q == 0) red[wv][k][16 * j + l16] = v;
-      }
-    __syncthreads();
-    if (threadIdx.x < 3 * PT) {
-      const int k = threadIdx.x / PT, g = threadIdx.x % PT;
-      tsum[k][g] += red[0][k][g] + red[1][k][g] + red[2][k][g] + red[3][k][g];
-    }
-    __syncthreads();
   }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) red[wv][k][lane] = tp[k];
+  __syncthreads();
   if (threadIdx.x < 3 * PT) {
     const int k = threadIdx.x / PT, g = threadIdx.x % PT;
-    const int64_t e = 3 * ((int64_t)b * PT + g) + k;
-    tpt[e] = (accum ? tpt[e] : 0.0) - tsum[k][g];
+    tpart[(int64_t)(lo + 2 * mgi - s0) * (4 * PT) + threadIdx.x] =
+        ((red[0][k][g] + red[1][k][g]) + red[2][k][g]) + red[3][k][g];
   }
+}
+
+// tpt[3 point + k] = -(sum over a batch's block pairs), or that added to tpt
+__global__ void __launch_bounds__(192) grad_points_kernel(int64_t s0, int64_t b0,
+                                                          const int *__restrict__ b_off,
+                                                          const double *__restrict__ tpart,
+                                                          int accum, double *__restrict__ tpt) {
+  const int64_t b = b0 + blockIdx.x;
+  const int k = threadIdx.x / PT, g = threadIdx.x % PT;
+  double t = 0.0;
+  for (int s = b_off[b]; s < b_off[b + 1]; s += 2) t += tpart[(s - s0) * (4 * PT) + threadIdx.x];
+  const int64_t e = 3 * (b * PT + g) + k;
+  tpt[e] = (accum ? tpt[e] : 0.0) - t;
 }
 
 // gacc[seg][I * 192 + t] += sum over batches of segment seg of cpart of block I
@@ -245,40 +256,6 @@ __device__ double becke_cell(int i, int natoms, const double *C, const double2 *
     if (Pi == 0.0) break;
   }
   return Pi;
-}
-
-// DPP move of a double (both halves) from the lane that CTRL selects inside the
-// same row of 16 lanes; every lane must be active.
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, false);
-  const unsigned hi =
-      (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// Sum over the 64 lanes of a wave; every lane must be active, and every lane
-// receives the same value.  Inside each row of 16 lanes by DPP moves (quad
-// permutations for lane ^ 1 and lane ^ 2, then the half-row and row mirrors):
-// each step adds the same two partial sums in every lane (a + b and b + a are
-// the same double), so all lanes of a row hold the same row sum.  The four row
-// sums are read out of lanes 0, 16, 32 and 48 and added in a fixed order.
-// No LDS instruction is involved (lane shuffles through ds_bpermute would
-// put twelve dependent LDS round trips in every sum).
-__device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_move<0xB1>(v);   // quad_perm [1, 0, 3, 2]
-  v += dpp_move<0x4E>(v);   // quad_perm [2, 3, 0, 1]
-  v += dpp_move<0x141>(v);  // row_half_mirror: lane 7 - i of each 8
-  v += dpp_move<0x140>(v);  // row_mirror: lane 15 - i of each 16
-  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 // One thread per sorted point, one wave per workgroup; per-atom sums in LDS
@@ -431,12 +408,18 @@ __global__ void __launch_bounds__(256) colsum_kernel(int nrow, int ncol,
 
 // ---------------------------------------------------------------------------
 void vkg_basis(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
-               const double *Pd, int narr, int gga, const double *tiles, const double *coef,
-               int cstride, bool accum, double *cpart, double *tpt) {
+               const double *Pt, int narr, int yarr, int gga, const double *tiles,
+               const double *coef, bool accum, double *cpart, double *tpart, double *tpt) {
   if (b1 <= b0) return;
-  hipLaunchKernelGGL(grad_basis_f64, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, pl.nbf_pad, Pd,
-                     pl.b_off.p, pl.b_fbl.p, s0, b0, narr, gga, tiles, coef, pl.funcs.p,
-                     pl.terms.p, pl.px.p, pl.py.p, pl.pz.p, cstride, accum ? 1 : 0, cpart, tpt);
+  const int nmg = (pl.max_mol_nfb + 1) / 2;
+  const int64_t nwg = (b1 - b0 + 7) / 8 * 8 * nmg;
+  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "gradient grid too large");
+  hipLaunchKernelGGL(grad_basis_f64, dim3((unsigned)nwg), dim3(256), 0, s, pl.tab(), Pt, pl.b_off.p,
+                     pl.b_fbl.p, s0, b0, b1, nmg, narr, yarr, gga, tiles, coef, pl.funcs.p,
+                     pl.terms.p, pl.px.p, pl.py.p, pl.pz.p, cpart, tpart);
+  NKX_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(grad_points_kernel, dim3((unsigned)(b1 - b0)), dim3(192), 0, s, s0, b0,
+                     pl.b_off.p, tpart, accum ? 1 : 0, tpt);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -13,9 +13,9 @@
 // (Phi, rows = points, k = functions) and writes Y in the same orientation
 // into the Z section, so both are B operands of P[mu][nu] with per-point
 // exponents.
+#include "grad_rows.hpp"
 #include "nkx_internal.hpp"
 #include "slices_i8.hpp"
-#include "sto_eval.hpp"
 #include "vxc_kernels.hpp"
 
 namespace nkx {
@@ -107,11 +107,11 @@ __global__ void __launch_bounds__(256) y_slots_i8(int64_t s0, const int *__restr
 // order; the K slot's Pm and Y sections are copied into LDS once per step for
 // the four waves (two buffers: the next step's copies are issued while the
 // current step computes; a second register set for the P fragments would
-// cost the occupancy).  The epilogue, after the last K of
-// an I, is the FP64 form's: STO gradient (and Hessian for GGA) in FP64 per
-// (mu, g), per-function sums over the batch's points into cpart, per-point
-// sums over functions into tpt (with the sign of the point-motion term).
-__global__ void __launch_bounds__(256) grad_basis_i8(
+// cost the occupancy).  The epilogue, after the last K of an I, is the FP64
+// form's (grad_rows.hpp): per-function sums over the batch's points into cpart,
+// per-point sums over functions into tpt (with the sign of the point-motion
+// term).
+__global__ void __launch_bounds__(256, 2) grad_basis_i8(
     MolTab mt, const signed char *__restrict__ Ps, const int *__restrict__ b_off,
     const int *__restrict__ b_fbl, int64_t s0, int64_t b0, int gga,
     const signed char *__restrict__ store, const double *__restrict__ coef,
@@ -129,15 +129,17 @@ __global__ void __launch_bounds__(256) grad_basis_i8(
   // a copy into one is known not to touch the other
   __shared__ __attribute__((aligned(16))) signed char bufA[2][SEC];
   __shared__ __attribute__((aligned(16))) signed char bufB[2][SEC];
-  __shared__ double cfs[4][PT];
-  __shared__ double red[4][3][PT];
-  __shared__ double tsum[3][PT];
   __shared__ int lbl[MAXNFB];  // local block index of the batch's live blocks
-  for (int e = threadIdx.x; e < 4 * PT; e += 256) {
+  __shared__ double red[4][3][PT];
+  // the epilogue's points (coordinates, b), kept in LDS for their registers
+  __shared__ double pts[6][PT];
+  for (int e = threadIdx.x; e < 6 * PT; e += 256) {
     const int c = e / PT, g = e % PT;
-    cfs[c][g] = coef[4 * ((int64_t)b * PT + g) + c];
+    const int64_t gp = (int64_t)b * PT + g;
+    pts[c][g] = c == 0 ? px[gp] : c == 1 ? py[gp] : c == 2 ? pz[gp] : coef[4 * gp + c - 2];
   }
-  for (int e = threadIdx.x; e < 3 * PT; e += 256) (&tsum[0][0])[e] = 0.0;
+  // this lane's point: sums over this wave's functions
+  double tp[3] = {0.0, 0.0, 0.0};
   const int n = hi - lo;
   for (int k = threadIdx.x; k < n; k += 256) lbl[k] = mt.blk_local[b_fbl[lo + k]];
   __syncthreads();
@@ -146,7 +148,6 @@ __global__ void __launch_bounds__(256) grad_basis_i8(
     const int mol = mt.blk_mol[b_fbl[lo]];
     const signed char *pbase = Ps + mt.Ps_off[mol];
     const int nfbm = mt.nfb[mol];
-    const int nsteps = n * n;
     // the K slot's sections of a step -> LDS buffer dst (direct copies)
     auto issue = [&](int st, signed char (*dst)[SEC]) {
       const int64_t sk = lo + st % n - s0;
@@ -154,99 +155,37 @@ __global__ void __launch_bounds__(256) grad_basis_i8(
       dma_section<4>(ybase + sk * ystride, &dst[1][0], (wv + 2) & 3, lane);
     };
     double X[4][4], W[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) X[j][r] = W[j][r] = 0.0;
-    // Epilogue of block I = b_fbl[mi]: c_mu(g) for the 16 (mu, g) pairs of
-    // this lane; result register r of lane l holds row 4 (l / 16) + r, point
+    // Epilogue of block I = b_fbl[mi] through the two LDS buffers (X and W of
+    // 64 rows fit them): wave w takes 16 functions, a point per lane.
+    // X and W leave the registers, which the epilogue needs; the next block's
+    // first copies wait for its end (the other workgroup of the CU runs
+    // meanwhile).  Result register r of lane l holds row 4 (l / 16) + r, point
     // l % 16 of a tile.
     auto epilogue = [&](int mi) {
-      const int fm = b_fbl[mi];
-      double cm[4][3], tp[4][3];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        for (int k = 0; k < 3; ++k) cm[r][k] = 0.0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        for (int k = 0; k < 3; ++k) tp[j][k] = 0.0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mu = 16 * wv + 4 * q + r;
-        const FuncRec rec = F[fm * FB + mu];
-        if (rec.norm == 0.0) continue;  // padding function
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int g = 16 * j + l16;
-          const int64_t gp = (int64_t)b * PT + g;
-          double c[3];
-          if (gga) {
-            double v, gr[3], h[6];
-            sto_value_grad_hess(rec, T, px[gp], py[gp], pz[gp], v, gr, h);
-            const double bx = cfs[1][g], by = cfs[2][g], bz = cfs[3][g];
-            const double x = X[j][r], w = W[j][r];
-            c[0] = -2.0 * (gr[0] * w + (h[0] * bx + h[1] * by + h[2] * bz) * x);
-            c[1] = -2.0 * (gr[1] * w + (h[1] * bx + h[3] * by + h[4] * bz) * x);
-            c[2] = -2.0 * (gr[2] * w + (h[2] * bx + h[4] * by + h[5] * bz) * x);
-          } else {
-            double v, gx, gy, gz;
-            sto_value_grad<double>(rec, T, px[gp], py[gp], pz[gp], v, gx, gy, gz);
-            const double w = W[j][r];
-            c[0] = -2.0 * gx * w;
-            c[1] = -2.0 * gy * w;
-            c[2] = -2.0 * gz * w;
-          }
-          for (int k = 0; k < 3; ++k) {
-            cm[r][k] += c[k];
-            tp[j][k] += c[k];
-          }
-        }
-      }
-      // per function: sum over the batch's points (j in registers, l16 lanes)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        for (int k = 0; k < 3; ++k) {
-          double v = cm[r][k];
-          v += __shfl_xor(v, 1);
-          v += __shfl_xor(v, 2);
-          v += __shfl_xor(v, 4);
-          v += __shfl_xor(v, 8);
-          if (l16 == 0) cpart[(mi - s0) * GC + (16 * wv + 4 * q + r) * 3 + k] = v;
-        }
-      // per point: sum over this block's functions (q lanes, then waves)
+      GradFuncs gf;
+      gf.load(F + (int64_t)__builtin_amdgcn_readfirstlane(b_fbl[mi]) * FB + 16 * wv, lane);
+      double *Xs = reinterpret_cast<double *>(&bufA[0][0]);
+      double *Ws = reinterpret_cast<double *>(&bufB[0][0]);
+      static_assert(sizeof(bufA) >= FB * GR_LD * sizeof(double), "X of a block in a buffer");
+      __syncthreads();  // the buffers' readers are done
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        for (int k = 0; k < 3; ++k) {
-          double v = tp[j][k];
-          v += __shfl_xor(v, 16);
-          v += __shfl_xor(v, 32);
-          if (q == 0) red[wv][k][16 * j + l16] = v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          Xs[(16 * wv + 4 * q + r) * GR_LD + 16 * j + l16] = X[j][r];
+          Ws[(16 * wv + 4 * q + r) * GR_LD + 16 * j + l16] = W[j][r];
         }
-      __syncthreads();
-      if (threadIdx.x < 3 * PT) {
-        const int k = threadIdx.x / PT, g = threadIdx.x % PT;
-        tsum[k][g] += red[0][k][g] + red[1][k][g] + red[2][k][g] + red[3][k][g];
-      }
-      __syncthreads();
+      // (the rows of a wave are the functions that it takes: no barrier)
+      const GradPoint pt{pts[0][lane], pts[1][lane], pts[2][lane],
+                         pts[3][lane], pts[4][lane], pts[5][lane]};
+      grad_rows<16>(gf, 0, T, pt, gga, Xs + 16 * wv * GR_LD, Ws + 16 * wv * GR_LD, lane,
+                cpart + (mi - s0) * GC + 48 * wv, tp);
+      __syncthreads();  // the buffers are free
     };
-    // one step (I, K): its P fragment, wait for its sections, issue the next
-    // step's copies, then the tile products; after the last K of an I, its
-    // epilogue
-    auto step = [&](int st, signed char (*cur)[SEC], signed char (*nxt)[SEC]) {
-      const int ii = st / n, kk = st - ii * n;
-      const signed char *pa =
-          pbase + ((int64_t)__builtin_amdgcn_readfirstlane(lbl[ii]) * nfbm +
-                   __builtin_amdgcn_readfirstlane(lbl[kk])) * SEC;
-      v4i A[4];
-#pragma unroll
-      for (int p = 0; p < 4; ++p) A[p] = ld16(pa + p * PLANE + (wv * 64 + lane) * 16);
-      const int eA = *reinterpret_cast<const int *>(pa + 4 * PLANE + 16 * wv + 4 * q);
-      wait_vm0();
-      __syncthreads();  // buffer cur complete, nxt free
-      if (st + 1 < nsteps) issue(st + 1, nxt);
+    auto products = [&](signed char (*cur)[SEC], const v4i (&Ac)[4], int eAc) {
       double sA[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sA[r] = pow2_or_zero((int)(signed char)(eA >> (8 * r)));
+      for (int r = 0; r < 4; ++r) sA[r] = pow2_or_zero((int)(signed char)(eAc >> (8 * r)));
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -258,7 +197,7 @@ __global__ void __launch_bounds__(256) grad_basis_i8(
           const int eB = sec[4 * PLANE + 16 * j + l16];
           const double sB = eB == -127 ? 0.0 : pow2(eB - 19);
           int hi4[4], lo4[4];
-          tile_product(A, B, hi4, lo4);
+          tile_product(Ac, B, hi4, lo4);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const double v = fma((double)lo4[r], 0x1p-14, (double)hi4[r]) * (sA[r] * sB);
@@ -269,24 +208,60 @@ __global__ void __launch_bounds__(256) grad_basis_i8(
           }
         }
       }
-      if (kk == n - 1) {  // uniform: the last K of block I
-        epilogue(lo + ii);
+    };
+    // one step (I, K): its P fragment, wait for its sections, issue the next
+    // step's copies (within a block), then the tile products.  (One loop over
+    // all steps: as nested loops their addresses become induction variables
+    // that cost 80 registers.)
+    auto step = [&](int st, signed char (*cur)[SEC], signed char (*nxt)[SEC]) {
+      const int ii = st / n, kk = st - ii * n;
+      const signed char *pa =
+          pbase + ((int64_t)__builtin_amdgcn_readfirstlane(lbl[ii]) * nfbm +
+                   __builtin_amdgcn_readfirstlane(lbl[kk])) * SEC;
+      v4i A[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) A[p] = ld16(pa + p * PLANE + (wv * 64 + lane) * 16);
+      const int eA = *reinterpret_cast<const int *>(pa + 4 * PLANE + 16 * wv + 4 * q);
+      wait_vm0();
+      __syncthreads();  // buffer cur complete, nxt free
+      if (kk + 1 < n) issue(st + 1, nxt);
+      products(cur, A, eA);
+    };
+    const int nsteps = n * n;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) X[j][r] = W[j][r] = 0.0;
+    issue(0, bufA);
+    for (int st = 0; st < nsteps; ++st) {
+      if (st & 1)
+        step(st, bufB, bufA);
+      else
+        step(st, bufA, bufB);
+      if ((st + 1) % n == 0) {  // uniform: the last K of block I
+        epilogue(lo + st / n);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) X[j][r] = W[j][r] = 0.0;
+        if (st + 1 < nsteps) {
+          if (st & 1)
+            issue(st + 1, bufA);
+          else
+            issue(st + 1, bufB);
+        }
       }
-    };
-    issue(0, bufA);
-    for (int st = 0; st < nsteps; st += 2) {
-      step(st, bufA, bufB);
-      if (st + 1 < nsteps) step(st + 1, bufB, bufA);
     }
   }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 3; ++k) red[wv][k][lane] = tp[k];
+  __syncthreads();
   if (threadIdx.x < 3 * PT) {
     const int k = threadIdx.x / PT, g = threadIdx.x % PT;
     const int64_t e = 3 * ((int64_t)b * PT + g) + k;
-    tpt[e] = (accum ? tpt[e] : 0.0) - tsum[k][g];
+    const double t = ((red[0][k][g] + red[1][k][g]) + red[2][k][g]) + red[3][k][g];
+    tpt[e] = (accum ? tpt[e] : 0.0) - t;
   }
 }
 

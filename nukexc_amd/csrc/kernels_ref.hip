@@ -15,6 +15,7 @@
 // of their size is written.
 #include <algorithm>
 
+#include "lane_sums.hpp"
 #include "nkx_internal.hpp"
 #include "xc_functionals.hpp"
 #include "xc_polarized.hpp"
@@ -41,22 +42,6 @@ struct RefGrads {
 struct RhoOut {
   double *rho, *gx, *gy, *gz, *sigma;  // all but rho may be NULL
 };
-
-// Sum of each of 16 values over the 16 lanes of a row; lane l returns the
-// total of value bitrev4(l).  Fifteen exchanges: each halves the values held.
-__device__ __forceinline__ double row_sum16(double (&v)[16], int l16) {
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int half = 8 >> b;
-    const bool up = (l16 >> b) & 1;
-#pragma unroll
-    for (int i = 0; i < half; ++i) {
-      const double lo = v[i], hi = v[i + half];
-      v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, 1 << b);
-    }
-  }
-  return v[0];
-}
 
 // ---------------------------------------------------------------------------
 // One workgroup of four waves per 64 points, a wave per 16.  MFMA rows are
@@ -176,7 +161,7 @@ __device__ __forceinline__ void mo_pass(int nbf, const double *const (&row)[NARR
     }
     if constexpr (NARR == 4) {
       const double tot = row_sum16(v, l16);
-      const int k = ((l16 & 1) << 3) | ((l16 & 2) << 1) | ((l16 & 4) >> 1) | ((l16 & 8) >> 3);
+      const int k = bitrev4(l16);
       red[s][k >> 2][16 * wv + 4 * (k & 3) + q] += tot;
     } else {
 #pragma unroll

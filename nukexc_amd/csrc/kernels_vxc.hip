@@ -23,7 +23,7 @@
 #include <algorithm>
 
 #include "nkx_internal.hpp"
-#include "sto_eval.hpp"
+#include "sto_run.hpp"
 #include "vxc_kernels.hpp"
 
 namespace nkx {
@@ -39,6 +39,8 @@ constexpr int PT = 64;   // points per batch
 constexpr int TILE = FB * PT;
 
 // ---------------------------------------------------------------------------
+// One workgroup per live slot: thread t takes the 16 consecutive functions
+// 16 (t / 64) .. +15 of the block at point t % 64 (sto_run.hpp).
 __global__ void __launch_bounds__(256) colloc_tiles_f64(
     int64_t s0, const int *__restrict__ slot_b, const int *__restrict__ b_fbl,
     const FuncRec *__restrict__ F, const HarmTerm *__restrict__ T,
@@ -46,29 +48,24 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
     const double *__restrict__ pz, int narr, int gga, double *__restrict__ tiles) {
   const int64_t s = s0 + blockIdx.x;
   const int b = slot_b[s];
-  const int fb = b_fbl[s];
-  __shared__ FuncRec fr[FB];
-  if (threadIdx.x < FB) fr[threadIdx.x] = F[fb * FB + threadIdx.x];
-  __syncthreads();
+  const int f0 = 16 * __builtin_amdgcn_readfirstlane(threadIdx.x / PT);
+  const FuncRec *fr = F + (int64_t)b_fbl[s] * FB + f0;
   const int g = threadIdx.x & (PT - 1);
-  const int row = threadIdx.x / PT;
   const int64_t gp = (int64_t)b * PT + g;
   const double x = px[gp], y = py[gp], z = pz[gp];
-  double *base = tiles + (int64_t)blockIdx.x * narr * TILE;
+  double *base = tiles + (int64_t)blockIdx.x * narr * TILE + f0 * PT + g;
+  StoRun run;
 #pragma unroll 1
-  for (int f = row; f < FB; f += 256 / PT) {
-    const FuncRec rec = fr[f];
-    const int e = f * PT + g;
+  for (int i = 0; i < 16; ++i) {
+    double v, gr[3];
     if (gga) {
-      double v, a, bb, c;
-      sto_value_grad<double>(rec, T, x, y, z, v, a, bb, c);
-      base[e] = v;
-      base[TILE + e] = a;
-      base[2 * TILE + e] = bb;
-      base[3 * TILE + e] = c;
+      run.eval<true, false>(fr[i], fr[i ? i - 1 : 0], i == 0, T, x, y, z, v, gr);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) base[(c + 1) * TILE + i * PT] = gr[c];
     } else {
-      base[e] = sto_value<double>(rec, T, x, y, z);
+      run.eval<false, false>(fr[i], fr[i ? i - 1 : 0], i == 0, T, x, y, z, v, gr);
     }
+    base[i * PT] = v;
   }
 }
 

@@ -5,7 +5,7 @@
 #include <type_traits>
 
 #include "nkx_internal.hpp"
-#include "sto_eval.hpp"
+#include "sto_run.hpp"
 #include "vxc_kernels.hpp"
 #include "slices_i8.hpp"
 #include "xc_functionals.hpp"
@@ -42,47 +42,19 @@ __global__ void __launch_bounds__(256) colloc_tiles_i8(
   const double x = px[gp], y = py[gp], z = pz[gp];
   signed char *base = store + (int64_t)blockIdx.x * slot_bytes_i8(gga);
   float *G = reinterpret_cast<float *>(base + OFF_G);
-  double dx = 0.0, dy = 0.0, dz = 0.0, r = 1.0, rinv = 1.0, R = 0.0, common = 0.0;
+  StoRun run;
 #pragma unroll 1
   for (int i = 0; i < 16; ++i) {
     const int f = f0 + i;
-    const FuncRec rec = fr[f];
-    const bool newc =
-        i == 0 || rec.cx != fr[f - 1].cx || rec.cy != fr[f - 1].cy || rec.cz != fr[f - 1].cz;
-    if (newc) {
-      dx = x - rec.cx;
-      dy = y - rec.cy;
-      dz = z - rec.cz;
-      r = sqrt(dx * dx + dy * dy + dz * dz);
-      rinv = 1.0 / r;
-    }
-    if (newc || rec.zeta != fr[f - 1].zeta || rec.k != fr[f - 1].k ||
-        rec.norm != fr[f - 1].norm) {
-      R = rec.norm * ipow(r, rec.k) * exp_neg_mixed(rec.zeta * r);
-      common = ((double)rec.k * rinv - rec.zeta) * R * rinv;
-    }
-    double S = 0.0, Sx = 0.0, Sy = 0.0, Sz = 0.0;
-    for (int t = 0; t < rec.term_cnt; ++t) {
-      const HarmTerm h = T[rec.term_off + t];
-      const double xa1 = ipow(dx, h.a > 0 ? h.a - 1 : 0);
-      const double yb1 = ipow(dy, h.b > 0 ? h.b - 1 : 0);
-      const double zc1 = ipow(dz, h.c > 0 ? h.c - 1 : 0);
-      const double xa = h.a > 0 ? xa1 * dx : 1.0;
-      const double yb = h.b > 0 ? yb1 * dy : 1.0;
-      const double zc = h.c > 0 ? zc1 * dz : 1.0;
-      S += h.coef * xa * yb * zc;
-      if (gga) {
-        if (h.a > 0) Sx += h.coef * h.a * xa1 * yb * zc;
-        if (h.b > 0) Sy += h.coef * h.b * xa * yb1 * zc;
-        if (h.c > 0) Sz += h.coef * h.c * xa * yb * zc1;
-      }
-    }
-    v[f][g] = R * S;
+    double val, gr[3];
     if (gga) {
-      G[f * PT + g] = (float)(R * Sx + S * (dx * common));
-      G[TILE + f * PT + g] = (float)(R * Sy + S * (dy * common));
-      G[2 * TILE + f * PT + g] = (float)(R * Sz + S * (dz * common));
+      run.eval<true, true>(fr[f], fr[i ? f - 1 : f], i == 0, T, x, y, z, val, gr);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) G[c * TILE + f * PT + g] = (float)gr[c];
+    } else {
+      run.eval<false, true>(fr[f], fr[i ? f - 1 : f], i == 0, T, x, y, z, val, gr);
     }
+    v[f][g] = val;
   }
   __syncthreads();
   {

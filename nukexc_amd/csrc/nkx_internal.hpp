@@ -128,13 +128,16 @@ struct HarmTerm {
   int a, b, c, pad;
 };
 
+// Function type code of a FuncRec.
+inline int func_type(int l, int m) { return l <= 2 ? l * l + l + m : -1; }
+
 // Per-function record consumed by the collocation kernels.
 struct FuncRec {
   double cx, cy, cz, zeta, norm;
   int k;          // n - l - 1, power of r in the radial part
   int term_off;   // first HarmTerm of this function
   int term_cnt;   // number of HarmTerms
-  int pad;
+  int type;       // l l + l + m to l = 2 (closed forms), -1 beyond
 };
 
 struct GridState {

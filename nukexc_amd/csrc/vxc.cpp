@@ -128,12 +128,14 @@ PlanPart make_part(int64_t npts, const BasisHost &B, double tol) {
       r.k = B.n[i] - B.l[i] - 1;
       r.term_off = (int)pt.terms.size();
       r.term_cnt = (int)t.size();
+      r.type = func_type(B.l[i], B.m[i]);
       pt.terms.insert(pt.terms.end(), t.begin(), t.end());
     } else {
       r.zeta = 1.0;
       r.norm = 0.0;
       r.term_off = 0;
       r.term_cnt = 0;
+      r.type = 0;
     }
     pt.fr[sp] = r;
   }
@@ -573,7 +575,7 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
       tt = tm.begin(kStageZ, s);
       if (!mixed) {
         fp64_functional(s, nspin, b0, b1, s0, pl, ig, xl, ws, b.slots_alloc, nullptr);
-        vk_z_slots(s, s0, s1, pl, narr, nspin, ig, ws.coef.p, ws.tiles64.p);
+        vk_z_slots(s, s0, s1, pl, narr, nspin, ig, 1.0, ws.coef.p, ws.tiles64.p);
       } else if (nspin == 2)
         vkm_density_finish_pol(s, b0, b1, s0, pl, ig, ws.mstore.p, ws.zstore_b.p, xl,
                                ws.coef.p, ws.coef.p + (size_t)4 * pl.npts_pad, ws.blockEN.p,
@@ -901,7 +903,7 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
     if (nspin == 2) ws.zstore_b.reserve((size_t)slots_alloc * mixed_zsection_bytes());
   } else {
     ws.tiles64.reserve((size_t)slots_alloc * narr * FB * PT);
-    ws.Pd.reserve((size_t)2 * nspin * pl.P_total);  // P, then its transpose
+    ws.Pd.reserve((size_t)nspin * pl.P_total);
   }
   ws.dpart.reserve(nspin * dsz);
   ws.coef.reserve((size_t)4 * nspin * pl.npts_pad);
@@ -923,9 +925,8 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
     if (mixed)
       vkm_gather_p(s, pl.nbf, pl.mol_nfb_h[0], pl.fperm_d.p, P[sp], ws.Ps.p + sp * psb);
     else
-      for (int tr = 0; tr < 2; ++tr)
-        vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, tr == 1, P[sp],
-                    ws.Pd.p + (size_t)(tr * nspin + sp) * pl.P_total);
+      vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, true, P[sp],
+                  ws.Pd.p + (size_t)sp * pl.P_total);
   }
   vk_fill0(s, gacc, (int64_t)n_ga);
   const int ig = gga ? 1 : 0;
@@ -958,13 +959,16 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
         vkg_fold(s, b0, b1, s0, pl, nseg, cpart, gacc);
       }
     } else {
-      vk_colloc(s, s0, s1, pl, narr, 1, ws.tiles64.p);
-      vk_density(s, nspin, 2, b0, b1, s0, pl, ws.Pd.p + (size_t)nspin * pl.P_total, narr, ig,
-                 ws.tiles64.p, ws.dpart.p, (int64_t)dsz);
+      vk_colloc(s, s0, s1, pl, narr, ig, ws.tiles64.p);
+      vk_density(s, nspin, 2, b0, b1, s0, pl, ws.Pd.p, narr, ig, ws.tiles64.p, ws.dpart.p,
+                 (int64_t)dsz);
       fp64_functional(s, nspin, b0, b1, s0, pl, ig, xl, ws, slots_alloc, epoint);
+      vk_z_slots(s, s0, s1, pl, narr, nspin, ig, 2.0, ws.coef.p, ws.tiles64.p);
+      // (the density partials are done with: scratch of the point sums)
       for (int sp = 0; sp < nspin; ++sp) {
-        vkg_basis(s, b0, b1, s0, pl, ws.Pd.p + (size_t)sp * pl.P_total, narr, ig, ws.tiles64.p,
-                  ws.coef.p + (size_t)4 * sp * pl.npts_pad, 4, sp > 0, cpart, tpt);
+        vkg_basis(s, b0, b1, s0, pl, ws.Pd.p + (size_t)sp * pl.P_total, narr, narr - nspin + sp,
+                  ig, ws.tiles64.p, ws.coef.p + (size_t)4 * sp * pl.npts_pad, sp > 0, cpart,
+                  ws.dpart.p, tpt);
         vkg_fold(s, b0, b1, s0, pl, nseg, cpart, gacc);
       }
     }

@@ -29,12 +29,13 @@ void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, 
 // Pt: the gathered transposes of nspin density matrices; group: consecutive
 // batches per workgroup (1, 2 or 4).  The functional is vkm_density_functional
 // or vkm_density_finish_pol (coef per spin 4 npts_pad apart), then vk_z_slots
-// forms the Z arrays.
+// forms the Z arrays, ascale a Phi + b . grad Phi (ascale 1; 2 for the Y of the
+// gradient).
 void vk_density(hipStream_t s, int nspin, int group, int64_t b0, int64_t b1, int64_t s0,
                 const Plan &pl, const double *Pt, int narr, int gga, const double *tiles,
                 double *part, int64_t pstride);
 void vk_z_slots(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int nspin,
-                int gga, const double *coef, double *tiles);
+                int gga, double ascale, const double *coef, double *tiles);
 // screened-grid set-up (kernels_sparse.hip): Morton order of the points
 // (AoS; w, owner may be NULL) in place and the box of each run of per points
 // (6 doubles per box); the CSR list of functions (host centres and radii)
@@ -121,13 +122,14 @@ void vkb_vgemm(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, con
 
 // nuclear gradient (kernels_grad.hip)
 // grad_basis: per batch, per-function partial sums of the basis-centre
-// derivative over the batch (cpart[(slot - s0) * 64 * 3 + mu * 3 + k]) and the
-// per-point sum tpt[3 * gp + k] with the sign of the point-motion term.
-// coef of the spin of Pd with a stride of cstride doubles per point; accum
-// adds into tpt (second spin) instead of writing it
+// derivative over the batch (cpart[(slot - s0) * 64 * 3 + mu * 3 + k]; only
+// their sums per atom count) and the per-point sum tpt[3 * gp + k] with the sign
+// of the point-motion term.  Pt: the gathered transpose of P; Y = 2 a Phi + b .
+// grad Phi in tile array yarr (vk_z_slots with ascale 2); tpart: 256 doubles of
+// scratch per slot; accum adds into tpt (second spin) instead of writing it
 void vkg_basis(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
-               const double *Pd, int narr, int gga, const double *tiles, const double *coef,
-               int cstride, bool accum, double *cpart, double *tpt);
+               const double *Pt, int narr, int yarr, int gga, const double *tiles,
+               const double *coef, bool accum, double *cpart, double *tpart, double *tpt);
 // mixed form (kernels_grad_i8.hip), on the int8 slot store after vkm_colloc,
 // vkm_density (split shape) and vkm_density_functional: Y = 2 a Phi + b . grad
 // Phi slices per slot (rows = points), then X = P Phi and W = P Y on integer
