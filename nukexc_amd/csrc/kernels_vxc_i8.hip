@@ -816,8 +816,11 @@ __global__ void __launch_bounds__(256) z_slots_i8(int64_t s0, const int *__restr
 // V contraction on 2 x 2 block super-tiles: acc(I, J) += Phi_I Z_J^T +
 // Z_I Phi_J^T over the batches where I and J are live, for the four tiles
 // (I_a, J_b) of a super-pair (blocks I_0 < I_1, J_0 < J_1 of one molecule;
-// a missing second block is -1; on the diagonal I_1 x J_0 is the transpose
-// of I_0 x J_1 and has no pair index).  One workgroup of eight waves per
+// a missing second block is -1).  On the diagonal (I = J) only Vbar = Phi Z^T of
+// the four tiles is formed and added to its transpose at the end: half the
+// products, and no wave idles for the tile I_1 x J_0, which has no pair index
+// (a mixed benzene build, whose two blocks are one diagonal super-pair: 402 ->
+// 258 us, an 8-molecule set 628 -> 441 us).  One workgroup of eight waves per
 // (super-pair, split); its batches b = lo + split + nsplit i are taken in
 // windows of 512 candidates, compacted in ascending order into an LDS list
 // of the four slots.  The Z and F sections of the J slots (shared by all
@@ -832,37 +835,36 @@ __global__ void __launch_bounds__(256) z_slots_i8(int64_t s0, const int *__restr
 // ascending order, F_I Z_J^T before Z_I F_J^T within a batch, as in the
 // one-pair kernel.  Each tile goes to vpart at its pair index (written by
 // the first chunk of a build, added by the later ones).
-__global__ void __launch_bounds__(512) vgemm_i8(
-    int nsp, int nsplit, const int4 *__restrict__ sp_blk, const int4 *__restrict__ sp_pidx,
-    int npairs, const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1,
-    int64_t s0, int gga, const signed char *__restrict__ store,
-    const signed char *__restrict__ zbase, int64_t zstride, int first,
-    double *__restrict__ vpart) {
-  // split-major: the super-pairs of one split run together and walk the same
-  // batches, sharing each batch's slots in the caches
-  const int sp = blockIdx.x % nsp;
-  const int split = blockIdx.x / nsp;
-  const int4 blk = sp_blk[sp];
+//
+// A wave has NG groups of 16 rows and NJ column groups of 16 of its tile: 32
+// rows x 64 columns (2, 4); with one J block 16 rows each (1, 4); with one block
+// in all 16 rows x 32 columns (1, 2).
+template <int NG, int NJ>
+__device__ __forceinline__ void vgemm_i8_tile(
+    int4 blk, int4 pix, int split, int nsplit, int npairs, const int *__restrict__ tile_slot,
+    const MolTab &mt, int64_t b0, int64_t b1, int64_t s0, int gga,
+    const signed char *__restrict__ store, const signed char *__restrict__ zbase,
+    int64_t zstride, int first, double *__restrict__ vpart, signed char (&bufA)[4][SEC],
+    signed char (&bufB)[4][SEC], int (&ls)[4][512], int (&wcnt)[8]) {
   // wave-uniform values through readfirstlane, so that the branches on them
   // are scalar branches
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wa = wv >> 2, wh = (wv >> 1) & 1, wb = wv & 1;
+  // this wave's tile (wa, wb), its row groups from rg0 and column groups from j0
+  const int wa = NJ == 2 ? 0 : wv >> 2, wb = NG == 2 ? wv & 1 : 0;
+  const int rg0 = NG == 2 ? wv & 2 : wv & 3, j0 = NJ == 2 ? wv >> 2 << 1 : 0;
   const int l16 = lane & 15, q = lane >> 4;
   const int64_t sb_bytes = slot_bytes_i8(gga);
-  // J sections, two buffers (Z_J0 F_J0 Z_J1 F_J1 each), declared apart so
-  // that a copy into one is known not to touch the other
-  __shared__ __attribute__((aligned(16))) signed char bufA[4][SEC];
-  __shared__ __attribute__((aligned(16))) signed char bufB[4][SEC];
-  __shared__ int ls[4][512];  // slots of I_0, I_1, J_0, J_1 per listed batch
-  __shared__ int wcnt[8];
-  // this wave's tile and its pair index (-1: no work for this wave)
-  const int4 pix = sp_pidx[sp];
+  // the tile's pair index (-1: no pair of its own)
   const int pp = wa ? (wb ? pix.w : pix.z) : (wb ? pix.y : pix.x);
-  double v64[2][4][4];
+  const bool diag = blk.x == blk.z;
+  // whether the wave's tile is formed: its pair is kept, or (diagonal) it is the
+  // transpose of one that is
+  const bool tile = pp >= 0 || (diag && wa > wb && pix.y >= 0);
+  double v64[NG][NJ][4];
 #pragma unroll
-  for (int g = 0; g < 2; ++g)
+  for (int g = 0; g < NG; ++g)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) v64[g][j][r] = 0.0;
   // batches of the super-pair's molecule inside [b0, b1)
@@ -873,17 +875,18 @@ __global__ void __launch_bounds__(512) vgemm_i8(
   int64_t tso[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) tso[u] = bl[u] >= 0 ? (int64_t)mt.blk_local[bl[u]] * mnb : -1;
-  const int64_t lo = b0 > mb0 ? b0 : mb0, hi = b1 < mb0 + mnb ? b1 : mb0 + mnb;
+  const int64_t lo = b0 > mb0 ? b0 : mb0,
+                hi = split < nsplit ? (b1 < mb0 + mnb ? b1 : mb0 + mnb) : lo;
 
   // this wave's I fragments (two 16-row groups) and row exponents
-  v4i Fr[2][4], Zr[2][4];
-  int eF[2] = {0, 0}, eZ[2] = {0, 0};
+  v4i Fr[NG][4], Zr[NG][4];
+  int eF[NG] = {}, eZ[NG] = {};
   auto f_section = [&](int s) { return store + (s - s0) * sb_bytes + OFF_F; };
   auto z_section = [&](int s) { return zbase + (s - s0) * zstride; };
   auto load_I = [&](const signed char *sec, v4i (*dst)[4], int *ex) {
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const int rg = 2 * wh + g;
+    for (int g = 0; g < NG; ++g) {
+      const int rg = rg0 + g;
 #pragma unroll
       for (int pl = 0; pl < 4; ++pl) dst[g][pl] = ld16(sec + pl * PLANE + (rg * 64 + lane) * 16);
       ex[g] = *reinterpret_cast<const int *>(sec + 4 * PLANE + 16 * rg + 4 * q);
@@ -891,7 +894,7 @@ __global__ void __launch_bounds__(512) vgemm_i8(
   };
   // whether the wave's tile has work in listed batch i
   auto active = [&](int i) {
-    return pp >= 0 && __builtin_amdgcn_readfirstlane(ls[wa][i]) >= 0 &&
+    return tile && __builtin_amdgcn_readfirstlane(ls[wa][i]) >= 0 &&
            __builtin_amdgcn_readfirstlane(ls[2 + wb][i]) >= 0;
   };
   // F_I of batch i; where the wave's tile is idle in batch i (or past the
@@ -908,7 +911,7 @@ __global__ void __launch_bounds__(512) vgemm_i8(
       const int sJ = __builtin_amdgcn_readfirstlane(ls[2 + jb][i]);
       if (sJ < 0) continue;
       dma_section<8>(z_section(sJ), &dst[2 * jb][0], (wv + 4 * jb) & 7, lane);
-      dma_section<8>(f_section(sJ), &dst[2 * jb + 1][0], (wv + 4 * jb + 2) & 7, lane);
+      if (!diag) dma_section<8>(f_section(sJ), &dst[2 * jb + 1][0], (wv + 4 * jb + 2) & 7, lane);
     }
   };
   // the first batch of a window: J sections through VGPRs and LDS stores
@@ -924,6 +927,7 @@ __global__ void __launch_bounds__(512) vgemm_i8(
       const signed char *src[2] = {z_section(sJ), f_section(sJ)};
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
+        if (u && diag) continue;
         v4i t[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -946,21 +950,21 @@ __global__ void __launch_bounds__(512) vgemm_i8(
     const signed char *sec = &cur[2 * wb + p][0];
     // rows and columns stored as zero have zero slices: no zero test on the
     // scales
-    double sc[4];
+    double sc[NJ];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sc[j] = pow2((int)sec[4 * PLANE + 16 * j + l16] - 19);
+    for (int j = 0; j < NJ; ++j) sc[j] = pow2((int)sec[4 * PLANE + 16 * (j0 + j) + l16] - 19);
     v4i B[2][4];
 #pragma unroll
-    for (int pl = 0; pl < 4; ++pl) B[0][pl] = ld16(sec + pl * PLANE + lane * 16);
+    for (int pl = 0; pl < 4; ++pl) B[0][pl] = ld16(sec + pl * PLANE + (j0 * 64 + lane) * 16);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j < 3) {
+    for (int j = 0; j < NJ; ++j) {
+      if (j + 1 < NJ) {
 #pragma unroll
         for (int pl = 0; pl < 4; ++pl)
-          B[(j + 1) & 1][pl] = ld16(sec + pl * PLANE + ((j + 1) * 64 + lane) * 16);
+          B[(j + 1) & 1][pl] = ld16(sec + pl * PLANE + ((j0 + j + 1) * 64 + lane) * 16);
       }
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
+      for (int g = 0; g < NG; ++g) {
         int h[4], o[4];
         tile_product(p ? Zr[g] : Fr[g], B[j & 1], h, o);
         const int er = p ? eZ[g] : eF[g];
@@ -978,11 +982,11 @@ __global__ void __launch_bounds__(512) vgemm_i8(
     wait_vm0();
     __syncthreads();  // buffer cur complete, nxt free
     const bool act = active(i);
-    if (act) load_I(z_section(__builtin_amdgcn_readfirstlane(ls[wa][i])), Zr, eZ);
+    if (act && !diag) load_I(z_section(__builtin_amdgcn_readfirstlane(ls[wa][i])), Zr, eZ);
     if (i + 1 < n) issue_J(i + 1, nxt);
     if (act) phase(0, cur);
     next_F(i + 1, n);
-    if (act) phase(1, cur);
+    if (act && !diag) phase(1, cur);
   };
 
   for (int64_t c0 = lo + split; c0 < hi; c0 += 512 * (int64_t)nsplit) {
@@ -1017,17 +1021,83 @@ __global__ void __launch_bounds__(512) vgemm_i8(
       if (i + 1 < n) step(i + 1, n, bufB, bufA);
     }
   }
-  if (pp < 0) return;
+  if (diag) {
+    // V(a, b) = Vbar(a, b) + Vbar(b, a)^T for (0, 0), (0, 1), (1, 1), tile by
+    // tile through LDS
+    double(*t)[FB + 1] = reinterpret_cast<double(*)[FB + 1]>(&bufA[0][0]);
+    static_assert(sizeof(bufA) >= FB * (FB + 1) * sizeof(double), "a tile in a buffer");
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int ta = k == 2 ? 1 : 0, tb = k == 0 ? 0 : 1;  // target; source (tb, ta)
+      __syncthreads();
+      if (wa == tb && wb == ta) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                t[16 * (rg0 + g) + 4 * q + r][16 * (j0 + j) + l16] = v64[g][j][r];
+      }
+      __syncthreads();
+      if (wa == ta && wb == tb) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                v64[g][j][r] += t[16 * (j0 + j) + l16][16 * (rg0 + g) + 4 * q + r];
+      }
+    }
+  }
+  if (pp < 0 || split >= nsplit) return;
   double *out = vpart + ((int64_t)split * npairs + pp) * (FB * FB);
 #pragma unroll
-  for (int g = 0; g < 2; ++g)
+  for (int g = 0; g < NG; ++g)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NJ; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int mu = 32 * wh + 16 * g + 4 * q + r, nu = 16 * j + l16;
+        const int mu = 16 * (rg0 + g) + 4 * q + r, nu = 16 * (j0 + j) + l16;
         out[mu * FB + nu] = first ? v64[g][j][r] : out[mu * FB + nu] + v64[g][j][r];
       }
+    }
+}
+
+__global__ void __launch_bounds__(512) vgemm_i8(
+    int nsp, int nsplit, int grouped, const int4 *__restrict__ sp_blk,
+    const int4 *__restrict__ sp_pidx, int npairs, const int *__restrict__ tile_slot, MolTab mt,
+    int64_t b0, int64_t b1, int64_t s0, int gga, const signed char *__restrict__ store,
+    const signed char *__restrict__ zbase, int64_t zstride, int first,
+    double *__restrict__ vpart) {
+  // J sections, two buffers (Z_J0 F_J0 Z_J1 F_J1 each), declared apart so
+  // that a copy into one is known not to touch the other
+  __shared__ __attribute__((aligned(16))) signed char bufA[4][SEC];
+  __shared__ __attribute__((aligned(16))) signed char bufB[4][SEC];
+  __shared__ int ls[4][512];  // slots of I_0, I_1, J_0, J_1 per listed batch
+  __shared__ int wcnt[8];
+  // split-major: the super-pairs of one split run together and walk the same
+  // batches, sharing each batch's slots in the caches; grouped: those of a
+  // split on one XCD (workgroups are dealt to the eight XCDs in turn; splits
+  // past the last find no batch)
+  int sp = blockIdx.x % nsp, split = blockIdx.x / nsp;
+  if (grouped) {
+    const int rr = blockIdx.x >> 3;
+    sp = rr % nsp;
+    split = rr / nsp * 8 + (blockIdx.x & 7);
+  }
+  const int4 blk = sp_blk[sp], pix = sp_pidx[sp];
+#define NKX_VTILE(NG, NJ)                                                                       \
+  vgemm_i8_tile<NG, NJ>(blk, pix, split, nsplit, npairs, tile_slot, mt, b0, b1, s0, gga, store, \
+                        zbase, zstride, first, vpart, bufA, bufB, ls, wcnt)
+  if (blk.w >= 0)
+    NKX_VTILE(2, 4);
+  else if (blk.y >= 0)
+    NKX_VTILE(1, 4);
+  else
+    NKX_VTILE(1, 2);
+#undef NKX_VTILE
 }
 
 // ---------------------------------------------------------------------------
@@ -1166,8 +1236,12 @@ void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
   // Z sections: each slot's own, or (second spin) SEC-strided in zstore_b
   const signed char *zbase = zstore_b ? zstore_b : store + OFF_Z;
   const int64_t zstride = zstore_b ? (int64_t)SEC : slot_bytes_i8(gga);
-  hipLaunchKernelGGL(vgemm_i8, dim3((unsigned)(pl.nspairs * nsplit)), dim3(512), 0, s,
-                     pl.nspairs, nsplit, reinterpret_cast<const int4 *>(pl.sp_blk.p),
+  // all super-pairs of a split on one XCD where they fit its 32 CUs twice at
+  // most: 32 waters (28 super-pairs) 19.1 -> 17.8 ms; 100 waters (210) lose by it
+  const bool grouped = pl.nspairs <= 64;
+  const int64_t ns = grouped ? (nsplit + 7) / 8 * 8 : nsplit;
+  hipLaunchKernelGGL(vgemm_i8, dim3((unsigned)(pl.nspairs * ns)), dim3(512), 0, s, pl.nspairs,
+                     nsplit, grouped ? 1 : 0, reinterpret_cast<const int4 *>(pl.sp_blk.p),
                      reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.npairs, pl.tile_slot.p,
                      pl.tab(), b0, b1, s0, gga, store, zbase, zstride, first ? 1 : 0,
                      vpart);

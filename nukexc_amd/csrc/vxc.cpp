@@ -400,20 +400,28 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
   return (int64_t)(budget / slot_bytes);
 }
 
-// Split count of the V contraction over batches, or the tuned value.  FP64:
-// about 4096 workgroups of a super-pair tile (one per CU at a time, the rest
-// balancing the tail: with 2048 the CUs of 16 waters were busy 84 % of the
-// time; every split costs a tile of partials per pair), at least four batches
-// each (31 splits of 32 batches left water on 31 CUs: 245 us, now 26).  int8 and bf16: about 8192 workgroups of a super-pair tile
-// or a pair, at least 32 batches each (on small molecules one batch per
-// workgroup is mostly set-up there).
+// Split count of the V contraction over batches, or the tuned value.  One
+// workgroup of a super-pair tile (bf16: of a pair) fits a CU at a time, so:
+//   one unit:  256 splits, one equal workgroup per CU (mixed benzene, 99 x 578
+//              points: 1536 us per build, 1617 with 320, 1608 with 335)
+//   a few:     512 splits each (16- and 24-atom molecules: within 1 % of the
+//              best of 32 .. 1024)
+//   many:      about 8192 workgroups (FP64: 4096), the tail of unequal units
+//              levelled by their number; every split costs a tile of partials
+//              per pair
+// and never less than four batches per split (mixed water: 146 us with 4 to 5,
+// 179 with 32), or in a molecule set 16 (FP64: 8) of an average molecule (8
+// molecules, mixed: 2782 us, 2893 with 4).
 int choose_nsplit(const Plan &pl, int precision, int tuned = 0) {
   const bool f64 = precision == NKX_PREC_FP64;
   const int64_t units = precision == NKX_PREC_MIXED_BF16 ? pl.npairs : pl.nspairs;
   if (units == 0) return 1;
-  const int64_t target = f64 ? 4096 : 8192;
-  int64_t ns = tuned > 0 ? tuned : (target + units - 1) / units;
-  if (tuned <= 0) ns = std::min<int64_t>(ns, pl.nb / (f64 ? 4 : 32));
+  int64_t ns = tuned;
+  if (tuned <= 0) {
+    const int64_t per = pl.nmol > 1 ? (f64 ? 8 : 16) * (int64_t)pl.nmol : 4;
+    ns = std::min<int64_t>((f64 ? 4096 : 8192) / units + 1, units == 1 ? 256 : 512);
+    ns = std::min<int64_t>(ns, pl.nb / per);
+  }
   ns = std::max<int64_t>(1, std::min<int64_t>(ns, pl.nb));
   return (int)ns;
 }
