@@ -240,40 +240,103 @@ __global__ void __launch_bounds__(256) pair_table_kernel(int natoms, const doubl
                   : make_double2(1.0 / (capped ? 5.0 : R), capped ? 0.0 : 1.0 / (R * R));
 }
 
-// Becke cell function P_i at (x, y, z); same screening and clamping as the
-// partition kernel, with mu_ij = (r_i - r_j) / R~_ij taken as a product with
-// the tabulated 1/R~_ij (tab = row i of the pair table).
-__device__ double becke_cell(int i, int natoms, const double *C, const double2 *tab, double x,
-                             double y, double z, double ri, bool cap) {
-  double Pi = 1.0;
-  for (int j = 0; j < natoms; ++j) {
-    if (j == i) continue;
-    const double rj = gdist(x, y, z, C + 3 * j);
-    if (cap && ri - rj <= -5.0) continue;  // mu <= -1: factor 1
-    double mu = (ri - rj) * tab[j].x;
-    mu = mu > 1.0 ? 1.0 : (mu < -1.0 ? -1.0 : mu);
-    Pi *= 0.5 * (1.0 - bp(bp(bp(mu))));
-    if (Pi == 0.0) break;
-  }
-  return Pi;
+// One thread per sorted point, one wave per workgroup; per-atom sums in LDS
+// (3 natoms doubles).  The candidates (atoms whose cell function can be nonzero
+// at some point of the wave) are taken WC at a time in registers: one sweep over
+// j multiplies their cell functions P_i and adds them to Z = sum P_i, and once Z
+// is known a second one adds the derivative terms of all of them, so that r_j is
+// formed once per WC candidates and the force on atom j is summed over them
+// before it is summed over the wave.  The cell functions of the first WKEEP
+// groups stay in LDS in between; those of later ones (more than 16 atoms near a
+// wave) are formed again.  Loops over atoms run in step across the wave (lanes
+// without a contribution add zero); each per-atom term is summed over the wave
+// (wave_sum: every lane active) and added to LDS by lane 0.  With one writer per
+// workgroup (no atomics) the sums, and so the gradient, come out the same on
+// every run.  The points of a wave are 64 consecutive sorted points (npts_pad
+// and the grid stride are multiples of 64), so every lane runs the same trip
+// count.  ptab: the atom-pair table of pair_table_kernel.  |mu| >= 1 gives the
+// factor 1 or 0 exactly and no derivative.
+//
+// Bound by FP64 VALU issue.  A 30-atom molecule, 648 000 points: 2267 us with
+// one candidate at a time (a square root per pair in both sweeps, three wave
+// sums per pair), 1333 with four, 1091 with the cell functions kept and the
+// quotient by s_ij through recip; WC = 3 and 6 cost 6 % more (registers).
+constexpr int WC = 4;   // candidates in registers
+constexpr int WKEEP = 4;  // groups of WC whose cell functions are kept in LDS
+
+// 1 / a, 0 < a normal: the estimate and two Newton steps (within an ulp)
+__device__ __forceinline__ double recip(double a) {
+  double y = __builtin_amdgcn_rcp(a);
+  y = fma(fma(-a, y, 1.0), y, y);
+  return fma(fma(-a, y, 1.0), y, y);
 }
 
-// One thread per sorted point, one wave per workgroup; per-atom sums in LDS
-// (3 natoms doubles).  Every loop over atoms runs in step across the wave
-// (lanes without a contribution add zero), so each per-atom term is summed
-// over the wave (wave_sum: every lane active) and added to LDS by lane 0: all
-// lanes of a wave touch the same atoms, and one LDS atomic per lane would
-// serialise on them.  With one writer per workgroup (no atomics) the sums, and
-// so the gradient, come out the same on every run.  The points of a wave are
-// 64 consecutive sorted points (npts_pad and the grid stride are multiples of
-// 64), so every lane runs the same trip count.  ptab: the atom-pair table of
-// pair_table_kernel.
+struct WeightCands {
+  int idx[WC];     // wave-uniform atom, -1: none
+  bool act[WC];    // the cell function of this lane's point can be nonzero
+  double r[WC];    // this lane's distance
+};
+
+// The next WC candidates from atom `next` on (at least one lane within 5 bohr of
+// its nearest atom's distance, or any lane without the cap); false when none is
+// left.
+__device__ __forceinline__ bool next_cands(WeightCands &c, int &next, int natoms,
+                                           const double *__restrict__ C, double x, double y,
+                                           double z, double rmin, bool cap, bool on) {
+  int n = 0;
+#pragma unroll
+  for (int k = 0; k < WC; ++k) {
+    c.idx[k] = -1;
+    c.act[k] = false;
+    c.r[k] = 1.0;
+  }
+  for (; next < natoms && n < WC; ++next) {
+    const double r = gdist(x, y, z, C + 3 * next);
+    const bool a = on && !(cap && r - rmin >= 5.0);
+    if (!__ballot(a)) continue;
+#pragma unroll
+    for (int k = 0; k < WC; ++k)
+      if (k == n) {
+        c.idx[k] = next;
+        c.act[k] = a;
+        c.r[k] = r;
+      }
+    ++n;
+  }
+  return n > 0;
+}
+
+// Becke cell functions P of the candidates at this lane's point.
+__device__ __forceinline__ void cand_cells(const WeightCands &c, int natoms,
+                                           const double *__restrict__ C,
+                                           const double2 *__restrict__ tab, double x, double y,
+                                           double z, bool cap, double (&P)[WC]) {
+  double rmax = 0.0;
+#pragma unroll
+  for (int k = 0; k < WC; ++k) {
+    P[k] = c.act[k] ? 1.0 : 0.0;
+    if (c.act[k]) rmax = fmax(rmax, c.r[k]);
+  }
+  for (int j = 0; j < natoms; ++j) {
+    const double rj = gdist(x, y, z, C + 3 * j);
+    if (cap && !__ballot(rmax - rj > -5.0)) continue;  // every factor is 1
+#pragma unroll
+    for (int k = 0; k < WC; ++k) {
+      if (c.idx[k] < 0 || c.idx[k] == j) continue;  // uniform
+      const double mu =
+          fmin(fmax((c.r[k] - rj) * tab[c.idx[k] * natoms + j].x, -1.0), 1.0);
+      P[k] *= 0.5 * (1.0 - bp(bp(bp(mu))));
+    }
+  }
+}
+
 __global__ void __launch_bounds__(64) grad_weights_kernel(
     int64_t npts_pad, int natoms, const double *__restrict__ C, const double *__restrict__ px,
     const double *__restrict__ py, const double *__restrict__ pz, const int *__restrict__ pown,
     const double *__restrict__ epoint, const double *__restrict__ tpt, int partition,
     const double2 *__restrict__ ptab, double *__restrict__ wpart) {
   extern __shared__ double acc[];
+  __shared__ double Pk[WKEEP * WC * 64];
   for (int e = threadIdx.x; e < 3 * natoms; e += blockDim.x) acc[e] = 0.0;
   __syncthreads();
   const bool cap = partition == 1;
@@ -292,79 +355,98 @@ __global__ void __launch_bounds__(64) grad_weights_kernel(
       z = pz[sp];
     }
     const bool wact = act && partition != 0 && wf != 0.0;
-    if (wact) {
+    if (__ballot(wact)) {
       if (cap)
         for (int i = 0; i < natoms; ++i) rmin = fmin(rmin, gdist(x, y, z, C + 3 * i));
-      for (int i = 0; i < natoms; ++i) {
-        const double ri = gdist(x, y, z, C + 3 * i);
-        if (cap && ri - rmin >= 5.0) continue;
-        const double Pi = becke_cell(i, natoms, C, ptab + i * natoms, x, y, z, ri, cap);
-        Z += Pi;
-        if (i == B) PB = Pi;
+      WeightCands c;
+      int g = 0;
+      for (int next = 0; next_cands(c, next, natoms, C, x, y, z, rmin, cap, wact); ++g) {
+        double P[WC];
+        cand_cells(c, natoms, C, ptab, x, y, z, cap, P);
+#pragma unroll
+        for (int k = 0; k < WC; ++k) {
+          if (g < WKEEP) Pk[(g * WC + k) * 64 + lane] = P[k];
+          Z += P[k];
+          if (c.idx[k] == B) PB = P[k];
+        }
       }
     }
     const bool gact = wact && PB > 0.0 && Z > 0.0;
     if (__ballot(gact)) {
-      for (int i = 0; i < natoms; ++i) {
-        bool li = gact;
-        double ri = 1.0, Pi = 0.0;
-        if (li) {
-          ri = gdist(x, y, z, C + 3 * i);
-          li = !(cap && ri - rmin >= 5.0);
+      const double iPB = gact ? 1.0 / PB : 0.0, iZ = gact ? 1.0 / Z : 0.0;
+      WeightCands c;
+      int g = 0;
+      for (int next = 0; next_cands(c, next, natoms, C, x, y, z, rmin, cap, wact); ++g) {
+        double P[WC];
+        if (g < WKEEP) {
+#pragma unroll
+          for (int k = 0; k < WC; ++k) P[k] = Pk[(g * WC + k) * 64 + lane];
+        } else {
+          cand_cells(c, natoms, C, ptab, x, y, z, cap, P);
         }
-        if (li) {
-          Pi = becke_cell(i, natoms, C, ptab + i * natoms, x, y, z, ri, cap);
-          li = Pi != 0.0;
+        double coef[WC], ui[WC][3], gi[WC][3];
+#pragma unroll
+        for (int k = 0; k < WC; ++k) {
+          coef[k] = gact && P[k] != 0.0 ? wf * ((c.idx[k] == B ? iPB : 0.0) - iZ) * P[k] : 0.0;
+          const double *Ci = C + 3 * max(c.idx[k], 0);
+          const double iri = c.r[k] > 0.0 ? 1.0 / c.r[k] : 0.0;  // 0: on the nucleus
+          ui[k][0] = (x - Ci[0]) * iri;
+          ui[k][1] = (y - Ci[1]) * iri;
+          ui[k][2] = (z - Ci[2]) * iri;
+          gi[k][0] = gi[k][1] = gi[k][2] = 0.0;
         }
-        if (!__ballot(li)) continue;
-        const double coefi = li ? wf * ((i == B ? 1.0 / PB : 0.0) - 1.0 / Z) * Pi : 0.0;
-        const double *Ci = C + 3 * i;
-        const double2 *ti = ptab + i * natoms;
-        const double iri = 1.0 / ri;
-        const double ui[3] = {(x - Ci[0]) * iri, (y - Ci[1]) * iri, (z - Ci[2]) * iri};
-        double gi[3] = {0.0, 0.0, 0.0};
         for (int j = 0; j < natoms; ++j) {
-          if (j == i) continue;
           const double *Cj = C + 3 * j;
-          double gj[3] = {0.0, 0.0, 0.0};
-          bool lj = li;
-          double rj = 1.0;
-          if (lj) {
-            rj = gdist(x, y, z, Cj);
-            lj = !(cap && ri - rj <= -5.0);
+          const double dj[3] = {x - Cj[0], y - Cj[1], z - Cj[2]};
+          const double rj = gdist(x, y, z, Cj);
+          double mu[WC];
+          bool in[WC], any = false;
+#pragma unroll
+          for (int k = 0; k < WC; ++k) {
+            mu[k] = c.idx[k] >= 0 ? (c.r[k] - rj) * ptab[c.idx[k] * natoms + j].x : 1.0;
+            in[k] = c.idx[k] != j && coef[k] != 0.0 && mu[k] > -1.0 && mu[k] < 1.0;
+            any = any || in[k];
           }
-          if (lj) {
-            const double d[3] = {Ci[0] - Cj[0], Ci[1] - Cj[1], Ci[2] - Cj[2]};
-            const double2 tij = ti[j];  // 1/R~, [not capped] / R^2
-            const double mu = (ri - rj) * tij.x;
-            if (mu > -1.0 && mu < 1.0) {  // clamped: s' = 0
-              const double p1 = bp(mu), p2 = bp(p1), p3 = bp(p2);
-              const double sv = 0.5 * (1.0 - p3);
-              const double ds = -0.5 * bdp(p2) * bdp(p1) * bdp(mu);
-              const double f = coefi * ds / sv;  // s > 0 because P_i > 0
-              const double ct = mu * tij.y;
-              const double irj = 1.0 / rj;
-              const double uj[3] = {(x - Cj[0]) * irj, (y - Cj[1]) * irj, (z - Cj[2]) * irj};
-              for (int k = 0; k < 3; ++k) {
-                gi[k] += f * (-ui[k] * tij.x - ct * d[k]);
-                if (j != B) gj[k] = f * (uj[k] * tij.x + ct * d[k]);
-              }
-            } else {
-              lj = false;
+          if (!__ballot(any)) continue;
+          const double irj = rj > 0.0 ? 1.0 / rj : 0.0;
+          double a = 0.0, gj[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+          for (int k = 0; k < WC; ++k) {
+            if (c.idx[k] < 0 || c.idx[k] == j || !__ballot(in[k])) continue;  // uniform
+            const double *Ci = C + 3 * c.idx[k];
+            const double2 tij = ptab[c.idx[k] * natoms + j];  // 1/R~, [not capped] / R^2
+            const double m = mu[k], p1 = bp(m), p2 = bp(p1), p3 = bp(p2);
+            const double sv = 0.5 * (1.0 - p3);  // > 0 because P_i > 0
+            const double ds = -0.5 * bdp(p2) * bdp(p1) * bdp(m);
+            const double f = in[k] ? coef[k] * ds * recip(sv) : 0.0;
+            const double fr = f * tij.x, ft = in[k] ? f * m * tij.y : 0.0;
+            a += fr;
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+              const double e = ft * (Ci[t] - Cj[t]);
+              gi[k][t] -= fr * ui[k][t] + e;
+              gj[t] += e;
             }
           }
-          if (!__ballot(lj && j != B)) continue;
-          for (int k = 0; k < 3; ++k) {
-            S[k] += gj[k];
-            const double v = wave_sum(gj[k]);
-            if (lane == 0) acc[3 * j + k] += v;
+          const bool mine = j == B;
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            const double g = mine ? 0.0 : gj[t] + a * (dj[t] * irj);
+            S[t] += g;
+            const double v = wave_sum(g);
+            if (lane == 0) acc[3 * j + t] += v;
           }
         }
-        for (int k = 0; k < 3; ++k) {
-          const double gv = (li && i != B) ? gi[k] : 0.0;
-          S[k] += gv;
-          const double v = wave_sum(gv);
-          if (lane == 0) acc[3 * i + k] += v;
+#pragma unroll
+        for (int k = 0; k < WC; ++k) {
+          if (c.idx[k] < 0) continue;  // uniform
+#pragma unroll
+          for (int t = 0; t < 3; ++t) {
+            const double g = c.idx[k] != B ? gi[k][t] : 0.0;
+            S[t] += g;
+            const double v = wave_sum(g);
+            if (lane == 0) acc[3 * c.idx[k] + t] += v;
+          }
         }
       }
     }
