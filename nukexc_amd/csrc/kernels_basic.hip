@@ -301,18 +301,17 @@ int64_t compact_points(hipStream_t s, int64_t n, double thr, const double *pin,
 // ---------------------------------------------------------------------------
 // Collocation in the reference layout: LayoutLeft (N_bf, N_pts), element
 // (mu, g) at mu + g * N_bf (stobasis.hpp:494-584).  One workgroup per 64
-// points, 32 functions at a time: a wave takes eight consecutive functions, a
-// point per lane (sto_run.hpp), into LDS tiles of 64 points x 32 functions
-// whose rows go out as runs of 32 doubles.
+// points, 4 FW functions at a time: a wave takes FW consecutive functions, a
+// point per lane (sto_run.hpp), into LDS tiles of 64 points x 4 FW functions
+// whose rows go out as runs of 4 FW doubles.
 //
 // Bound by its writes with the gradient (3.4 TB/s), by those and FP64 VALU issue
-// without.  One thread per element, functions fastest, loads a function record
-// per element and evaluates every exponential, root and quotient again: 375 us
-// per call on benzene (120 functions, 342 144 points); now 110 us for the values
-// and 292 us for the three gradients.
-constexpr int CR_F = 32, CR_LD = CR_F + 1;
-
-template <bool VAL, bool GRAD>
+// without; by the chain of one wave's functions on small grids.  One thread per
+// element, functions fastest, loads a function record per element and evaluates
+// every exponential, root and quotient again: 375 us per call on benzene (120
+// functions, 342 144 points); now 110 us for the values and 292 us for the three
+// gradients.
+template <bool VAL, bool GRAD, int FW>
 __global__ void __launch_bounds__(256) colloc_ref_kernel(int nbf, const FuncRec *__restrict__ F,
                                                          const HarmTerm *__restrict__ T,
                                                          int64_t npts,
@@ -320,6 +319,7 @@ __global__ void __launch_bounds__(256) colloc_ref_kernel(int nbf, const FuncRec 
                                                          double *phi, double *gx, double *gy,
                                                          double *gz) {
   constexpr int NARR = (VAL ? 1 : 0) + (GRAD ? 3 : 0), G0 = VAL ? 1 : 0;
+  constexpr int CR_F = 4 * FW, CR_LD = CR_F + 1;
   __shared__ double t[NARR][64][CR_LD];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t g0 = (int64_t)blockIdx.x * 64;
@@ -327,18 +327,20 @@ __global__ void __launch_bounds__(256) colloc_ref_kernel(int nbf, const FuncRec 
   const double x = pts[3 * g], y = pts[3 * g + 1], z = pts[3 * g + 2];
   double *const out[4] = {VAL ? phi : gx, VAL ? gx : gy, VAL ? gy : gz, gz};
   const int c = threadIdx.x & (CR_F - 1);
-  for (int m0 = 0; m0 < nbf; m0 += CR_F) {
-    const int f0 = m0 + 8 * wv, n = min(8, nbf - f0);
+  for (int m0 = blockIdx.y * CR_F; m0 < nbf; m0 += gridDim.y * CR_F) {
+    // the functions of a short last tile are dealt to all four waves
+    const int q = (min(CR_F, nbf - m0) + 3) >> 2, i0 = q * wv;
+    const int f0 = m0 + i0, n = min(q, nbf - f0);
     StoRun run;
 #pragma unroll 1
     for (int i = 0; i < n; ++i) {
       const FuncRec *fr = F + f0 + i;
       double v, gr[3];
       run.eval<GRAD, false>(fr[0], fr[i ? -1 : 0], i == 0, T, x, y, z, v, gr);
-      if (VAL) t[0][lane][8 * wv + i] = v;
+      if (VAL) t[0][lane][i0 + i] = v;
       if (GRAD) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) t[(G0 + k) % NARR][lane][8 * wv + i] = gr[k];
+        for (int k = 0; k < 3; ++k) t[(G0 + k) % NARR][lane][i0 + i] = gr[k];
       }
     }
     __syncthreads();
@@ -357,12 +359,31 @@ void launch_collocation_ref(hipStream_t s, int nbf, const FuncRec *f, const Harm
   if (nbf <= 0 || npts <= 0) return;
   const int64_t nwg = (npts + 63) / 64;
   NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "too many points");
-#define NKX_COLLOC(V, G)                                                                     \
-  hipLaunchKernelGGL((colloc_ref_kernel<V, G>), dim3((unsigned)nwg), dim3(256), 0, s, nbf, f, \
-                     t, npts, pts, phi, gx, gy, gz)
-  if (gx && phi) NKX_COLLOC(true, true);
-  else if (gx) NKX_COLLOC(false, true);
-  else NKX_COLLOC(true, false);
+  // Small outputs: narrow tiles (FW 4, 2 below one workgroup per CU), each a
+  // workgroup of its own, for shorter chains and more waves in flight; the lines
+  // that two tiles share meet in the last-level cache (256 MB, shared with what
+  // else is held).  Larger ones: those lines would go to memory twice, so one
+  // workgroup writes all tiles of its points, 32 functions wide.  Both calls
+  // (FW 8 in a loop / FW 4 each its own): 9 MB of output 72.3 / 69.6 us, 71 MB
+  // 96 / 83, 0.5 GB 269 / 308, 2.2 GB 799 / 1246; FW 2 at 4 MB 64.5 for 67.2.
+  const int64_t bytes = (int64_t)8 * nbf * npts * ((phi ? 1 : 0) + (gx ? 3 : 0));
+  const int fw = bytes > ((int64_t)1 << 26) ? 8 : nwg < 256 ? 2 : 4;
+  const unsigned ny = fw == 8 ? 1 : (unsigned)((nbf + 4 * fw - 1) / (4 * fw));
+#define NKX_COLLOC_FW(V, G, W)                                                              \
+  hipLaunchKernelGGL((colloc_ref_kernel<V, G, W>), dim3((unsigned)nwg, ny), dim3(256), 0, s, \
+                     nbf, f, t, npts, pts, phi, gx, gy, gz)
+#define NKX_COLLOC(V, G)                 \
+  if (fw == 8) NKX_COLLOC_FW(V, G, 8);   \
+  else if (fw == 4) NKX_COLLOC_FW(V, G, 4); \
+  else NKX_COLLOC_FW(V, G, 2)
+  if (gx && phi) {
+    NKX_COLLOC(true, true);
+  } else if (gx) {
+    NKX_COLLOC(false, true);
+  } else {
+    NKX_COLLOC(true, false);
+  }
+#undef NKX_COLLOC_FW
 #undef NKX_COLLOC
   NKX_HIP_CHECK(hipGetLastError());
 }

@@ -49,6 +49,13 @@ def test_collocation(nbf, npts):
         c.close()
 
 
+@pytest.mark.parametrize("nbf,npts", [(1, 16321), (15, 16385), (16, 16384), (17, 16447),
+                                      (33, 130001), (70, 130001)])
+def test_collocation_tile_widths(nbf, npts):
+    """Tiles of 16 functions (from 256 blocks of points) and 32 (above 64 MB)."""
+    test_collocation(nbf, npts)
+
+
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-7), ("mixed", 5e-7)])
 def test_gradient_with_f_functions(precision, tol):
     rng = np.random.default_rng(8)
