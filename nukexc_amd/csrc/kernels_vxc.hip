@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
     int64_t s0, const int *__restrict__ slot_b, const int *__restrict__ b_fbl,
     const FuncRec *__restrict__ F, const HarmTerm *__restrict__ T,
     const double *__restrict__ px, const double *__restrict__ py,
-    const double *__restrict__ pz, int narr, int gga, double *__restrict__ tiles) {
+    const double *__restrict__ pz, int narr, double *__restrict__ tiles) {
   const int64_t s = s0 + blockIdx.x;
   const int b = slot_b[s];
   const int f0 = 16 * __builtin_amdgcn_readfirstlane(threadIdx.x / PT);
@@ -58,13 +58,7 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
 #pragma unroll 1
   for (int i = 0; i < 16; ++i) {
     double v, gr[3];
-    if (gga) {
-      run.eval<true, false>(fr[i], fr[i ? i - 1 : 0], i == 0, T, x, y, z, v, gr);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) base[(c + 1) * TILE + i * PT] = gr[c];
-    } else {
-      run.eval<false, false>(fr[i], fr[i ? i - 1 : 0], i == 0, T, x, y, z, v, gr);
-    }
+    run.eval<false, false>(fr[i], fr[i ? i - 1 : 0], i == 0, T, x, y, z, v, gr);
     base[i * PT] = v;
   }
 }
@@ -462,12 +456,12 @@ void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, bool tra
   NKX_HIP_CHECK(hipGetLastError());
 }
 
-void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int gga,
+void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr,
                double *tiles) {
   if (s1 <= s0) return;
   hipLaunchKernelGGL(colloc_tiles_f64, dim3((unsigned)(s1 - s0)), dim3(256), 0, s, s0,
                      pl.slot_b.p, pl.b_fbl.p, pl.funcs.p, pl.terms.p, pl.px.p, pl.py.p, pl.pz.p,
-                     narr, gga, tiles);
+                     narr, tiles);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

@@ -467,7 +467,7 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   b.group = tuned_group > 0 ? tuned_group : (precision == NKX_PREC_MIXED ? 65 : 2);
   b.gga = gga;
   const int nmol = pl.nmol;
-  b.narr = (gga ? 4 : 1) + nspin;
+  b.narr = 1 + nspin;  // Phi, Z per spin
   b.nsplit = choose_nsplit(pl, precision, tuned_split);
   b.bf16 = precision == NKX_PREC_MIXED_BF16;
   b.mixed = precision == NKX_PREC_MIXED || b.bf16;
@@ -565,7 +565,7 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
       vkm_colloc(s, s0, s1, pl, ig, ws.mstore.p);
       vkm_pm_group(s, b0, b1, s0, pl, ig, ws.mstore.p);
     } else
-      vk_colloc(s, s0, s1, pl, narr, ig, ws.tiles64.p);
+      vk_colloc(s, s0, s1, pl, narr, ws.tiles64.p);
     tm.end(tt, s);
     tt = tm.begin(kStageDensity, s);
     if (bf16)
@@ -881,7 +881,7 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
                 "basis function " + std::to_string(i) + " is not centred on an atom of the grid");
   }
   NKX_REQUIRE(pl.nmol == 1, NKX_ERR_STATE, "the gradient runs on the ctx grid and basis");
-  const int narr = 4 + nspin;  // Phi, grad Phi (3), Z per spin
+  const int narr = 1 + nspin;  // Phi, Z per spin
   // FP64: the tile arrays; mixed: the int8 slot (sections and FP32 grad Phi),
   // the second spin's Y sections and the density partials; both plus the
   // per-slot gradient partials
@@ -967,7 +967,7 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
         vkg_fold(s, b0, b1, s0, pl, nseg, cpart, gacc);
       }
     } else {
-      vk_colloc(s, s0, s1, pl, narr, ig, ws.tiles64.p);
+      vk_colloc(s, s0, s1, pl, narr, ws.tiles64.p);
       vk_density(s, nspin, 2, b0, b1, s0, pl, ws.Pd.p, narr, ig, ws.tiles64.p, ws.dpart.p,
                  (int64_t)dsz);
       fp64_functional(s, nspin, b0, b1, s0, pl, ig, xl, ws, slots_alloc, epoint);
@@ -1009,7 +1009,7 @@ void density_points(Ctx &c, const double *P, double *rho, double *gx, double *gy
   NKX_REQUIRE(pl.nmol == 1, NKX_ERR_STATE, "the per-point density runs on the ctx grid and basis");
   Workspace &ws = c.ws;
   hipStream_t s = c.stream;
-  const int narr = 5;
+  const int narr = 1;  // Phi
   int64_t max_slots =
       chunk_slot_budget(((size_t)narr * FB * PT + 4 * PT) * sizeof(double), c.opt.mem_budget);
   for (int64_t b = 0; b < pl.nb; ++b)
@@ -1025,7 +1025,7 @@ void density_points(Ctx &c, const double *P, double *rho, double *gx, double *gy
   none.n = 0;
   vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, true, P, ws.Pd.p);
   for_each_chunk(pl, slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
-    vk_colloc(s, s0, s1, pl, narr, 1, ws.tiles64.p);
+    vk_colloc(s, s0, s1, pl, narr, ws.tiles64.p);
     vk_density(s, 1, 2, b0, b1, s0, pl, ws.Pd.p, narr, 1, ws.tiles64.p, ws.dpart.p, 0);
     vkm_density_functional(s, b0, b1, s0, pl, 1, none, ws.coef.p, ws.blockEN.p, ws.dpart.p,
                            nullptr, ws.gbuf.p);
@@ -1089,7 +1089,7 @@ void overlap_build(Ctx &c, double *S) {
   vk_fill0(s, S, (int64_t)pl.nbf * pl.nbf);
   double *const *Stab = upload_ptrs(c, std::vector<double *>{S});
   for_each_chunk(pl, slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
-    vk_colloc(s, s0, s1, pl, narr, 0, ws.tiles64.p);
+    vk_colloc(s, s0, s1, pl, narr, ws.tiles64.p);
     vk_zoverlap(s, s0, s1, pl, narr, ws.tiles64.p);
     vk_vgemm(s, b0, b1, s0, pl, nsplit, narr, 1, b0 == 0, ws.tiles64.p, ws.vpart.p);
   });

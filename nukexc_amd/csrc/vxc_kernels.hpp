@@ -22,7 +22,8 @@ void vk_plan_fill(hipStream_t s, int64_t nb, int nfb, int blk0, int64_t b0,
 // Pd = P permuted and zero-padded, or its transpose
 void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, bool transpose,
                  const double *P, double *Pd);
-void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int gga,
+// Phi per live slot, array 0 of narr
+void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr,
                double *tiles);
 // FP64 density contraction (kernels_density.hip): column sums of Phi X and grad
 // Phi X, X = P Phi, per live slot (4 x 64 doubles), spin s at part + s pstride.

@@ -78,3 +78,37 @@ def test_density_of_an_asymmetric_matrix(case):
     ref = [(phi[0] * X).sum(0)] + [2 * (d * X).sum(0) for d in phi[1:4]]
     for a, b in zip(out[:4], ref):
         assert np.abs(a.cpu().numpy() - b).max() <= 1e-10 * max(1.0, np.abs(b).max())
+
+
+@pytest.mark.parametrize("nbf", [1, 5, 64, 65, 130])
+def test_gradients_formed_in_the_kernels(nbf):
+    """grad Phi of the column sums and of Z is evaluated where it is used:
+    shells up to l = 5 in an order that breaks every run, both spins."""
+    rng = np.random.default_rng(nbf)
+    ctr = rng.normal(size=(4, 3)) * 2.0
+    f = []
+    for i in range(nbf):
+        l = int(rng.integers(0, 6 if i % 2 else 3))
+        f.append((l + 1 + int(rng.integers(0, 2)), l, int(rng.integers(-l, l + 1)),
+                  float(rng.choice([0.8, 1.3, 2.1])), *ctr[rng.integers(0, 4)]))
+    basis = nk.make_manual_basis(f)
+    n = 777
+    pts = ctr[rng.integers(0, 4, n)] + rng.normal(size=(n, 3)) * 1.5
+    w = rng.uniform(0.01, 0.1, n)
+    Ca, Cb = (rng.normal(size=(nbf, 3)) / nbf ** 0.5 for _ in range(2))
+    Pa, Pb = Ca @ Ca.T, Cb @ Cb.T
+    p, gx, gy, gz = O.collocation(basis_dict(basis), pts, grad=True)
+    ref = O.vxc_polarized(p, w, (101, 130), Pa, Pb, gx=gx, gy=gy, gz=gz)
+    c = nk.Context(0)
+    try:
+        c.set_basis(basis)
+        c.set_grid(nk.FlatGrid(torch.tensor(pts, device="cuda"), torch.tensor(w, device="cuda"),
+                               torch.tensor(ctr, device="cuda"), np.ones(4, np.int32),
+                               torch.zeros(n, dtype=torch.int32, device="cuda")))
+        dev = lambda a: torch.tensor(a, device="cuda")
+        u = c.vxc_polarized(dev(Pa), dev(Pb), funcs=(101, 130), precision="fp64")
+    finally:
+        c.close()
+    assert abs(u.energy - ref[0]) <= 1e-11 * abs(ref[0])
+    for V, R in zip((u.potential_alpha, u.potential_beta), ref[-2:]):
+        assert np.abs(V.cpu().numpy() - R).max() <= 1e-10 * max(1.0, np.abs(R).max())
