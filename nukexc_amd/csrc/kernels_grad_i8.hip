@@ -62,41 +62,16 @@ __global__ void __launch_bounds__(256) y_slots_i8(int64_t s0, const int *__restr
 #pragma unroll
       for (int e = 0; e < 16; ++e) gv[c][e] = 0.0f;
   }
-  const signed char *c0 = reinterpret_cast<const signed char *>(&fp[0]);
-  const signed char *c1 = reinterpret_cast<const signed char *>(&fp[1]);
-  const signed char *c2 = reinterpret_cast<const signed char *>(&fp[2]);
-  const signed char *c3 = reinterpret_cast<const signed char *>(&fp[3]);
-  // 2^(eP - 6) scales the slices exactly; 0 for a point stored as zero
-  const double sP = pow2_or_zero(eP == -127 ? -127 : eP - 6);
+  const double sP = unslice_scale(eP);
   double y[16];
-  double m = 0.0;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
-    const double v = (double)c0[e] + ldexp((double)c1[e], -7) + ldexp((double)c2[e], -14) +
-                     ldexp((double)c3[e], -21);
-    const double ph = v * sP;
-    const double yy = gga ? z_value(ph, (double)gv[0][e], (double)gv[1][e], (double)gv[2][e],
-                                    a2, bx, by, bz)
-                          : a2 * ph;
-    y[e] = yy;
-    m = fmax(m, fabs(yy));
+    const double ph = (double)unslice_int(fp, e) * sP;
+    y[e] = gga ? z_value(ph, (double)gv[0][e], (double)gv[1][e], (double)gv[2][e], a2, bx, by, bz)
+               : a2 * ph;
   }
-  m = fmax(m, __shfl_xor(m, 16));
-  m = fmax(m, __shfl_xor(m, 32));
-  const int ey = row_exp(m);
-  __attribute__((aligned(16))) signed char out[4][16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    signed char sc[4];
-    slice4(y[e], ey, sc);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) out[p][e] = sc[p];
-  }
-  signed char *ys = yout + (int64_t)blockIdx.x * ystride;
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-    *reinterpret_cast<v4i *>(ys + p * PLANE + t * 16) = *reinterpret_cast<const v4i *>(out[p]);
-  if (l < 16) ys[4 * PLANE + g] = (signed char)ey;
+  const int ey = item_row_exp(y);
+  store_item(y, ey, yout + (int64_t)blockIdx.x * ystride);
 }
 
 // One workgroup (four waves) per batch.  For each live block I of the batch,

@@ -16,8 +16,12 @@ namespace nkx {
 int64_t mixed_slot_bytes(int gga) { return slot_bytes_i8(gga); }
 
 // ---------------------------------------------------------------------------
-// Collocation: one workgroup per live slot; FP64 values in LDS, row maxima
-// along functions (F) and along points (Pm), slices in both orders.  Thread
+// Collocation: one workgroup per live slot; FP64 values in LDS, from where each
+// thread takes the 16 elements it slices in either order (F rows functions, Pm
+// rows points), the row exponents by shuffles between the four threads of a row.
+// Bound by FP64 VALU issue (60 %) and the 80 KB it writes per slot (3.8 TB/s):
+// benzene, 686 000 points, 505 -> 455 us with slice16 and one pass over the tile
+// per order (a pass for the maxima before it cost bank conflicts).  Thread
 // t evaluates the 16 consecutive functions 16 (t / 64) .. +15 of the block
 // at point t % 64 (one function at a time for the whole wave, a point per
 // lane).  Functions are sorted by centre, so consecutive functions that
@@ -32,7 +36,6 @@ __global__ void __launch_bounds__(256) colloc_tiles_i8(
   const int b = slot_b[s];
   const int fb = b_fbl[s];
   __shared__ double v[FB][65];
-  __shared__ int eF[FB], eP[PT];
   const int g = threadIdx.x & (PT - 1);
   // the wave's functions are wave-uniform: their records are scalar loads and
   // the branches on them scalar branches
@@ -57,28 +60,13 @@ __global__ void __launch_bounds__(256) colloc_tiles_i8(
     v[f][g] = val;
   }
   __syncthreads();
-  {
-    // row maxima along functions (F) and along points (Pm): four threads per
-    // row, 16 elements each, then the four partial maxima by shuffles
-    const int rr = threadIdx.x >> 2, qt = threadIdx.x & 3;
-    double m = 0.0, mp = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      m = fmax(m, fabs(v[rr][16 * qt + k]));
-      mp = fmax(mp, fabs(v[16 * qt + k][rr]));
-    }
-    m = fmax(m, __shfl_xor(m, 1));
-    m = fmax(m, __shfl_xor(m, 2));
-    mp = fmax(mp, __shfl_xor(mp, 1));
-    mp = fmax(mp, __shfl_xor(mp, 2));
-    if (qt == 0) {
-      eF[rr] = row_exp(m);
-      eP[rr] = row_exp(mp);
-    }
-  }
-  __syncthreads();
-  store_section<false>(v, eF, base + OFF_F);
-  store_section<true>(v, eP, base + OFF_PM);
+  double e[16];
+  tile_item<false>(v, e);
+  const int eF = item_row_exp(e);
+  store_item(e, eF, base + OFF_F);
+  tile_item<true>(v, e);
+  const int eP = item_row_exp(e);
+  store_item(e, eP, base + OFF_PM);
 }
 
 // P (FP64, original order) -> one section per 64 x 64 block pair (fm, fk),
@@ -118,7 +106,10 @@ __global__ void __launch_bounds__(256) gather_p_i8(int nbf, int nfb,
     ex[threadIdx.x] = row_exp(m);
   }
   __syncthreads();
-  store_section<false>(v, ex, Ps + (int64_t)blockIdx.x * SEC);
+  double it[16];
+  tile_item<false>(v, it);
+  max_hi(it);
+  store_item(it, ex[16 * (threadIdx.x >> 6) + (threadIdx.x & 15)], Ps + (int64_t)blockIdx.x * SEC);
 }
 
 
@@ -153,32 +144,23 @@ __global__ void __launch_bounds__(256) pm_group_i8(int64_t s0, int64_t b0,
       v4i w[4];
 #pragma unroll
       for (int pl = 0; pl < 4; ++pl) w[pl] = ld16(sec + pl * PLANE + off);
-      const signed char *c0 = reinterpret_cast<const signed char *>(&w[0]);
-      const signed char *c1 = reinterpret_cast<const signed char *>(&w[1]);
-      const signed char *c2 = reinterpret_cast<const signed char *>(&w[2]);
-      const signed char *c3 = reinterpret_cast<const signed char *>(&w[3]);
-      __attribute__((aligned(16))) signed char out[4][16];
+      unsigned U[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        int V = (int)c0[e] * (1 << 21) + (int)c1[e] * (1 << 14) + (int)c2[e] * (1 << 7) +
-                (int)c3[e];
+        int V = unslice_int(w, e);
         if (sh > 28) {
           V = 0;
         } else {
           const int qv = V >> sh, rv = V - qv * (1 << sh), half = 1 << (sh - 1);
           V = qv + ((rv > half || (rv == half && (qv & 1))) ? 1 : 0);
         }
-#pragma unroll
-        for (int pl = 3; pl > 0; --pl) {
-          const int d = ((V + 64) & 127) - 64;
-          out[pl][e] = (signed char)d;
-          V = (V - d) >> 7;
-        }
-        out[0][e] = (signed char)V;
+        U[e] = (unsigned)(V + kDigitBias);
       }
+      v4i out[4];
+      pack16(U, out);
 #pragma unroll
       for (int pl = 0; pl < 4; ++pl)
-        *reinterpret_cast<v4i *>(sec + pl * PLANE + off) = *reinterpret_cast<const v4i *>(out[pl]);
+        *reinterpret_cast<v4i *>(sec + pl * PLANE + off) = out[pl];
     }
     __syncthreads();  // every thread has read the old exponents of the group
     if (ch == 0)
@@ -589,19 +571,12 @@ __global__ void __launch_bounds__(256) density_x2_i8(
 #pragma unroll
             for (int e = 0; e < 16; ++e) gv[c][e] = 0.0f;
         }
-        const signed char *c0 = reinterpret_cast<const signed char *>(&pw4[0]);
-        const signed char *c1 = reinterpret_cast<const signed char *>(&pw4[1]);
-        const signed char *c2 = reinterpret_cast<const signed char *>(&pw4[2]);
-        const signed char *c3 = reinterpret_cast<const signed char *>(&pw4[3]);
-        // 2^(eP - 6) scales the slices exactly; 0 for a point stored as zero
-        const double sP = pow2_or_zero(eP == -127 ? -127 : eP - 6);
+        const double sP = unslice_scale(eP);
         double sm[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const double x = Xs(16 * qq + e)[g];
-          const double v = (double)c0[e] + ldexp((double)c1[e], -7) +
-                           ldexp((double)c2[e], -14) + ldexp((double)c3[e], -21);
-          sm[0] += (v * sP) * x;
+          sm[0] += ((double)unslice_int(pw4, e) * sP) * x;
           sm[1] += (double)gv[0][e] * x;
           sm[2] += (double)gv[1][e] * x;
           sm[3] += (double)gv[2][e] * x;
@@ -768,14 +743,8 @@ __global__ void __launch_bounds__(256) z_slots_i8(int64_t s0, const int *__restr
       for (int q4 = 0; q4 < 4; ++q4) gq[c][q4] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
   __syncthreads();
-  const signed char *c0 = reinterpret_cast<const signed char *>(&fp[0]);
-  const signed char *c1 = reinterpret_cast<const signed char *>(&fp[1]);
-  const signed char *c2 = reinterpret_cast<const signed char *>(&fp[2]);
-  const signed char *c3 = reinterpret_cast<const signed char *>(&fp[3]);
-  // 2^(eF - 6) scales the slices exactly; 0 for a row stored as zero
-  const double sF = pow2_or_zero(eF == -127 ? -127 : eF - 6);
+  const double sF = unslice_scale(eF);
   double z[16];
-  double m = 0.0;
 #pragma unroll
   for (int q4 = 0; q4 < 4; ++q4) {
     const float gxa[4] = {gq[0][q4].x, gq[0][q4].y, gq[0][q4].z, gq[0][q4].w},
@@ -784,32 +753,15 @@ __global__ void __launch_bounds__(256) z_slots_i8(int64_t s0, const int *__restr
 #pragma unroll
     for (int e4 = 0; e4 < 4; ++e4) {
       const int e = 4 * q4 + e4, g = k0 + e;
-      const double v = (double)c0[e] + ldexp((double)c1[e], -7) + ldexp((double)c2[e], -14) +
-                       ldexp((double)c3[e], -21);
-      const double ph = v * sF;
+      const double ph = (double)unslice_int(fp, e) * sF;
       const double zz = gga ? z_value(ph, (double)gxa[e4], (double)gya[e4], (double)gza[e4],
                                       cf[g][0], cf[g][1], cf[g][2], cf[g][3])
                             : cf[g][0] * ph;
       z[e] = zz;
-      m = fmax(m, fabs(zz));
     }
   }
-  m = fmax(m, __shfl_xor(m, 16));
-  m = fmax(m, __shfl_xor(m, 32));
-  const int ez = row_exp(m);
-  __attribute__((aligned(16))) signed char out[4][16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    signed char sc[4];
-    slice4(z[e], ez, sc);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) out[p][e] = sc[p];
-  }
-  signed char *zs = zout + (int64_t)blockIdx.x * zstride;
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-    *reinterpret_cast<v4i *>(zs + p * PLANE + t * 16) = *reinterpret_cast<const v4i *>(out[p]);
-  if (l < 16) zs[4 * PLANE + row] = (signed char)ez;
+  const int ez = item_row_exp(z);
+  store_item(z, ez, zout + (int64_t)blockIdx.x * zstride);
 }
 
 // ---------------------------------------------------------------------------

@@ -77,31 +77,91 @@ __device__ __forceinline__ int row_exp(double m) {
   return e;
 }
 
-__device__ __forceinline__ void slice4(double x, int e, signed char s[4]) {
-  if (e == -127) {
-    s[0] = s[1] = s[2] = s[3] = 0;
-    return;
-  }
-  double y = ldexp(x, 6 - e);  // |y| < 64
-  double a = rint(y);
-  s[0] = (signed char)a;
-  double r = y - a;  // |r| <= 1/2, exact
+// 2^e as a double, e in the normal range
+__device__ __forceinline__ double pow2(int e) {
+  return __longlong_as_double((long long)(e + 1023) << 52);
+}
+// 2^e, or 0 for the zero-row exponent marker -127
+__device__ __forceinline__ double pow2_or_zero(int e) { return e == -127 ? 0.0 : pow2(e); }
+
+// Byte 0 of a .. d as one word
+__device__ __forceinline__ int bytes4(unsigned a, unsigned b, unsigned c, unsigned d) {
+  return (int)(__builtin_amdgcn_perm(b, a, 0x0c0c0400u) |
+               __builtin_amdgcn_perm(d, c, 0x04000c0cu));
+}
+
+// Slices of 16 elements |x| < 2^e, none NaN (e = -127: all zero): four roundings
+// half to even, each of the exact remainder of the one before.  A rounding is one
+// FMA onto 1.5 2^52, whose low byte is the slice: thirteen instructions an element
+// with the packing, where ldexp, rint, conversions and byte stores took 24.
+__device__ __forceinline__ void slice16(const double (&x)[16], int e, v4i (&out)[4]) {
+  const double sc = e == -127 ? 0.0 : pow2(6 - e);
+  constexpr double M = 0x1.8p52;
 #pragma unroll
-  for (int i = 1; i < 4; ++i) {
-    y = r * 128.0;
-    a = rint(y);
-    s[i] = (signed char)a;
-    r = y - a;
+  for (int w = 0; w < 4; ++w) {
+    unsigned d[4][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double t = fma(x[4 * w + k], sc, M);
+      double r = fma(x[4 * w + k], sc, M - t);  // exact, |r| <= 1/2
+      d[0][k] = (unsigned)__double2loint(t);
+#pragma unroll
+      for (int p = 1; p < 4; ++p) {
+        t = fma(r, 128.0, M);
+        if (p < 3) r = fma(r, 128.0, M - t);
+        d[p][k] = (unsigned)__double2loint(t);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) out[p][w] = bytes4(d[p][0], d[p][1], d[p][2], d[p][3]);
   }
 }
 
-__device__ __forceinline__ double unslice(const signed char *plane0, int off, int e) {
-  if (e == -127) return 0.0;
-  const double v = (double)plane0[off] + ldexp((double)plane0[PLANE + off], -7) +
-                   ldexp((double)plane0[2 * PLANE + off], -14) +
-                   ldexp((double)plane0[3 * PLANE + off], -21);
-  return ldexp(v, e - 6);
+// The four planes of 16 integers |V| <= 2^27 as balanced base-128 digits: V =
+// a0 2^21 + a1 2^14 + a2 2^7 + a3, a1 .. a3 in [-64, 63].  With V + kDigitBias
+// given (element e in byte e of a plane) the lower digits are seven-bit fields
+// a + 64; b - 64 for the four fields of a word at once is (b | 80) - 40, top bits
+// flipped.
+constexpr int kDigitBias = 64 * (1 + (1 << 7) + (1 << 14));
+__device__ __forceinline__ void pack16(const unsigned (&U)[16], v4i (&out)[4]) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int sh = 21 - 7 * p;
+      const unsigned b = (unsigned)bytes4(U[4 * w] >> sh, U[4 * w + 1] >> sh, U[4 * w + 2] >> sh,
+                                          U[4 * w + 3] >> sh);
+      out[p][w] = p == 0 ? (int)b : (int)(((b | 0x80808080u) - 0x40404040u) ^ 0x80808080u);
+    }
 }
+
+// High words of the largest |x| of 16; elements that are not finite are set to
+// zero first
+__device__ __forceinline__ unsigned max_hi(double (&x)[16]) {
+  auto top = [&]() {
+    unsigned m = 0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) m = max(m, (unsigned)__double2hiint(x[e]) & 0x7fffffffu);
+    return m;
+  };
+  unsigned m = top();
+  if (m >= 0x7ff00000u) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (!isfinite(x[e])) x[e] = 0.0;
+    m = top();
+  }
+  return m;
+}
+
+// Element e of 16 packed ones: its integer V, and all of them times `scale`
+// (2^(exponent - 27), or zero for a row stored as zero): exact.
+__device__ __forceinline__ int unslice_int(const v4i (&w)[4], int e) {
+  const int sh = 24 - 8 * (e & 3);
+  auto d = [&](int p) { return (int)((unsigned)w[p][e >> 2] << sh) >> 24; };
+  return (d(0) << 21) + (d(1) << 14) + (d(2) << 7) + d(3);
+}
+__device__ __forceinline__ double unslice_scale(int e) { return e == -127 ? 0.0 : pow2(e - 27); }
 
 __device__ __forceinline__ v4i ld16(const signed char *p) {
   return *reinterpret_cast<const v4i *>(p);
@@ -160,35 +220,37 @@ __device__ __forceinline__ double z_value(double ph, double gx, double gy, doubl
   return fma(bz, gz, fma(by, gy, fma(bx, gx, a * ph)));
 }
 
-// Slice a 64 x 64 FP64 tile held in LDS (v[row][k], row stride 65; TR: the
-// tile read transposed, v[k][row]) with per-row exponents ex[row] into a
-// section at dst (fragment order); one thread per (row fragment, lane) item,
-// 256 threads.  Inlined and specialised on TR: as a called function with a
-// run-time flag every element paid for the select and the call for its
-// register saves.  A row stored as zero (exponent -127) is sliced as 0.0
-// with exponent 0, so that slice4 takes no branch; its stored exponent stays
-// -127.
+// Item t of a 64 x 64 FP64 tile held in LDS (v[row][k], row stride 65; TR: the
+// tile read transposed, v[k][row]): row 16 (t / 64) + t % 16, k 16 ((t % 64) /
+// 16) .. +15.  Conflict-free in both orders.
 template <bool TR>
-__device__ __forceinline__ void store_section(const double (*v)[65], const int *ex,
-                                              signed char *dst) {
-  const int t = threadIdx.x;
-  const int rt = t >> 6, l = t & 63;
-  const int row = 16 * rt + (l & 15), k0 = 16 * (l >> 4);
-  const int er = ex[row];
-  const bool zero = er == -127;
-  __attribute__((aligned(16))) signed char out[4][16];
+__device__ __forceinline__ void tile_item(const double (*v)[65], double (&x)[16]) {
+  const int l = threadIdx.x & 63;
+  const int row = 16 * (threadIdx.x >> 6) + (l & 15), k0 = 16 * (l >> 4);
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const double x = TR ? v[k0 + e][row] : v[row][k0 + e];
-    signed char s[4];
-    slice4(zero ? 0.0 : x, zero ? 0 : er, s);
+  for (int e = 0; e < 16; ++e) x[e] = TR ? v[k0 + e][row] : v[row][k0 + e];
+}
+
+// Item t sliced with its row's exponent ex into a section at dst (fragment
+// order), 256 threads.
+__device__ __forceinline__ void store_item(const double (&x)[16], int ex, signed char *dst) {
+  const int t = threadIdx.x, l = t & 63;
+  v4i out[4];
+  slice16(x, ex, out);
 #pragma unroll
-    for (int p = 0; p < 4; ++p) out[p][e] = s[p];
-  }
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-    *reinterpret_cast<v4i *>(dst + p * PLANE + t * 16) = *reinterpret_cast<const v4i *>(out[p]);
-  if (t < 64) dst[4 * PLANE + t] = (signed char)ex[t];
+  for (int p = 0; p < 4; ++p) *reinterpret_cast<v4i *>(dst + p * PLANE + t * 16) = out[p];
+  if (l < 16) dst[4 * PLANE + 16 * (t >> 6) + l] = (signed char)ex;
+}
+
+// row_exp of the four items of a row (lanes l, l ^ 16, l ^ 32, l ^ 48); elements
+// that are not finite are set to zero.  The high word of the largest magnitude
+// holds its exponent.
+__device__ __forceinline__ int item_row_exp(double (&x)[16]) {
+  unsigned m = max_hi(x);
+  m = max(m, (unsigned)__shfl_xor((int)m, 16));
+  m = max(m, (unsigned)__shfl_xor((int)m, 32));
+  const int e = (int)(m >> 20) - 1022;
+  return e < -119 ? -127 : e;
 }
 
 // Direct global -> LDS copy of one section (4 planes + the 256-byte exponent
@@ -214,11 +276,5 @@ __device__ __forceinline__ void dma_section(const signed char *src, signed char 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima)
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-// 2^e as a double, e in the normal range
-__device__ __forceinline__ double pow2(int e) {
-  return __longlong_as_double((long long)(e + 1023) << 52);
-}
-// 2^e, or 0 for the zero-row exponent marker -127
-__device__ __forceinline__ double pow2_or_zero(int e) { return e == -127 ? 0.0 : pow2(e); }
 }  // namespace
 }  // namespace nkx

@@ -42,3 +42,29 @@ def test_closed_and_open_shell(case, split):
         assert (V - ref.potential).abs().max().item() <= 1e-7 * max(big, 1.0)
         assert torch.equal(V, V.t())
     assert abs(r.energy - ref.energy) <= 1e-6 and abs(r.n_el - ref.n_el) <= 1e-6
+
+
+@pytest.mark.parametrize("kind", ["zero", "tiny", "rows", "nan"])
+def test_slices_of_unusual_matrices(case, kind):
+    """Elements that are zero, below the smallest stored exponent, far apart in
+    one row, or not a number (which counts as zero, bit for bit)."""
+    c, nbf, P, ref = case
+    Q = P.clone()
+    if kind == "zero":
+        Q.zero_()
+    elif kind == "tiny":
+        Q *= 1e-200
+    elif kind == "rows":
+        s = torch.pow(2.0, -4.0 * (torch.arange(nbf, device="cuda", dtype=torch.float64) % 9))
+        Q = s[:, None] * Q * s[None, :]
+    else:
+        Q[0, nbf - 1] = Q[nbf - 1, 0] = 0.0
+    r = c.vxc(Q, precision="mixed")
+    if kind == "nan":
+        Q[0, nbf - 1] = Q[nbf - 1, 0] = float("nan")
+        n = c.vxc(Q, precision="mixed")
+        assert n.energy == r.energy and n.n_el == r.n_el and torch.equal(n.potential, r.potential)
+        return
+    f = c.vxc(Q, precision="fp64")
+    assert torch.isfinite(r.potential).all()
+    assert abs(r.energy - f.energy) <= 1e-6 and abs(r.n_el - f.n_el) <= 1e-6
