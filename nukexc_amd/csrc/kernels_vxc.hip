@@ -422,18 +422,19 @@ __global__ void __launch_bounds__(256) fill0_kernel(int64_t n, double *__restric
     x[i] = 0.0;
 }
 
-// Pd = P permuted and zero-padded, or its transpose
-__global__ void __launch_bounds__(256) gather_p_f64(int nbf, int nbf_pad,
-                                                    const int *__restrict__ fperm, int tr,
-                                                    const double *__restrict__ P,
-                                                    double *__restrict__ Pd) {
+// out = P permuted and zero-padded, or its transpose, one matrix per blockIdx.y
+__global__ void __launch_bounds__(256) gather_p_f64(GatherArgs a, int tr) {
+  const GatherP g = a.g[blockIdx.y];
+  const int nbf = g.nbf, nbf_pad = g.nfb * FB;
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (int64_t)nbf_pad * nbf_pad) return;
   const int i = (int)(e / nbf_pad), j = (int)(e % nbf_pad);
   double v = 0.0;
-  if (i < nbf && j < nbf)
-    v = tr ? P[(int64_t)fperm[j] * nbf + fperm[i]] : P[(int64_t)fperm[i] * nbf + fperm[j]];
-  Pd[e] = v;
+  if (i < nbf && j < nbf) {
+    const int fi = g.fperm[i], fj = g.fperm[j];
+    v = g.P[tr ? (int64_t)fj * nbf + fi : (int64_t)fi * nbf + fj];
+  }
+  static_cast<double *>(g.out)[e] = v;
 }
 
 // Z = (w/2) Phi for the overlap build (S = Phi W Phi^T through vgemm).
@@ -448,12 +449,19 @@ __global__ void __launch_bounds__(256) zoverlap_f64(int64_t s0, const int *__res
 }
 
 // ---------------------------------------------------------------------------
-void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, bool transpose,
-                 const double *P, double *Pd) {
-  const int64_t n = (int64_t)nbf_pad * nbf_pad;
-  hipLaunchKernelGGL(gather_p_f64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, nbf,
-                     nbf_pad, fperm, transpose ? 1 : 0, P, Pd);
-  NKX_HIP_CHECK(hipGetLastError());
+void vk_gather_p(hipStream_t s, const std::vector<GatherP> &g, bool transpose) {
+  for (size_t k = 0; k < g.size(); k += kGatherMax) {
+    GatherArgs a{};
+    const size_t n = std::min<size_t>(kGatherMax, g.size() - k);
+    int64_t e = 0;
+    for (size_t i = 0; i < n; ++i) {
+      a.g[i] = g[k + i];
+      e = std::max(e, (int64_t)FB * a.g[i].nfb * FB * a.g[i].nfb);
+    }
+    hipLaunchKernelGGL(gather_p_f64, dim3((unsigned)((e + 255) / 256), (unsigned)n), dim3(256), 0,
+                       s, a, transpose ? 1 : 0);
+    NKX_HIP_CHECK(hipGetLastError());
+  }
 }
 
 void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr,

@@ -538,6 +538,7 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
   int t = tm.begin(kStageFinal, s);
   uint16_t *bstore = reinterpret_cast<uint16_t *>(ws.mstore.p);
   uint16_t *bPs = reinterpret_cast<uint16_t *>(ws.Ps.p);
+  std::vector<GatherP> gp;
   for (int sp = 0; sp < nspin; ++sp)
     for (int m = 0; m < nmol; ++m) {
       const double *Pm = P[(size_t)sp * nmol + m];
@@ -545,15 +546,18 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
       const int *fp = pl.fperm_d.p + (size_t)pl.mol_blk0_h[m] * FB;
       if (bf16)
         vkb_gather_p(s, nbf, pl.nfb, fp, Pm, bPs);
-      else if (mixed)
-        vkm_gather_p(s, nbf, pl.mol_nfb_h[m], fp, Pm,
-                     ws.Ps.p + (size_t)sp * b.psb + pl.mol_Ps_off_h[m]);
       else
-        vk_gather_p(s, nbf, pl.mol_ld_h[m], fp, true, Pm,
-                    ws.Pd.p + (size_t)sp * pl.P_total + pl.mol_P_off_h[m]);
+        gp.push_back({Pm, fp,
+                      mixed ? (void *)(ws.Ps.p + (size_t)sp * b.psb + pl.mol_Ps_off_h[m])
+                            : (void *)(ws.Pd.p + (size_t)sp * pl.P_total + pl.mol_P_off_h[m]),
+                      nbf, pl.mol_nfb_h[m]});
       // the elements of block pairs without a common batch are never written
       if (!pl.pairs_full) vk_fill0(s, V[(size_t)sp * nmol + m], (int64_t)nbf * nbf);
     }
+  if (mixed && !bf16)
+    vkm_gather_p(s, gp);
+  else
+    vk_gather_p(s, gp, true);
   tm.end(t, s);
   for_each_chunk(pl, b.slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
     const int ig = b.gga ? 1 : 0;
@@ -929,13 +933,15 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
          *gacc = cpart + n_cp, *gfun = gacc + n_ga, *wpart = gfun + n_gf, *wsum = wpart + n_wp;
   ws.gint.reserve(pl.npts_pad);
 
-  for (int sp = 0; sp < nspin; ++sp) {
-    if (mixed)
-      vkm_gather_p(s, pl.nbf, pl.mol_nfb_h[0], pl.fperm_d.p, P[sp], ws.Ps.p + sp * psb);
-    else
-      vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, true, P[sp],
-                  ws.Pd.p + (size_t)sp * pl.P_total);
-  }
+  std::vector<GatherP> gp;
+  for (int sp = 0; sp < nspin; ++sp)
+    gp.push_back({P[sp], pl.fperm_d.p,
+                  mixed ? (void *)(ws.Ps.p + sp * psb) : (void *)(ws.Pd.p + (size_t)sp * pl.P_total),
+                  pl.nbf, pl.mol_nfb_h[0]});
+  if (mixed)
+    vkm_gather_p(s, gp);
+  else
+    vk_gather_p(s, gp, true);
   vk_fill0(s, gacc, (int64_t)n_ga);
   const int ig = gga ? 1 : 0;
   double *coef_b = ws.coef.p + (size_t)4 * pl.npts_pad;
@@ -1023,7 +1029,7 @@ void density_points(Ctx &c, const double *P, double *rho, double *gx, double *gy
   ws.gbuf.reserve((size_t)4 * pl.npts_pad);
   XcList none{};
   none.n = 0;
-  vk_gather_p(s, pl.nbf, pl.nbf_pad, pl.fperm_d.p, true, P, ws.Pd.p);
+  vk_gather_p(s, {{P, pl.fperm_d.p, ws.Pd.p, pl.nbf, pl.mol_nfb_h[0]}}, true);
   for_each_chunk(pl, slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
     vk_colloc(s, s0, s1, pl, narr, ws.tiles64.p);
     vk_density(s, 1, 2, b0, b1, s0, pl, ws.Pd.p, narr, 1, ws.tiles64.p, ws.dpart.p, 0);

@@ -19,9 +19,21 @@ void vk_plan_screen(hipStream_t s, int64_t nb, int nbf, int nfb, const double *b
 void vk_plan_fill(hipStream_t s, int64_t nb, int nfb, int blk0, int64_t b0,
                   const unsigned char *live, const int *b_off, int *b_fbl, int *slot_b,
                   int *tile_slot, int *pairs);
-// Pd = P permuted and zero-padded, or its transpose
-void vk_gather_p(hipStream_t s, int nbf, int nbf_pad, const int *fperm, bool transpose,
-                 const double *P, double *Pd);
+// One density matrix to gather: P (device, nbf x nbf), the molecule's function
+// permutation, its blocks and where the gathered form goes.  Any number in one
+// launch per kGatherMax.
+struct GatherP {
+  const double *P;
+  const int *fperm;
+  void *out;
+  int nbf, nfb;
+};
+constexpr int kGatherMax = 32;
+struct GatherArgs {
+  GatherP g[kGatherMax];
+};
+// out = P permuted and zero-padded (64 nfb square), or its transpose
+void vk_gather_p(hipStream_t s, const std::vector<GatherP> &g, bool transpose);
 // Phi per live slot, array 0 of narr
 void vk_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr,
                double *tiles);
@@ -73,8 +85,7 @@ void vk_fill0(hipStream_t s, double *x, int64_t n);
 // the gathered P mixed_p_bytes(nfb)
 int64_t mixed_slot_bytes(int gga);
 int64_t mixed_p_bytes(int nfb);
-void vkm_gather_p(hipStream_t s, int nbf, int nfb, const int *fperm, const double *P,
-                  signed char *Ps);
+void vkm_gather_p(hipStream_t s, const std::vector<GatherP> &g);
 void vkm_colloc(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int gga,
                 signed char *store);
 // Pm sections of a batch's exponent groups re-sliced to shared point exponents
