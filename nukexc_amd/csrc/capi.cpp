@@ -311,35 +311,46 @@ void build_grid(nkx::Ctx &c, int natoms, const double *xyz, const int *Z, int nr
   const int64_t n = poff.back();
   const int nshell = (int)sh_atom.size();
   hipStream_t s = c.stream;
-  nkx::DevBuf<double> p0, w0, xr, xw, xa, xc;
-  nkx::DevBuf<int> o0, xat, xru, xro, xrn;
-  nkx::DevBuf<int64_t> cnt, xpo;
-  xr.upload(sh_r.data(), sh_r.size(), s);
-  xw.upload(sh_w.data(), sh_w.size(), s);
-  xat.upload(sh_atom.data(), sh_atom.size(), s);
-  xru.upload(sh_rule.data(), sh_rule.size(), s);
-  xpo.upload(poff.data(), poff.size(), s);
-  xro.upload(rule_off.data(), rule_off.size(), s);
-  xrn.upload(rule_n.data(), rule_n.size(), s);
-  xa.upload(ang.data(), ang.size(), s);
-  xc.upload(xyz, 3 * (size_t)natoms, s);
-  p0.reserve(3 * n);
-  w0.reserve(n);
-  o0.reserve(n);
-  nkx::launch_grid_shells(s, nshell, xat.p, xr.p, xw.p, xru.p, xpo.p, xro.p, xrn.p, xc.p, xa.p,
-                          p0.p, w0.p, o0.p);
+  nkx::GridScratch &g = c.grid_ws;
+  double *xr, *xw, *xa, *xc;
+  int *xat, *xru, *xro, *xrn;
+  int64_t *xpo;
+  nkx::TablePack pack;
+  pack.add(xr, sh_r.data(), sh_r.size());
+  pack.add(xw, sh_w.data(), sh_w.size());
+  pack.add(xat, sh_atom.data(), sh_atom.size());
+  pack.add(xru, sh_rule.data(), sh_rule.size());
+  pack.add(xpo, poff.data(), poff.size());
+  pack.add(xro, rule_off.data(), rule_off.size());
+  pack.add(xrn, rule_n.data(), rule_n.size());
+  pack.add(xa, ang.data(), ang.size());
+  pack.add(xc, xyz, 3 * (size_t)natoms);
+  pack.upload(g.pin, g.tab, s);
+  g.pts.reserve(3 * n);
+  g.w.reserve(n);
+  g.owner.reserve(n);
+  nkx::launch_grid_shells(s, nshell, xat, xr, xw, xru, xpo, xro, xrn, xc, xa, g.pts.p, g.w.p,
+                          g.owner.p);
   out.centers_host.assign(xyz, xyz + 3 * natoms);
-  out.centers.upload(xyz, 3 * (size_t)natoms, s);
+  out.centers.upload(reinterpret_cast<const double *>(g.pin.p + pack.items.back().off),
+                     3 * (size_t)natoms, s);
   out.natoms = natoms;
   c.becke_rtab.reserve((size_t)natoms * natoms);
-  nkx::launch_becke(s, natoms, out.centers.p, n, p0.p, o0.p, w0.p, nkx::BECKE_CAPPED,
+  nkx::launch_becke(s, natoms, out.centers.p, n, g.pts.p, g.owner.p, g.w.p, nkx::BECKE_CAPPED,
                     c.becke_rtab.p);
-  cnt.reserve((n + 1023) / 1024 + 1);
+  g.counts.reserve((n + 1023) / 1024 + 1);
   out.pts.reserve(3 * n);
   out.w.reserve(n);
   out.owner.reserve(n);
-  out.npts = nkx::compact_points(s, n, w_thr, p0.p, w0.p, o0.p, out.pts.p, out.w.p,
-                                 out.owner.p, nullptr, cnt.p);
+  out.npts = nkx::compact_points(s, n, w_thr, g.pts.p, g.w.p, g.owner.p, out.pts.p, out.w.p,
+                                 out.owner.p, g.counts.p,
+                                 reinterpret_cast<int64_t *>(c.out_doubles(1)));
+  if (n > nkx::kGridScratchPoints) {
+    g.pts.release();
+    g.w.release();
+    g.owner.release();
+    g.counts.release();
+  }
   out.version++;
 }
 

@@ -273,29 +273,49 @@ __global__ void __launch_bounds__(kCompactBlock) compact_scatter(
   }
 }
 
+// Exclusive sums of the block counts in place; their total to page-locked memory.
+__global__ void __launch_bounds__(kCompactBlock) compact_scan(int64_t nb,
+                                                              int64_t *__restrict__ counts,
+                                                              int64_t *__restrict__ total) {
+  __shared__ int64_t part[kCompactBlock / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int64_t run = 0;
+  for (int64_t i0 = 0; i0 < nb; i0 += kCompactBlock) {
+    const int64_t i = i0 + threadIdx.x;
+    const int64_t c = i < nb ? counts[i] : 0;
+    int64_t v = c;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t u = __shfl_up(v, o);
+      if (lane >= o) v += u;
+    }
+    if (lane == 63) part[wv] = v;
+    __syncthreads();
+    int64_t before = run;
+    for (int k = 0; k < kCompactBlock / 64; ++k) {
+      if (k < wv) before += part[k];
+      run += part[k];
+    }
+    if (i < nb) counts[i] = before + v - c;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *total = run;
+}
+
 int64_t compact_points(hipStream_t s, int64_t n, double thr, const double *pin,
                        const double *win, const int *oin, double *pout, double *wout,
-                       int *oout, int * /*unused*/, int64_t *counts) {
+                       int *oout, int64_t *counts, int64_t *total) {
   if (n == 0) return 0;
   const int64_t nb = (n + kCompactBlock - 1) / kCompactBlock;
   hipLaunchKernelGGL(compact_count, dim3((unsigned)nb), dim3(kCompactBlock), 0, s, n, thr, win,
                      counts);
   NKX_HIP_CHECK(hipGetLastError());
-  std::vector<int64_t> h(nb);
-  NKX_HIP_CHECK(hipMemcpyAsync(h.data(), counts, nb * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  NKX_HIP_CHECK(hipStreamSynchronize(s));
-  int64_t tot = 0;
-  for (int64_t i = 0; i < nb; ++i) {
-    const int64_t c = h[i];
-    h[i] = tot;
-    tot += c;
-  }
-  NKX_HIP_CHECK(hipMemcpyAsync(counts, h.data(), nb * sizeof(int64_t), hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(compact_scan, dim3(1), dim3(kCompactBlock), 0, s, nb, counts, total);
+  NKX_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(compact_scatter, dim3((unsigned)nb), dim3(kCompactBlock), 0, s, n, thr, pin,
                      win, oin, counts, pout, wout, oout);
   NKX_HIP_CHECK(hipGetLastError());
   NKX_HIP_CHECK(hipStreamSynchronize(s));
-  return tot;
+  return *total;
 }
 
 // ---------------------------------------------------------------------------

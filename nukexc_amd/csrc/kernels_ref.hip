@@ -603,9 +603,9 @@ void xc_ref(Ctx &c, int nbf, int64_t npts, const RefGrads &in, bool grad, const 
   const int64_t ne = (npts + MP - 1) / MP;
   const size_t n_cf = 4 * NS * (size_t)npts, n_pt = (size_t)NS * nsplit * nbf * nbf;
   const size_t n_vb = nbf > 64 ? (size_t)NS * nbf * nbf : 0;
-  c.ws.scratch.reserve(n_cf + n_pt + n_vb + ne + 1);
-  double *coef = c.ws.scratch.p, *part = coef + n_cf, *vb = part + n_pt, *ep = vb + n_vb,
-         *Ed = ep + ne;
+  c.ws.scratch.reserve(n_cf + n_pt + n_vb + ne);
+  double *coef = c.ws.scratch.p, *part = coef + n_cf, *vb = part + n_pt, *ep = vb + n_vb;
+  double *Ed = c.out_doubles(1);
   const RhoOut none{};
   if (npts > 0) {
     constexpr int mode = NS == 2 ? kMoSpins : kMoXc;
@@ -636,8 +636,8 @@ void xc_ref(Ctx &c, int nbf, int64_t npts, const RefGrads &in, bool grad, const 
                        V0, V1);
     NKX_HIP_CHECK(hipGetLastError());
   }
-  NKX_HIP_CHECK(hipMemcpyAsync(E, Ed, sizeof(double), hipMemcpyDeviceToHost, s));
   NKX_HIP_CHECK(hipStreamSynchronize(s));
+  *E = *Ed;
 }
 
 }  // namespace

@@ -372,11 +372,15 @@ __device__ __forceinline__ void en_reduce(MolTab mt, int mol, const double *__re
     for (int c = 0; c < 3; ++c) out[3 * mol + c] = sv[c][0];
 }
 
+struct VArgs {
+  double *p[kVArgs];
+};
 __global__ void __launch_bounds__(256) finish_kernel(
     int npairs, int nsplit, int nz, const int *__restrict__ pair_I,
     const int *__restrict__ pair_J, const int *__restrict__ fperm, MolTab mt, int nmol,
     const int *__restrict__ mol_nbf, const double *__restrict__ vpart,
-    double *const *__restrict__ Vmol, const double *__restrict__ en, double *__restrict__ enout) {
+    VArgs va, double *const *__restrict__ Vmol, const double *__restrict__ en,
+    double *__restrict__ enout) {
   __shared__ double sv[3][256];
   const int64_t nv = (int64_t)npairs * nz * FB;
   if ((int64_t)blockIdx.x >= nv) {
@@ -410,7 +414,8 @@ __global__ void __launch_bounds__(256) finish_kernel(
   if (seg || j >= nbf || (I == J && mu > nu)) return;
   v = ((sv[0][nu] + sv[0][FB + nu]) + sv[0][2 * FB + nu]) + sv[0][3 * FB + nu];
   const int oi = fperm[I * FB + mu], oj = fperm[J * FB + nu];
-  double *V = Vmol[(int64_t)zs * nmol + mol];
+  const int out = zs * nmol + __builtin_amdgcn_readfirstlane(mol);
+  double *V = Vmol ? Vmol[out] : va.p[out];
   V[(int64_t)oi * nbf + oj] = v;
   V[(int64_t)oj * nbf + oi] = v;
 }
@@ -494,20 +499,22 @@ void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
 }
 
 void vk_finish(hipStream_t s, const Plan &pl, int nsplit, int nz, const double *vpart,
-               double *const *Vmol_dev, const double *en, double *enout) {
+               double *const *V, double *const *Vmol_dev, const double *en, double *enout) {
   const int64_t nv = (int64_t)pl.npairs * nz * FB;
   const int64_t nwg = nv + (en ? pl.nmol : 0);
   if (nwg == 0) return;
   NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "reduction grid too large");
+  VArgs va{};
+  if (!Vmol_dev) std::copy(V, V + (size_t)nz * pl.nmol, va.p);
   hipLaunchKernelGGL(finish_kernel, dim3((unsigned)nwg), dim3(256), 0, s, pl.npairs, nsplit, nz,
                      pl.pair_I.p, pl.pair_J.p, pl.fperm_d.p, pl.tab(), pl.nmol, pl.mol_nbf.p,
-                     vpart, Vmol_dev, en, enout);
+                     vpart, va, Vmol_dev, en, enout);
   NKX_HIP_CHECK(hipGetLastError());
 }
 
 void vk_en_reduce(hipStream_t s, const Plan &pl, const double *en, double *out) {
   hipLaunchKernelGGL(finish_kernel, dim3(pl.nmol), dim3(256), 0, s, 0, 0, 0, nullptr, nullptr,
-                     nullptr, pl.tab(), pl.nmol, nullptr, nullptr, nullptr, en, out);
+                     nullptr, pl.tab(), pl.nmol, nullptr, nullptr, VArgs{}, nullptr, en, out);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

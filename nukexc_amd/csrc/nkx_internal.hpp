@@ -223,6 +223,17 @@ struct PlanScratch {
   PinBuf pin_fn, pin_tab, pin_cnt;
 };
 
+// Scratch of the grid build, kept between builds of up to kGridScratchPoints
+// product points (36 bytes each) and given back after larger ones.
+constexpr int64_t kGridScratchPoints = (int64_t)1 << 22;
+struct GridScratch {
+  DevBuf<char> tab;      // shells, angular rules, centres
+  DevBuf<double> pts, w;
+  DevBuf<int> owner;
+  DevBuf<int64_t> counts;
+  PinBuf pin;
+};
+
 struct Options {
   double screen_tol = 1e-12;
   int batch_points = 64;
@@ -242,7 +253,6 @@ struct Workspace {
   DevBuf<double> vpart;            // split-K partial V tiles
   DevBuf<double> dpart;            // per spin and slot: column sums of the density contraction
   DevBuf<signed char> zstore_b;    // int8 form, second spin: Z sections per slot
-  DevBuf<double> red;              // small reduction outputs
   DevBuf<double> scratch;
   DevBuf<double> gbuf;             // nuclear-gradient buffers
   DevBuf<int> gint;
@@ -321,6 +331,15 @@ struct Ctx {
   PlanScratch plan_ws;
   Workspace ws;
   GraphState graph;
+  // results that kernels write straight into page-locked memory (E, N, the
+  // parts of a gradient, a count); read after the stream was waited for, before
+  // the next call that uses it
+  PinBuf out;
+  double *out_doubles(size_t n) {
+    out.reserve(n * sizeof(double));
+    return reinterpret_cast<double *>(out.p);
+  }
+  GridScratch grid_ws;
   DevBuf<double> becke_rtab;     // inter-atomic distances of the last partition
 };
 
@@ -352,10 +371,11 @@ void launch_becke(hipStream_t s, int natoms, const double *centers, int64_t npts
 constexpr int BECKE_SCRATCH_ATOMS = 512;
 void becke_scratch_init(int device);
 double *becke_scratch(int device);
+// Points with w > thr in order; counts: a number per 1024 points; total: page-
+// locked.  Waits for the stream.
 int64_t compact_points(hipStream_t s, int64_t n, double thr, const double *pts_in,
                        const double *w_in, const int *own_in, double *pts_out,
-                       double *w_out, int *own_out, int *scratch_flags,
-                       int64_t *scratch_scan);
+                       double *w_out, int *own_out, int64_t *counts, int64_t *total);
 
 void launch_collocation_ref(hipStream_t s, int nbf, const FuncRec *f,
                             const HarmTerm *t, int64_t npts, const double *pts,

@@ -448,10 +448,11 @@ void for_each_chunk(const Plan &pl, int64_t max_slots, F &&fn) {
 
 namespace {
 // Device table of output pointers (kept alive in the workspace until the
-// build synchronises).
-double *const *upload_ptrs(Ctx &c, const std::vector<double *> &ptrs) {
-  c.ws.vptr_h = ptrs;
-  c.ws.vptr.upload(c.ws.vptr_h.data(), c.ws.vptr_h.size(), c.stream);
+// build synchronises); none for as many as vk_finish takes by value.
+double *const *upload_ptrs(Ctx &c, double *const *V, size_t n) {
+  if (n <= (size_t)kVArgs) return nullptr;
+  c.ws.vptr_h.assign(V, V + n);
+  c.ws.vptr.upload(c.ws.vptr_h.data(), n, c.stream);
   return c.ws.vptr.p;
 }
 }  // namespace
@@ -506,7 +507,6 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   ws.blockEN.reserve((size_t)3 * pl.nb);
   b.vsz = (size_t)b.nsplit * std::max(pl.npairs, 1) * FB * FB;
   ws.vpart.reserve(nspin * b.vsz);
-  ws.red.reserve((size_t)3 * pl.nmol);
   return b;
 }
 
@@ -611,11 +611,9 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
     tm.end(tt, s);
   });
   t = tm.begin(kStageFinal, s);
-  vk_finish(s, pl, nsplit, nspin, ws.vpart.p, Vtab, ws.blockEN.p, ws.red.p);
+  vk_finish(s, pl, nsplit, nspin, ws.vpart.p, V, Vtab, ws.blockEN.p, en_dst);
   tm.end(t, s);
   tm.end(t_build, s);
-  NKX_HIP_CHECK(hipMemcpyAsync(en_dst, ws.red.p, (size_t)3 * nmol * sizeof(double),
-                               hipMemcpyDeviceToHost, s));
 }
 
 // One V_xc build on plan pl.  Molecule m, spin sp: density matrix
@@ -627,9 +625,9 @@ void build_on_plan(Ctx &c, Plan &pl, int nspin, const double *const *P, const Xc
   const BuildSetup b =
       prepare_build(c.ws, pl, nspin, gga, precision, c.opt.vgemm_split, c.opt.density_group,
                     c.opt.mem_budget);
-  double *const *Vtab = upload_ptrs(c, std::vector<double *>(V, V + (size_t)nspin * nmol));
-  std::vector<double> en((size_t)3 * nmol);
-  enqueue_build(c, c.ws, pl, b, P, xl, V, Vtab, en.data());
+  double *const *Vtab = upload_ptrs(c, V, (size_t)nspin * nmol);
+  double *en = c.out_doubles((size_t)3 * nmol);
+  enqueue_build(c, c.ws, pl, b, P, xl, V, Vtab, en);
   NKX_HIP_CHECK(hipStreamSynchronize(c.stream));
   c.timing.collect();
   c.work.flops_density = 2.0 * nspin * pl.work_nb2g;
@@ -920,17 +918,18 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
   ws.dpart.reserve(nspin * dsz);
   ws.coef.reserve((size_t)4 * nspin * pl.npts_pad);
   ws.blockEN.reserve((size_t)3 * pl.nb);
-  ws.red.reserve(3);
-  // gradient buffers: ptab, epoint, tpt, cpart, gacc, gfun, wpart, wsum
+  // gradient buffers: ptab, epoint, tpt, cpart, gacc, wpart
   const size_t n_ep = pl.npts_pad, n_tp = 3 * pl.npts_pad, n_cp = (size_t)slots_alloc * 3 * FB;
   const size_t n_ga = (size_t)nseg * pl.nbf_pad * 3, n_gf = (size_t)pl.nbf_pad * 3;
   const size_t n_wp = (size_t)nblk * 3 * natoms, n_ws = (size_t)3 * natoms;
   // atom-pair table first, rounded to 256 bytes, so the others keep the
   // alignment of the allocation
   const size_t n_pt = ((size_t)2 * natoms * natoms + 31) & ~(size_t)31;
-  ws.gbuf.reserve(n_pt + n_ep + n_tp + n_cp + n_ga + n_gf + n_wp + n_ws);
+  ws.gbuf.reserve(n_pt + n_ep + n_tp + n_cp + n_ga + n_wp);
   double *ptab = ws.gbuf.p, *epoint = ptab + n_pt, *tpt = epoint + n_ep, *cpart = tpt + n_tp,
-         *gacc = cpart + n_cp, *gfun = gacc + n_ga, *wpart = gfun + n_gf, *wsum = wpart + n_wp;
+         *gacc = cpart + n_cp, *wpart = gacc + n_ga;
+  // the results, page-locked: E, N; sums per atom; sums per function
+  double *en = c.out_doubles(3 + n_ws + n_gf), *wsum = en + 3, *gfun = wsum + n_ws;
   ws.gint.reserve(pl.npts_pad);
 
   std::vector<GatherP> gp;
@@ -988,20 +987,15 @@ void xc_grad(Ctx &c, int nspin, const double *const *P, const XcList &xl, bool g
     }
   });
   vkg_colsum(s, nseg, pl.nbf_pad * 3, gacc, gfun);
-  vk_en_reduce(s, pl, ws.blockEN.p, ws.red.p);
+  vk_en_reduce(s, pl, ws.blockEN.p, en);
   vkg_owners(s, pl, c.grid.owner.p, ws.gint.p);
   vkg_weights(s, pl, natoms, c.grid.centers.p, ws.gint.p, epoint, tpt, partition, nblk, ptab,
               wpart);
   vkg_colsum(s, nblk, 3 * natoms, wpart, wsum);
-  std::vector<double> gf(n_gf), wsh(n_ws);
-  double en[3];
-  NKX_HIP_CHECK(hipMemcpyAsync(gf.data(), gfun, n_gf * sizeof(double), hipMemcpyDeviceToHost, s));
-  NKX_HIP_CHECK(hipMemcpyAsync(wsh.data(), wsum, n_ws * sizeof(double), hipMemcpyDeviceToHost, s));
-  NKX_HIP_CHECK(hipMemcpyAsync(en, ws.red.p, sizeof(en), hipMemcpyDeviceToHost, s));
   NKX_HIP_CHECK(hipStreamSynchronize(s));
-  for (int k = 0; k < 3 * natoms; ++k) grad[k] = wsh[k];
+  for (int k = 0; k < 3 * natoms; ++k) grad[k] = wsum[k];
   for (int sp = 0; sp < pl.nbf; ++sp)
-    for (int k = 0; k < 3; ++k) grad[3 * fatom[sp] + k] += gf[3 * sp + k];
+    for (int k = 0; k < 3; ++k) grad[3 * fatom[sp] + k] += gfun[3 * sp + k];
   *E = en[0];
 }
 
@@ -1093,13 +1087,12 @@ void overlap_build(Ctx &c, double *S) {
   const size_t vsz = (size_t)nsplit * std::max(pl.npairs, 1) * FB * FB;
   ws.vpart.reserve(vsz);
   vk_fill0(s, S, (int64_t)pl.nbf * pl.nbf);
-  double *const *Stab = upload_ptrs(c, std::vector<double *>{S});
   for_each_chunk(pl, slots_alloc, [&](int64_t b0, int64_t b1, int64_t s0, int64_t s1) {
     vk_colloc(s, s0, s1, pl, narr, ws.tiles64.p);
     vk_zoverlap(s, s0, s1, pl, narr, ws.tiles64.p);
     vk_vgemm(s, b0, b1, s0, pl, nsplit, narr, 1, b0 == 0, ws.tiles64.p, ws.vpart.p);
   });
-  vk_finish(s, pl, nsplit, 1, ws.vpart.p, Stab, nullptr, nullptr);
+  vk_finish(s, pl, nsplit, 1, ws.vpart.p, &S, nullptr, nullptr, nullptr);
   NKX_HIP_CHECK(hipStreamSynchronize(s));
 }
 

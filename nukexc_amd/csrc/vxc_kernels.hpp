@@ -71,11 +71,12 @@ void vk_zoverlap(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr
 // writes the partials (the later ones add to them)
 void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
               int narr, int nz, bool first, const double *tiles, double *vpart);
-// V of spin z and molecule m is Vmol_dev[z * nmol + m] (device array of device
-// pointers), from the nz sets of partials; en (may be NULL): per-batch
+// V of spin z and molecule m is V[z * nmol + m] (host array of device pointers,
+// also as a device array Vmol_dev where there are more than kVArgs), from the nz sets of partials; en (may be NULL): per-batch
 // triples summed per molecule into enout as vk_en_reduce
+constexpr int kVArgs = 32;
 void vk_finish(hipStream_t s, const Plan &pl, int nsplit, int nz, const double *vpart,
-               double *const *Vmol_dev, const double *en, double *enout);
+               double *const *V, double *const *Vmol_dev, const double *en, double *enout);
 // out[3 m + c] = (E, N_alpha, N_beta) of molecule m
 void vk_en_reduce(hipStream_t s, const Plan &pl, const double *en, double *out);
 void vk_fill0(hipStream_t s, double *x, int64_t n);
