@@ -87,8 +87,9 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
 // rows fall on sixteen different bank groups.
 //
 // Bound by the FP64 MFMA rate (busy 70 % of the cycles; the rest is the wait at
-// a stage's start, one workgroup per CU): 16 waters take 8.7 ms, 48 TFLOP/s,
-// a 12-atom molecule with two spins 402 us, water 26 us.  One workgroup per
+// a stage's start, one workgroup per CU): 16 waters take 7.9 ms, 52 TFLOP/s,
+// a 12-atom molecule with two spins 341 us, water 24 us (8.5 ms, 361 us and 27 us
+// with each stage's slots looked up in LDS between its barrier and its copies).  One workgroup per
 // block pair, both products on the diagonal too, read four tiles for every two
 // products of them (58 GB on 16 waters): 9.9 ms, 737 us and 245 us.
 constexpr int VS = 16;             // points of a stage
@@ -147,13 +148,21 @@ __global__ void __launch_bounds__(512) vgemm_f64(
   struct AFrag {
     v4d f[2], z[2];  // rows of Phi_I, Z_I per row group
   };
-  auto slot = [&](int u, int i) { return __builtin_amdgcn_readfirstlane(ls[u][i]); };
-  // operands of stage st (point group) of listed batch i: this wave's rows to
+  // a listed batch's slots of this wave's I block and of the J blocks, read a
+  // batch ahead (so that no LDS look-up sits between a barrier and the copies)
+  struct Slots {
+    int I, J[2];
+  };
+  auto slots = [&](int i) {
+    return Slots{__builtin_amdgcn_readfirstlane(ls[wa][i]),
+                 {__builtin_amdgcn_readfirstlane(ls[2][i]),
+                  __builtin_amdgcn_readfirstlane(ls[3][i])}};
+  };
+  // operands of stage st (point group) of a batch: this wave's rows to
   // registers (those of slot s0 where its tile is idle: never used), the J
   // blocks to LDS
-  auto issue = [&](int i, int st, double (*dst)[VSEC], AFrag &a) {
-    const int sI = slot(wa, i);
-    const double *pI = tiles + (int64_t)(sI >= 0 ? sI - s0 : 0) * narr * TILE +
+  auto issue = [&](const Slots &sl, int st, double (*dst)[VSEC], AFrag &a) {
+    const double *pI = tiles + (int64_t)(sl.I >= 0 ? sl.I - s0 : 0) * narr * TILE +
                        (row0 + l16) * PT + VS * st + 4 * q;
     a.f[0] = ld4(pI);
     if (two) a.f[1] = ld4(pI + 16 * PT);
@@ -165,11 +174,11 @@ __global__ void __launch_bounds__(512) vgemm_f64(
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb) {
       if (jb && !two) continue;
-      const int sJ = slot(2 + jb, i);
-      if (sJ < 0) continue;
+      if (sl.J[jb] < 0) continue;
       const int r = 8 * wv + (lane >> 3);
       const int c = (lane & 7) ^ ((r >> 1) & 7);
-      const double *src = tiles + (int64_t)(sJ - s0) * narr * TILE + r * PT + VS * st + 2 * c;
+      const double *src =
+          tiles + (int64_t)(sl.J[jb] - s0) * narr * TILE + r * PT + VS * st + 2 * c;
       __builtin_amdgcn_global_load_lds(src + zoff, &dst[jb][8 * wv * VS], 16, 0, 0);
       if (!diag) __builtin_amdgcn_global_load_lds(src, &dst[2 + jb][8 * wv * VS], 16, 0, 0);
     }
@@ -198,18 +207,13 @@ __global__ void __launch_bounds__(512) vgemm_f64(
     }
   };
   AFrag a0, a1;
-  // stage t of a window of n batches: wait for its operands, start the next
-  // stage's, form its products
-  auto step = [&](int t, int n, double (*cur)[VSEC], double (*nxt)[VSEC], const AFrag &a,
-                  AFrag &an) {
+  auto ready = [&]() {  // the stage's operands are there, the other buffer is free
     wait_vm0();
-    __syncthreads();  // cur complete, nxt free
-    if (t + 1 < 4 * n) issue((t + 1) >> 2, (t + 1) & 3, nxt, an);
-    const int i = t >> 2;
-    if (slot(wa, i) >= 0 && slot(2 + wb, i) >= 0) {
-      phase(&cur[wb][0], a.f);
-      if (!diag) phase(&cur[2 + wb][0], a.z);
-    }
+    __syncthreads();
+  };
+  auto products = [&](double (*cur)[VSEC], const AFrag &a) {
+    phase(&cur[wb][0], a.f);
+    if (!diag) phase(&cur[2 + wb][0], a.z);
   };
 
   for (int64_t c0 = lo + split; c0 < hi; c0 += 512 * (int64_t)nsplit) {
@@ -238,10 +242,24 @@ __global__ void __launch_bounds__(512) vgemm_f64(
     }
     __syncthreads();
     if (n == 0) continue;
-    issue(0, 0, bufA, a0);
-    for (int t = 0; t < 4 * n; t += 2) {  // an even number of stages
-      step(t, n, bufA, bufB, a0, a1);
-      step(t + 1, n, bufB, bufA, a1, a0);
+    Slots cur = slots(0);
+    issue(cur, 0, bufA, a0);
+    for (int i = 0; i < n; ++i) {
+      const bool live = cur.I >= 0 && (wb ? cur.J[1] : cur.J[0]) >= 0;
+      ready();
+      issue(cur, 1, bufB, a1);
+      if (live) products(bufA, a0);
+      ready();
+      issue(cur, 2, bufA, a0);
+      const Slots nxt = slots(i + 1 < n ? i + 1 : i);
+      if (live) products(bufB, a1);
+      ready();
+      issue(cur, 3, bufB, a1);
+      if (live) products(bufA, a0);
+      ready();
+      if (i + 1 < n) issue(nxt, 0, bufA, a0);
+      if (live) products(bufB, a1);
+      cur = nxt;
     }
   }
 

@@ -849,23 +849,31 @@ __device__ __forceinline__ void vgemm_i8_tile(
       ex[g] = *reinterpret_cast<const int *>(sec + 4 * PLANE + 16 * rg + 4 * q);
     }
   };
-  // whether the wave's tile has work in listed batch i
-  auto active = [&](int i) {
-    return tile && __builtin_amdgcn_readfirstlane(ls[wa][i]) >= 0 &&
-           __builtin_amdgcn_readfirstlane(ls[2 + wb][i]) >= 0;
+  // a listed batch's slots of this wave's I block and of the J blocks, read a
+  // batch ahead of their use (so that no LDS look-up sits between a barrier and
+  // the copies: 185 -> 177 us on benzene, 16.9 -> 16.4 ms on 32 waters)
+  struct Slots {
+    int I, J[2];
   };
-  // F_I of batch i; where the wave's tile is idle in batch i (or past the
-  // list) the loads read slot s0 instead, whose values go unused, so that
-  // every path issues the same loads and the waits after them stay exact
-  auto next_F = [&](int i, int n) {
-    const int sI = i < n && active(i) ? __builtin_amdgcn_readfirstlane(ls[wa][i]) : (int)s0;
+  auto slots = [&](int i) {
+    return Slots{__builtin_amdgcn_readfirstlane(ls[wa][i]),
+                 {__builtin_amdgcn_readfirstlane(ls[2][i]),
+                  __builtin_amdgcn_readfirstlane(ls[3][i])}};
+  };
+  // whether the wave's tile has work in a batch
+  auto active = [&](const Slots &sl) { return tile && sl.I >= 0 && (wb ? sl.J[1] : sl.J[0]) >= 0; };
+  // F_I of a batch; where the wave's tile is idle in it (or past the list) the
+  // loads read slot s0 instead, whose values go unused, so that every path
+  // issues the same loads and the waits after them stay exact
+  auto next_F = [&](bool any, const Slots &sl) {
+    const int sI = any && active(sl) ? sl.I : (int)s0;
     load_I(f_section(sI), Fr, eF);
   };
-  // J sections of listed batch i -> LDS buffer dst (direct copies)
-  auto issue_J = [&](int i, signed char (*dst)[SEC]) {
+  // J sections of a batch -> LDS buffer dst (direct copies)
+  auto issue_J = [&](const Slots &sl, signed char (*dst)[SEC]) {
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb) {
-      const int sJ = __builtin_amdgcn_readfirstlane(ls[2 + jb][i]);
+      const int sJ = sl.J[jb];
       if (sJ < 0) continue;
       dma_section<8>(z_section(sJ), &dst[2 * jb][0], (wv + 4 * jb) & 7, lane);
       if (!diag) dma_section<8>(f_section(sJ), &dst[2 * jb + 1][0], (wv + 4 * jb + 2) & 7, lane);
@@ -876,10 +884,10 @@ __device__ __forceinline__ void vgemm_i8_tile(
   // compiler's wait insertion stops telling the copies into bufB apart from
   // the reads of bufA and waits for them before every batch's first LDS
   // read), and F_I
-  auto fill = [&](int n, signed char (*dst)[SEC]) {
+  auto fill = [&](const Slots &sl, signed char (*dst)[SEC]) {
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb) {
-      const int sJ = __builtin_amdgcn_readfirstlane(ls[2 + jb][0]);
+      const int sJ = sl.J[jb];
       if (sJ < 0) continue;
       const signed char *src[2] = {z_section(sJ), f_section(sJ)};
 #pragma unroll
@@ -898,7 +906,7 @@ __device__ __forceinline__ void vgemm_i8_tile(
         }
       }
     }
-    next_F(0, n);
+    next_F(true, sl);
   };
   // one phase of a batch: A = F_I (p = 0) or Z_I (p = 1) against the Z or F
   // section of J_b; the B fragment of column fragment j + 1 is read from LDS
@@ -935,15 +943,19 @@ __device__ __forceinline__ void vgemm_i8_tile(
   // one listed batch: wait for its operands, load Z_I, start the next
   // batch's J copies, then the two phases with F_I of the next batch loaded
   // between them
-  auto step = [&](int i, int n, signed char (*cur)[SEC], signed char (*nxt)[SEC]) {
+  auto step = [&](int i, int n, Slots &sc, Slots &sn, signed char (*cur)[SEC],
+                  signed char (*nxt)[SEC]) {
     wait_vm0();
     __syncthreads();  // buffer cur complete, nxt free
-    const bool act = active(i);
-    if (act && !diag) load_I(z_section(__builtin_amdgcn_readfirstlane(ls[wa][i])), Zr, eZ);
-    if (i + 1 < n) issue_J(i + 1, nxt);
+    const bool act = active(sc);
+    if (act && !diag) load_I(z_section(sc.I), Zr, eZ);
+    if (i + 1 < n) issue_J(sn, nxt);
+    const Slots s2 = slots(i + 2 < n ? i + 2 : n - 1);
     if (act) phase(0, cur);
-    next_F(i + 1, n);
+    next_F(i + 1 < n, sn);
     if (act && !diag) phase(1, cur);
+    sc = sn;
+    sn = s2;
   };
 
   for (int64_t c0 = lo + split; c0 < hi; c0 += 512 * (int64_t)nsplit) {
@@ -972,10 +984,11 @@ __device__ __forceinline__ void vgemm_i8_tile(
     }
     __syncthreads();
     if (n == 0) continue;
-    fill(n, bufA);
+    Slots sc = slots(0), sn = slots(n > 1 ? 1 : 0);
+    fill(sc, bufA);
     for (int i = 0; i < n; i += 2) {
-      step(i, n, bufA, bufB);
-      if (i + 1 < n) step(i + 1, n, bufB, bufA);
+      step(i, n, sc, sn, bufA, bufB);
+      if (i + 1 < n) step(i + 1, n, sc, sn, bufB, bufA);
     }
   }
   if (diag) {
