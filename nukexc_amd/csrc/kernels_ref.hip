@@ -311,7 +311,8 @@ __global__ void __launch_bounds__(64) xc_pol_ref(int64_t npts, int gga, XcList x
 // Bound by reading the four matrices up to about 64 functions, by the FP64
 // MFMA rate above.  With Z as a matrix of its own and a VALU kernel with
 // atomics this took 318 + 772 us per spin on benzene and 81 + 247 us on water;
-// now 511 us for both spins (33 TFLOP/s) and 15 us (3.5 TB/s).
+// now 450 us for both spins (38 TFLOP/s; 510 us with every wave forming Z after
+// its products) and 15 us (3.5 TB/s).
 template <int TM>
 struct ZvShape {
   static constexpr int threads = TM == 128 ? 512 : 256;
@@ -396,18 +397,24 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
     load(k0);
     __syncthreads();
     store(0, 0);
+    if (nst > 1) load(k0 + KP);
     __syncthreads();
   }
+  // Waves w and w + 4 share a SIMD: one forms Z before its products, the other
+  // after them, so that the matrix cores do not wait for both.
+  const bool first = TM == 128 && wv < 4;
   int ring = 1;  // of stage s + 1
   for (int s = 0; s < nst; ++s) {
-    const int64_t kn = k0 + (int64_t)(s + 1) * KP;
     const bool more = s + 1 < nst;
-    double cn = 0.0;
-    if (more) {
-      load(kn);
-      cn = load_coef(kn + KP);
-    }
+    const double cn = more ? load_coef(k0 + (int64_t)(s + 2) * KP) : 0.0;
     const int b = s & 1;
+    // the next stage into the other buffer, and the loads of the one after
+    auto next = [&]() {
+      if (!more) return;
+      store(b ^ 1, ring);
+      if (s + 2 < nst) load(k0 + (int64_t)(s + 2) * KP);
+    };
+    if (first) next();
 #pragma unroll
     for (int ks = 0; ks < KP; ks += 4) {
       double av[NI], zv[NS][NJ];
@@ -428,11 +435,9 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
                                                                    acc[sp][i][j], 0, 0, 0);
           }
     }
+    if (!first) next();
     const int ring2 = ring == 2 ? 0 : ring + 1;
-    if (more) {
-      store_coef(ring2, cn);
-      store(b ^ 1, ring);
-    }
+    if (more) store_coef(ring2, cn);
     ring = ring2;
     __syncthreads();
   }
