@@ -132,9 +132,14 @@ struct StoRun {
   __device__ __forceinline__ void eval(const FuncRec &f, const FuncRec &prev, bool first,
                                        const HarmTerm *__restrict__ T, double x, double y,
                                        double z, double &v, double (&gr)[3]) {
-    const bool newc = first || f.cx != prev.cx || f.cy != prev.cy || f.cz != prev.cz;
+    // bit patterns compared: scalar instructions on uniform records, no chain of
+    // branches
+    auto diff = [](double a, double b) { return __double_as_longlong(a) ^ __double_as_longlong(b); };
+    const bool newc =
+        first || (diff(f.cx, prev.cx) | diff(f.cy, prev.cy) | diff(f.cz, prev.cz)) != 0;
+    const bool news = (diff(f.zeta, prev.zeta) | diff(f.norm, prev.norm) | (f.k ^ prev.k)) != 0;
     if (newc) centre(x - f.cx, y - f.cy, z - f.cz);
-    if (newc || f.zeta != prev.zeta || f.k != prev.k || f.norm != prev.norm)
+    if (newc || news)
       shell<MIXED>(f.k, f.zeta, f.norm);
     double S, g[3];
     harmonic<GRAD>(f.type, f.term_off, f.term_cnt, T, S, g);
