@@ -34,7 +34,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 def kernel_name(precision, stage, shape):
     """Name of the kernel behind a timing stage for a density shape code."""
     if precision == "fp64":
-        return {"density": "density_x_f64", "vgemm": "vgemm_f64",
+        return {"density": "density_fused_f64", "vgemm": "vgemm_f64",
                 "collocation": "colloc_tiles_f64"}[stage]
     if precision == "mixed_bf16":
         return {"density": "density_fused_mixed", "vgemm": "vgemm_mixed",

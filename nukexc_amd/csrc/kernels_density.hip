@@ -1,5 +1,5 @@
 // FP64 density stage of the batched build (gfx950): the contraction X = P Phi
-// with its column sums (density_x_f64) and the Z arrays (z_slots_f64); the
+// with its column sums (density_fused_f64) and the Z arrays (z_slots_f64); the
 // per-batch functional between them is the one of the int8 form.
 #include <algorithm>
 
@@ -60,7 +60,7 @@ __device__ __forceinline__ void wave_fence() {
 // VGPRs, two barriers per step and 94 KB of LDS took 22.1 ms together with the
 // Z stage.
 template <bool GGA>
-__global__ void __launch_bounds__(256, 3) density_x_f64(
+__global__ void __launch_bounds__(256, 3) density_fused_f64(
     MolTab mt, int64_t pspin, int nspin, int group, const double *__restrict__ Pt,
     const int *__restrict__ b_off, const int *__restrict__ b_fbl, int64_t s0, int64_t b0,
     int64_t b1, int nmg, int narr, const FuncRec *__restrict__ F,
@@ -295,7 +295,7 @@ void vk_density(hipStream_t s, int nspin, int group, int64_t b0, int64_t b1, int
   const int64_t ng = ((b1 - b0 + g - 1) / g + 7) / 8 * 8;
   const int64_t nwg = ng * nmg * nspin;
   NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "density grid too large");
-  hipLaunchKernelGGL(gga ? density_x_f64<true> : density_x_f64<false>, dim3((unsigned)nwg),
+  hipLaunchKernelGGL(gga ? density_fused_f64<true> : density_fused_f64<false>, dim3((unsigned)nwg),
                      dim3(256), 0, s, pl.tab(), pl.P_total, nspin, g, Pt, pl.b_off.p, pl.b_fbl.p,
                      s0, b0, b1, nmg, narr, pl.funcs.p, pl.terms.p, pl.px.p, pl.py.p, pl.pz.p,
                      tiles, pstride, part);

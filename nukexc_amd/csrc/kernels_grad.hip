@@ -38,7 +38,7 @@ constexpr int GC = FB * 3;  // per-slot partial: 64 functions x 3 components
 // of a batch's live blocks, then grad_rows.  One workgroup of four waves per
 // (batch, pair of list blocks); a wave holds 32 rows of its block x 64 points
 // of both products (16 rows of the only block where the pair has one).  The
-// contraction is that of density_x_f64 (kernels_density.hip) in stages of 16
+// contraction is that of density_fused_f64 (kernels_density.hip) in stages of 16
 // functions: Phi and Y of the next stage go straight into the other LDS
 // buffer and the next P fragments into the other register set while the
 // current stage's products run.  The epilogue passes X and W of a wave through
@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(256, 2) grad_basis_f64(
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       // rows 2 rp, 2 rp + 1: 16 bytes per lane, halves exchanged in rows with
-      // bit 2 set (density_x_f64)
+      // bit 2 set (density_fused_f64)
       const int rp = 2 * wv + u, r = 2 * rp + (lane >> 5);
       const int c = (lane & 31) ^ (((rp >> 1) & 1) << 3);
       const double *g = src + r * PT + 2 * c;

@@ -246,7 +246,7 @@ struct Options {
 struct Workspace {
   DevBuf<double> Pd;               // permuted padded density matrix (FP64)
   DevBuf<signed char> Ps;          // int8 slice sections of the permuted P
-  DevBuf<double> tiles64;          // Phi, gx, gy, gz, Z tiles (FP64)
+  DevBuf<double> tiles64;          // Phi and Z tiles (FP64)
   DevBuf<signed char> mstore;      // mixed-form tile store (int8 slices + FP32 gradients)
   DevBuf<double> coef;             // per padded point and spin: a, bx, by, bz
   DevBuf<double> blockEN;          // per batch: E, N_alpha, N_beta partial sums
