@@ -59,8 +59,9 @@ struct RhoOut {
 // tiles on.  A thread per point with a scalar loop over orbitals and
 // functions reads each matrix once per orbital, uncoalesced: 41.6 ms per spin
 // on benzene (120 functions, 259 200 points, 21 and 20 orbitals), 288 us on
-// water (25 functions, 64 800 points, 5 orbitals); this form takes 364 us for
-// both spins (2.7 TB/s, 34 TFLOP/s) and 24 us.
+// water (25 functions, 64 800 points, 5 orbitals); this form takes 340 us for
+// both spins (2.9 TB/s; 364 us with tiles of each spin's own, four instead of
+// three) and 24 us.
 //
 // MODE 0 writes rho, grad rho and sigma of one spin; 1 evaluates the
 // functional and writes the Z coefficients (w v_rho / 2, 2 w v_sigma grad rho)
@@ -69,11 +70,12 @@ struct RhoOut {
 // the contraction can spare at two waves per SIMD.
 enum MoMode { kMoDensity = 0, kMoXc = 1, kMoSpins = 2 };
 
-// One pass of a wave over the functions with NT orbital tiles t0 .. t0 + NT - 1
-// of the nt0 + nt1 of both spins; row[a]: this lane's point in matrix a.
+// One pass of a wave over the functions with NT tiles of 16 orbitals, t0 .. t0 +
+// NT - 1 of the n0 + n1 orbitals of both spins in a row (a tile may hold both);
+// row[a]: this lane's point in matrix a.
 template <int NARR, int NT, int NS>
 __device__ __forceinline__ void mo_pass(int nbf, const double *const (&row)[NARR], int t0,
-                                        int nt0, int n0, int n1, const double *__restrict__ C0,
+                                        int n0, int n1, const double *__restrict__ C0,
                                         const double *__restrict__ C1,
                                         const double *__restrict__ f0,
                                         const double *__restrict__ f1, int l16, int q, int wv,
@@ -94,10 +96,10 @@ __device__ __forceinline__ void mo_pass(int nbf, const double *const (&row)[NARR
   const double *cp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const bool s1 = NS == 2 && t0 + t >= nt0;  // uniform
-    const int n = s1 ? n1 : n0;
-    const int col = 16 * (s1 ? t0 + t - nt0 : t0 + t) + l16;
-    cp[t] = (s1 ? C1 : C0) + (int64_t)(col < n ? col : n - 1) * nbf + 4 * q;
+    const int n = NS == 2 ? n0 + n1 : n0;
+    const int col = min(16 * (t0 + t) + l16, n - 1);
+    const bool s1 = NS == 2 && col >= n0;
+    cp[t] = (s1 ? C1 : C0) + (int64_t)(s1 ? col - n0 : col) * nbf + 4 * q;
   }
   v4d acc[NT][NARR];
 #pragma unroll
@@ -147,9 +149,8 @@ __device__ __forceinline__ void mo_pass(int nbf, const double *const (&row)[NARR
     for (int k = 0; k < 4 * NARR; ++k) v[k] = 0.0;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int col = 16 * (t0 + t - (s ? nt0 : 0)) + l16;
-      const bool own = NS == 1 || (t0 + t >= nt0) == (s == 1);  // uniform
-      if (own && col < (s ? n1 : n0)) {
+      const int c0 = 16 * (t0 + t) - (s ? n0 : 0), col = c0 + l16;  // of the spin
+      if (c0 > -16 && col >= 0 && col < (s ? n1 : n0)) {
         const double f = s ? f1[col] : f0[col];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -190,14 +191,14 @@ __global__ void __launch_bounds__(256, MAXT == 1 ? 3 : 2) density_mo(
   const double *row[NARR];
 #pragma unroll
   for (int a = 0; a < NARR; ++a) row[a] = in.a[a] + off;
-  const int nt0 = (n0 + 15) / 16, nt = nt0 + (NS == 2 ? (n1 + 15) / 16 : 0);
+  const int nt = ((NS == 2 ? n0 + n1 : n0) + 15) / 16;
   // sums over the orbitals; a slot belongs to one wave until the barrier
   __shared__ double red[NS][NARR][MP];
 #pragma unroll
   for (int k = 0; k < NS * NARR; ++k)
     if (q == 0) (&red[0][0][0])[k * MP + 16 * wv + l16] = 0.0;
 #define NKX_PASS(NT, T0) \
-  mo_pass<NARR, NT, NS>(nbf, row, T0, nt0, n0, n1, C0, C1, f0, f1, l16, q, wv, red)
+  mo_pass<NARR, NT, NS>(nbf, row, T0, n0, n1, C0, C1, f0, f1, l16, q, wv, red)
   if constexpr (MAXT == 1) {
     if (nt) NKX_PASS(1, 0);
   } else {
@@ -557,13 +558,14 @@ void launch_density_mo(hipStream_t s, int nbf, int64_t npts, const RefGrads &in,
                        const double *w, double *coef, double *epart) {
   const int64_t nwg = (npts + MP - 1) / MP;
   NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "too many points");
-  // one tile of orbitals (at most 16, one spin): three waves per SIMD instead
-  // of two, as the loads are what bounds it
+  // one tile of orbitals (at most 16 in all): three waves per SIMD instead of
+  // two, as the loads are what bounds it (open-shell water 136 us per call with
+  // the form for four tiles, 129)
 #define NKX_MO(MAXT)                                                                        \
   hipLaunchKernelGGL((density_mo<NARR, MAXT, MODE>), dim3((unsigned)nwg), dim3(256), 0, s,  \
                      nbf, npts, in, m0.nocc, m1.nocc, m0.C, m1.C, m0.f, m1.f, out, xl, w,   \
                      coef, epart)
-  if (MODE != kMoSpins && m0.nocc <= 16) NKX_MO(1);
+  if (m0.nocc + (MODE == kMoSpins ? m1.nocc : 0) <= 16) NKX_MO(1);
   else NKX_MO(4);
 #undef NKX_MO
   NKX_HIP_CHECK(hipGetLastError());

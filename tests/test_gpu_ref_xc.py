@@ -101,3 +101,28 @@ def test_open_shell(ctx, nbf, n, nocc):
         for s, V in enumerate((res.potential_alpha, res.potential_beta)):
             b = [2 * vs[:, 2 * s] * x + vs[:, 1] * y for x, y in zip(gr[s], gr[1 - s])] if gga else []
             _near(V, _v(m, w, vr[:, s], b))
+
+
+@pytest.mark.parametrize("na,nb", [(1, 15), (8, 8), (16, 1), (5, 12), (21, 20), (33, 31), (30, 35),
+                                   (2, 62)])
+def test_spins_sharing_a_tile_of_orbitals(ctx, na, nb):
+    """Alpha and beta orbitals in one row of tiles of 16: the border inside a
+    tile, at its edges, in a later pass."""
+    m, d, _, _, w, _, _ = _data(70, 300, 5, 3)
+    rng = np.random.default_rng(100 * na + nb)
+    C = [rng.normal(size=(70, k)) / 70 ** 0.5 for k in (na, nb)]
+    f = [rng.uniform(0.2, 1.0, k) for k in (na, nb)]
+    psi = [[c.T @ x for x in m] for c in C]
+    rho = [(k[:, None] * p[0] ** 2).sum(0) for k, p in zip(f, psi)]
+    gr = [[2 * (k[:, None] * p[0] * q).sum(0) for q in p[1:]] for k, p in zip(f, psi)]
+    t = lambda a: torch.tensor(a, device="cuda")
+    sg = [sum(x * y for x, y in zip(gr[i], gr[j])) for i, j in ((0, 0), (0, 1), (1, 1))]
+    e, vr, vs = [x.cpu().numpy() for x in
+                 api.functional_eval_polarized(ctx, (101, 130), t(np.stack(rho, 1)),
+                                               t(np.stack(sg, 1)))]
+    res = api.compute_gga_lsda(ctx, *d, t(w), C[0], f[0], C[1], f[1], (101, 130))
+    E = (w * (rho[0] + rho[1]) * e).sum()
+    assert abs(res.energy - E) <= 1e-11 * abs(E)
+    for s, V in enumerate((res.potential_alpha, res.potential_beta)):
+        _near(V, _v(m, w, vr[:, s], [2 * vs[:, 2 * s] * x + vs[:, 1] * y
+                                     for x, y in zip(gr[s], gr[1 - s])]))
