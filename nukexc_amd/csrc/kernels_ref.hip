@@ -59,9 +59,9 @@ struct RhoOut {
 // tiles on.  A thread per point with a scalar loop over orbitals and
 // functions reads each matrix once per orbital, uncoalesced: 41.6 ms per spin
 // on benzene (120 functions, 259 200 points, 21 and 20 orbitals), 288 us on
-// water (25 functions, 64 800 points, 5 orbitals); this form takes 340 us for
-// both spins (2.9 TB/s; 364 us with tiles of each spin's own, four instead of
-// three) and 24 us.
+// water (25 functions, 64 800 points, 5 orbitals); this form takes 328 us for
+// both spins (3.0 TB/s; 364 us with tiles of each spin's own, four instead of
+// three, and the last functions' loads under conditions) and 23 us.
 //
 // MODE 0 writes rho, grad rho and sigma of one spin; 1 evaluates the
 // functional and writes the Z coefficients (w v_rho / 2, 2 w v_sigma grad rho)
@@ -86,11 +86,13 @@ __device__ __forceinline__ void mo_pass(int nbf, const double *const (&row)[NARR
     const v4u t = *reinterpret_cast<const v4u *>(p + 16 * kk);
     return v4d{t[0], t[1], t[2], t[3]};
   };
+  // of the last, partial block; past the end the last function again, and zero
+  // for the orbitals (loads under a condition become branches, each with a wait
+  // for the loads before it)
   auto load_tail = [&](const double *p) -> v4d {
-    v4d t = {0.0, 0.0, 0.0, 0.0};
+    v4d t;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (16 * nfull + 4 * q + e < nbf) t[e] = p[16 * nfull + e];
+    for (int e = 0; e < 4; ++e) t[e] = p[min(16 * nfull + e, nbf - 1 - 4 * q)];
     return t;
   };
   const double *cp[NT];
@@ -136,9 +138,14 @@ __device__ __forceinline__ void mo_pass(int nbf, const double *const (&row)[NARR
   }
   if (16 * nfull < nbf) {
 #pragma unroll
+    for (int a = 0; a < NARR; ++a) A[a] = load_tail(row[a]);
+#pragma unroll
     for (int t = 0; t < NT; ++t) B[t] = load_tail(cp[t]);
 #pragma unroll
-    for (int a = 0; a < NARR; ++a) A[a] = load_tail(row[a]);
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (16 * nfull + 4 * q + e >= nbf) B[t][e] = 0.0;
     products(A, B);
   }
   // f psi psi_a summed over the pass's orbitals, spin by spin
@@ -312,8 +319,8 @@ __global__ void __launch_bounds__(64) xc_pol_ref(int64_t npts, int gga, XcList x
 // Bound by reading the four matrices up to about 64 functions, by the FP64
 // MFMA rate above.  With Z as a matrix of its own and a VALU kernel with
 // atomics this took 318 + 772 us per spin on benzene and 81 + 247 us on water;
-// now 450 us for both spins (38 TFLOP/s; 510 us with every wave forming Z after
-// its products) and 15 us (3.5 TB/s).
+// now 405 us for both spins (42 TFLOP/s; 450 us with the loads under conditions
+// and 510 with every wave forming Z after its products too) and 11.5 us (4.5 TB/s).
 template <int TM>
 struct ZvShape {
   static constexpr int threads = TM == 128 ? 512 : 256;
@@ -343,18 +350,25 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
   const int64_t k0 = (int64_t)split * kchunk;
   const int64_t k1 = k0 + kchunk < npts ? k0 + kchunk : npts;
   const int c = threadIdx.x % TM, r0 = threadIdx.x / TM;
-  const bool diag = m0 == n0, okm = m0 + c < nbf, okn = n0 + c < nbf;
+  const bool diag = m0 == n0;
+  // functions and points past the end repeat the last one: those functions are
+  // not written out, those points have zero coefficients.  (Loads under a
+  // condition become branches, each with a wait for the loads before it.)
+  const int cm = min(m0 + c, nbf - 1), cz = min(n0 + c, nbf - 1);
 
   double xa[4], xz[NARR][4];  // a stage's elements of this thread, rows r0 + RPT u
   auto load = [&](int64_t kb) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int64_t g = kb + r0 + RPT * u;
-      const int64_t e = g * nbf + c;
-      const bool in_k = g < k1;
+      const int64_t e = min(kb + r0 + RPT * u, k1 - 1) * nbf;
 #pragma unroll
-      for (int a = 0; a < NARR; ++a) xz[a][u] = in_k && okn ? in.a[a][e + n0] : 0.0;
-      xa[u] = diag ? xz[0][u] : (in_k && okm ? in.a[0][e + m0] : 0.0);
+      for (int a = 0; a < NARR; ++a) xz[a][u] = in.a[a][e + cz];
+      if (diag) xa[u] = xz[0][u];  // uniform
+    }
+    if (!diag) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        xa[u] = in.a[0][min(kb + r0 + RPT * u, k1 - 1) * nbf + cm];
     }
   };
   auto load_coef = [&](int64_t kb) -> double {
@@ -392,6 +406,7 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
   const int ni = min(NI, max(0, ((nbf - m0 + 15) / 16 - wr + S::WR - 1) / S::WR));
   const int nj = min(NJ, max(0, ((nbf - n0 + 15) / 16 - wc + S::WC - 1) / S::WC));
   const int nst = k1 > k0 ? (int)((k1 - k0 + KP - 1) / KP) : 0;
+  double cn = 0.0;  // this thread's coefficient of the stage after the next
   if (nst) {
     store_coef(0, load_coef(k0));
     store_coef(1, load_coef(k0 + KP));
@@ -399,6 +414,7 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
     __syncthreads();
     store(0, 0);
     if (nst > 1) load(k0 + KP);
+    cn = load_coef(k0 + 2 * KP);
     __syncthreads();
   }
   // Waves w and w + 4 share a SIMD: one forms Z before its products, the other
@@ -407,38 +423,41 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
   int ring = 1;  // of stage s + 1
   for (int s = 0; s < nst; ++s) {
     const bool more = s + 1 < nst;
-    const double cn = more ? load_coef(k0 + (int64_t)(s + 2) * KP) : 0.0;
     const int b = s & 1;
-    // the next stage into the other buffer, and the loads of the one after
+    const int ring2 = ring == 2 ? 0 : ring + 1;
+    // the next stage into the other buffer, the coefficients of the one after,
+    // and then the loads (nothing after them waits before the next stage)
     auto next = [&]() {
       if (!more) return;
       store(b ^ 1, ring);
+      store_coef(ring2, cn);
       if (s + 2 < nst) load(k0 + (int64_t)(s + 2) * KP);
+      cn = load_coef(k0 + (int64_t)(s + 3) * KP);
     };
     if (first) next();
+    {
 #pragma unroll
-    for (int ks = 0; ks < KP; ks += 4) {
-      double av[NI], zv[NS][NJ];
+      for (int ks = 0; ks < KP; ks += 4) {
+        double av[NI], zv[NS][NJ];
 #pragma unroll
-      for (int i = 0; i < NI; ++i) av[i] = As[b][ks + q][16 * (wr + S::WR * i) + l16];
+        for (int i = 0; i < NI; ++i) av[i] = As[b][ks + q][16 * (wr + S::WR * i) + l16];
 #pragma unroll
-      for (int sp = 0; sp < NS; ++sp)
+        for (int sp = 0; sp < NS; ++sp)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) zv[sp][j] = Zs[b][sp][ks + q][16 * (wc + S::WC * j) + l16];
+          for (int j = 0; j < NJ; ++j) zv[sp][j] = Zs[b][sp][ks + q][16 * (wc + S::WC * j) + l16];
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          if (i < ni && j < nj) {  // uniform
+          for (int j = 0; j < NJ; ++j)
+            if (i < ni && j < nj) {  // uniform
 #pragma unroll
-            for (int sp = 0; sp < NS; ++sp)
-              acc[sp][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i], zv[sp][j],
-                                                                   acc[sp][i][j], 0, 0, 0);
-          }
+              for (int sp = 0; sp < NS; ++sp)
+                acc[sp][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i], zv[sp][j],
+                                                                     acc[sp][i][j], 0, 0, 0);
+            }
+      }
     }
     if (!first) next();
-    const int ring2 = ring == 2 ? 0 : ring + 1;
-    if (more) store_coef(ring2, cn);
     ring = ring2;
     __syncthreads();
   }
