@@ -271,13 +271,15 @@ __global__ void __launch_bounds__(256) z_slots_f64(
               fma(k[s][3], gr[2], fma(k[s][2], gr[1], fma(k[s][1], gr[0], k[s][0] * v)));
     }
   } else {
+    double v[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const double v = phi[i * PT];
+    for (int i = 0; i < 16; ++i) v[i] = phi[i * PT];
 #pragma unroll
-      for (int s = 0; s < 2; ++s)
-        if (s < nspin) zt[s * TILE + i * PT] = k[s][0] * v;
-    }
+    for (int s = 0; s < 2; ++s)
+      if (s < nspin) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) zt[s * TILE + i * PT] = k[s][0] * v[i];
+      }
   }
 }
 
