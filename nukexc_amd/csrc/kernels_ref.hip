@@ -609,13 +609,13 @@ void launch_zv(hipStream_t s, int nbf, int64_t npts, int64_t kchunk, int nsplit,
 
 // Splits of the points of the V contraction: about one workgroup per CU for
 // tiles of 128 (one fits at a time), two for the smaller ones, each with at
-// least 64 points.
+// least 64 points.  Without points one split of none, which leaves Vbar zero.
 int ref_splits(int nbf, int64_t npts, int64_t *kchunk) {
   const int tm = nbf <= 32 ? 32 : (nbf <= 64 ? 64 : 128);
   const int64_t nt = (nbf + tm - 1) / tm;
   const int64_t want = std::max<int64_t>(1, (tm == 128 ? 256 : 512) / (nt * nt));
   const int64_t ns = std::max<int64_t>(1, std::min<int64_t>(want, npts / 64));
-  *kchunk = ((npts + ns - 1) / ns + 31) / 32 * 32;
+  *kchunk = std::max<int64_t>(32, ((npts + ns - 1) / ns + 31) / 32 * 32);
   return (int)std::max<int64_t>(1, (npts + *kchunk - 1) / *kchunk);
 }
 
