@@ -696,7 +696,7 @@ void xc_from_collocation(Ctx &c, int nbf, int64_t npts, const double *phi, const
                          const double *gy, const double *gz, const double *w, int nocc,
                          const double *C, const double *f, const XcList &xl, bool gga,
                          double *E, double *V) {
-  const MoSpin mo{nocc, C, f};
+  const MoSpin mo{std::max(nocc, 0), C, f};  // a negative count: no orbitals
   xc_ref<1>(c, nbf, npts, RefGrads{{phi, gx, gy, gz}}, gga && gx, w, mo, mo, xl, E, V, V);
 }
 
