@@ -168,6 +168,8 @@ struct MolTab {
 // screening options change.  A plan holds one molecule (the ctx grid and
 // basis) or a molecule set.
 struct Plan {
+  uint64_t builds = 0;        // constructions begun: a captured build holds this plan's
+                              // buffers, offsets and counts as they were at one of them
   uint64_t grid_version = ~0ull, basis_version = ~0ull;
   double screen_tol = -1;
   int pt = 0;                 // points per batch
@@ -295,7 +297,7 @@ struct GraphState {
   int nmol = 1;
   int nspin = 1;                // 2: an open-shell capture (one molecule)
   bool molset = false;          // captured on the molecule-set plan
-  uint64_t mplan_version = 0;
+  uint64_t plan_builds = 0;     // that plan's count at the capture
   std::vector<double *> vtab_h;
   DevBuf<double *> vtab;
   Workspace ws;
@@ -327,7 +329,6 @@ struct Ctx {
   uint64_t basis_version = 0;
   Plan plan;
   Plan mplan;                    // plan of the molecule set (nkx_molset_create)
-  uint64_t mplan_version = 0;    // bumped by every nkx_molset_create
   PlanScratch plan_ws;
   Workspace ws;
   GraphState graph;

@@ -163,9 +163,10 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
   hipStream_t s = c.stream;
   PlanScratch &sc = c.plan_ws;
   const int nmol = (int)mols.size();
-  pl.nmol = 0;  // until the plan is whole
   std::vector<PlanPart> parts;
   for (int m = 0; m < nmol; ++m) parts.push_back(make_part(mols[m].npts, *bases[m], tol));
+  ++pl.builds;  // from here on what a captured build holds of the plan is gone
+  pl.nmol = 0;  // until the plan is whole
   pl.mol_nbf_h.resize(nmol);
   pl.mol_ld_h.resize(nmol);
   pl.mol_nfb_h.resize(nmol);
@@ -382,7 +383,6 @@ void build_molset_plan(Ctx &c, const std::vector<MolPoints> &mols,
   for (const BasisHost &x : bases) b.push_back(&x);
   build_plan(c, c.mplan, mols, b, c.opt.screen_tol);
   c.mplan.screen_tol = c.opt.screen_tol;
-  ++c.mplan_version;
 }
 
 namespace {
@@ -788,6 +788,7 @@ void graph_capture(Ctx &c, int nspin, const double *const *P, const XcList &xl, 
   capture_on_plan(c, c.plan, nspin, P, xl, gga, precision, V);
   GraphState &gs = c.graph;
   gs.molset = false;
+  gs.plan_builds = c.plan.builds;
   gs.grid_version = c.grid.version;
   gs.basis_version = c.basis_version;
   gs.screen_tol = c.opt.screen_tol;
@@ -799,7 +800,7 @@ void molset_graph_capture(Ctx &c, const double *const *P, const XcList &xl, bool
   capture_on_plan(c, c.mplan, 1, P, xl, gga, precision, V);
   GraphState &gs = c.graph;
   gs.molset = true;
-  gs.mplan_version = c.mplan_version;
+  gs.plan_builds = c.mplan.builds;
   gs.screen_tol = c.mplan.screen_tol;
 }
 
@@ -809,11 +810,13 @@ void graph_launch(Ctx &c, double *E, double *N) {
   GraphState &gs = c.graph;
   NKX_REQUIRE(gs.exec, NKX_ERR_STATE, "no captured build: call nkx_graph_capture");
   if (gs.molset)
-    NKX_REQUIRE(gs.mplan_version == c.mplan_version, NKX_ERR_STATE,
+    NKX_REQUIRE(gs.plan_builds == c.mplan.builds, NKX_ERR_STATE,
                 "the molecule set changed since the capture");
   else
+    // the count too: the settings may be those of the capture again and the plan
+    // one of others made in between
     NKX_REQUIRE(gs.grid_version == c.grid.version && gs.basis_version == c.basis_version &&
-                    gs.screen_tol == c.opt.screen_tol,
+                    gs.screen_tol == c.opt.screen_tol && gs.plan_builds == c.plan.builds,
                 NKX_ERR_STATE, "grid, basis or screening changed since the capture");
   NKX_HIP_CHECK(hipGraphLaunch(gs.exec, c.stream));
   NKX_HIP_CHECK(hipStreamSynchronize(c.stream));
