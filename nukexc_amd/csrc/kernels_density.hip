@@ -3,6 +3,7 @@
 // per-batch functional between them is the one of the int8 form.
 #include <algorithm>
 
+#include "lane_sums.hpp"
 #include "nkx_internal.hpp"
 #include "sto_run.hpp"
 #include "vxc_kernels.hpp"
@@ -21,13 +22,6 @@ constexpr int STG = KS * PT;    // doubles of a stage
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima)
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-// LDS accesses of one wave stay in order across it
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // ---------------------------------------------------------------------------
 // X = P Phi for one pair of a batch's live blocks and, per block, the column

@@ -160,8 +160,10 @@ __global__ void __launch_bounds__(256, 2) grad_basis_f64(
           Xs[(4 * r + q) * GR_LD + 16 * j + l16] = accX[g][j][2 * h + r];
           Ws[(4 * r + q) * GR_LD + 16 * j + l16] = accW[g][j][2 * h + r];
         }
+      wave_fence();
       grad_rows<8>(gf, 8 * h, T, pt, gga, Xs, Ws, lane,
                    cpart + (im - s0) * GC + 3 * (row0 + 16 * g + 8 * h), tp);
+      wave_fence();
     }
   }
 #pragma unroll

@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(256, 2) grad_basis_i8(
           Xs[(16 * wv + 4 * q + r) * GR_LD + 16 * j + l16] = X[j][r];
           Ws[(16 * wv + 4 * q + r) * GR_LD + 16 * j + l16] = W[j][r];
         }
-      // (the rows of a wave are the functions that it takes: no barrier)
+      wave_fence();  // the rows of a wave are the functions that it takes: no barrier
       const GradPoint pt{pts[0][lane], pts[1][lane], pts[2][lane],
                          pts[3][lane], pts[4][lane], pts[5][lane]};
       grad_rows<16>(gf, 0, T, pt, gga, Xs + 16 * wv * GR_LD, Ws + 16 * wv * GR_LD, lane,

@@ -204,6 +204,7 @@ __global__ void __launch_bounds__(256, MAXT == 1 ? 3 : 2) density_mo(
 #pragma unroll
   for (int k = 0; k < NS * NARR; ++k)
     if (q == 0) (&red[0][0][0])[k * MP + 16 * wv + l16] = 0.0;
+  wave_fence();
 #define NKX_PASS(NT, T0) \
   mo_pass<NARR, NT, NS>(nbf, row, T0, n0, n1, C0, C1, f0, f1, l16, q, wv, red)
   if constexpr (MAXT == 1) {

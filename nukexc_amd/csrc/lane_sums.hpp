@@ -1,9 +1,20 @@
-// Sums of several values over the lanes of a wave with few exchanges.
+// Exchanges between the lanes of a wave: sums of several values with few moves,
+// and the order of LDS accesses.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 namespace nkx {
+
+// LDS accesses of one wave stay in order across it: needed between the writes of
+// some lanes and the reads of others, which the compiler takes for unrelated
+// where the addresses of one lane differ.  Costs no instruction (a wave's LDS
+// accesses are carried out in order).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // Sum of each of 16 values over the 16 lanes of a row; lane l of the row
 // returns the total of value bitrev4(l).  Fifteen exchanges: each halves the
