@@ -377,8 +377,15 @@ void launch_collocation_ref(hipStream_t s, int nbf, const FuncRec *f, const Harm
                             int64_t npts, const double *pts, double *phi, double *gx,
                             double *gy, double *gz) {
   if (nbf <= 0 || npts <= 0) return;
+  const int64_t step = max_workgroups(256) * 64;  // points of a launch
+  if (npts > step) {
+    auto at = [&](double *p) { return p ? p + step * nbf : p; };
+    launch_collocation_ref(s, nbf, f, t, step, pts, phi, gx, gy, gz);
+    launch_collocation_ref(s, nbf, f, t, npts - step, pts + 3 * step, at(phi), at(gx), at(gy),
+                           at(gz));
+    return;
+  }
   const int64_t nwg = (npts + 63) / 64;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "too many points");
   // Small outputs: narrow tiles (FW 4, 2 below one workgroup per CU), each a
   // workgroup of its own, for shorter chains and more waves in flight; the lines
   // that two tiles share meet in the last-level cache (256 MB, shared with what

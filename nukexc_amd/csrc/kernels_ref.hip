@@ -508,14 +508,16 @@ __global__ void __launch_bounds__(ZvShape<TM>::threads) zv_ref(
 // for small bases: 9.5 us for 25 functions and 507 splits; tiles of 16 x 16
 // summed with their mirror images in one workgroup (37 us) leave three CUs to
 // issue all the loads.
-__global__ void __launch_bounds__(512) finish_ref(int64_t n, int nsplit, int nwv,
+__global__ void __launch_bounds__(512) finish_ref(int64_t n, int nsplit, unsigned nwv,
                                                   const double *__restrict__ part,
                                                   double *__restrict__ V0,
                                                   double *__restrict__ V1, int64_t ne,
                                                   const double *__restrict__ epart,
                                                   double *__restrict__ E) {
   __shared__ double sh[512];
-  if ((int)blockIdx.x >= nwv) {
+  const unsigned wg = blockIdx.y * gridDim.x + blockIdx.x;
+  if (wg >= nwv) {
+    if (wg > nwv) return;
     double e = 0.0;
     for (int64_t i = threadIdx.x; i < ne; i += 512) e += epart[i];
     sh[threadIdx.x] = e;
@@ -527,8 +529,8 @@ __global__ void __launch_bounds__(512) finish_ref(int64_t n, int nsplit, int nwv
     if (threadIdx.x == 0) *E = sh[0];
     return;
   }
-  const int per = (int)((n + 63) / 64), sp = blockIdx.x / per;
-  const int64_t i = (int64_t)(blockIdx.x % per) * 64 + (threadIdx.x & 63);
+  const unsigned per = (unsigned)((n + 63) / 64), sp = wg / per;
+  const int64_t i = (int64_t)(wg % per) * 64 + (threadIdx.x & 63);
   const int wv = threadIdx.x >> 6;
   double v = 0.0;
   if (i < n) {
@@ -576,19 +578,25 @@ template <int NARR, int MODE>
 void launch_density_mo(hipStream_t s, int nbf, int64_t npts, const RefGrads &in,
                        const MoSpin &m0, const MoSpin &m1, const RhoOut &out, const XcList &xl,
                        const double *w, double *coef, double *epart) {
-  const int64_t nwg = (npts + MP - 1) / MP;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "too many points");
   // one tile of orbitals (at most 16 in all): three waves per SIMD instead of
   // two, as the loads are what bounds it (open-shell water 136 us per call with
   // the form for four tiles, 129)
 #define NKX_MO(MAXT)                                                                        \
   hipLaunchKernelGGL((density_mo<NARR, MAXT, MODE>), dim3((unsigned)nwg), dim3(256), 0, s,  \
-                     nbf, npts, in, m0.nocc, m1.nocc, m0.C, m1.C, m0.f, m1.f, out, xl, w,   \
-                     coef, epart)
-  if (m0.nocc + (MODE == kMoSpins ? m1.nocc : 0) <= 16) NKX_MO(1);
-  else NKX_MO(4);
+                     nbf, n, x, m0.nocc, m1.nocc, m0.C, m1.C, m0.f, m1.f, o, xl, at(w, g),  \
+                     at(coef, (MODE == kMoSpins ? 8 : 4) * g), at(epart, g / MP))
+  auto at = [](auto *p, int64_t i) { return p ? p + i : p; };
+  const int64_t step = max_workgroups(256) * MP;  // points of a launch
+  for (int64_t g = 0; g < npts; g += step) {
+    const int64_t n = std::min(step, npts - g), nwg = (n + MP - 1) / MP;
+    RefGrads x;
+    for (int a = 0; a < 4; ++a) x.a[a] = at(in.a[a], g * nbf);
+    const RhoOut o{at(out.rho, g), at(out.gx, g), at(out.gy, g), at(out.gz, g), at(out.sigma, g)};
+    if (m0.nocc + (MODE == kMoSpins ? m1.nocc : 0) <= 16) NKX_MO(1);
+    else NKX_MO(4);
+    NKX_HIP_CHECK(hipGetLastError());
+  }
 #undef NKX_MO
-  NKX_HIP_CHECK(hipGetLastError());
 }
 
 template <int NARR, int NS>
@@ -597,7 +605,7 @@ void launch_zv(hipStream_t s, int nbf, int64_t npts, int64_t kchunk, int nsplit,
   const int tm = nbf <= 32 ? 32 : (nbf <= 64 ? 64 : 128);
   const int64_t nt = (nbf + tm - 1) / tm;
   const int64_t nwg = nt * nt * nsplit;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "V contraction grid too large");
+  NKX_REQUIRE(nwg <= max_workgroups(512), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
 #define NKX_ZV(TM)                                                                            \
   hipLaunchKernelGGL((zv_ref<TM, NARR, NS>), dim3((unsigned)nwg), dim3(ZvShape<TM>::threads), 0, \
                      s, nbf, npts, kchunk, nsplit, in, coef, part)
@@ -641,6 +649,7 @@ void xc_ref(Ctx &c, int nbf, int64_t npts, const RefGrads &in, bool grad, const 
     else
       launch_density_mo<1, mode>(s, nbf, npts, in, m0, m1, none, xl, w, coef, ep);
     if (NS == 2) {
+      NKX_REQUIRE(ne <= max_workgroups(MP), NKX_ERR_UNSUPPORTED, "too many points");
       hipLaunchKernelGGL(xc_pol_ref, dim3((unsigned)ne), dim3(MP), 0, s, npts, grad ? 1 : 0, xl,
                          w, coef, ep);
       NKX_HIP_CHECK(hipGetLastError());
@@ -654,11 +663,12 @@ void xc_ref(Ctx &c, int nbf, int64_t npts, const RefGrads &in, bool grad, const 
   const bool mirror = nbf > 64;
   const int64_t n = (int64_t)nbf * nbf, nwv = NS * ((n + 63) / 64);
   NKX_REQUIRE(nwv + 1 < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "too many functions");
-  hipLaunchKernelGGL(finish_ref, dim3((unsigned)nwv + 1), dim3(512), 0, s, n, nsplit, (int)nwv,
+  hipLaunchKernelGGL(finish_ref, grid_2d(nwv + 1, 512), dim3(512), 0, s, n, nsplit, (unsigned)nwv,
                      part, mirror ? vb : V0, mirror ? vb + n : V1, ne, ep, Ed);
   NKX_HIP_CHECK(hipGetLastError());
   if (mirror) {
     const int64_t nt = (nbf + 31) / 32;
+    NKX_REQUIRE(NS * nt * nt <= max_workgroups(256), NKX_ERR_UNSUPPORTED, "too many functions");
     hipLaunchKernelGGL(mirror_ref, dim3((unsigned)(NS * nt * nt)), dim3(256), 0, s, nbf, n, vb,
                        V0, V1);
     NKX_HIP_CHECK(hipGetLastError());

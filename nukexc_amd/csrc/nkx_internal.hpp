@@ -115,6 +115,18 @@ struct DevView {
   T *p = nullptr;
 };
 
+// Workgroups of `threads` that a launch takes in one dimension: work items are
+// counted in 32 bits, and more of them run as many as the remainder says, without
+// an error.  Launches beyond it are cut into several, or use two dimensions.
+constexpr int64_t max_workgroups(int threads) { return (((int64_t)1 << 32) - 1) / threads; }
+
+// nwg workgroups in two dimensions where one is too few; the kernel's index is
+// blockIdx.y * gridDim.x + blockIdx.x, and those from nwg on do nothing.
+inline dim3 grid_2d(int64_t nwg, int threads) {
+  const int64_t y = (nwg + max_workgroups(threads) - 1) / max_workgroups(threads);
+  return dim3((unsigned)((nwg + y - 1) / y), (unsigned)y);
+}
+
 // STO basis on the device, one record per function.
 struct BasisHost {
   int nbf = 0;
