@@ -288,14 +288,15 @@ void vk_density(hipStream_t s, int nspin, int group, int64_t b0, int64_t b1, int
   const int g0 = group == 66 ? 2 : (group >= 65 ? 1 : group);  // the int8 form's codes
   const int g = g0 == 1 || g0 == 2 ? g0 : 4;
   const int nmg = (pl.max_mol_nfb + 1) / 2;
-  const int64_t ng = ((b1 - b0 + g - 1) / g + 7) / 8 * 8;
-  const int64_t nwg = ng * nmg * nspin;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "density grid too large");
-  hipLaunchKernelGGL(gga ? density_fused_f64<true> : density_fused_f64<false>, dim3((unsigned)nwg),
-                     dim3(256), 0, s, pl.tab(), pl.P_total, nspin, g, Pt, pl.b_off.p, pl.b_fbl.p,
-                     s0, b0, b1, nmg, narr, pl.funcs.p, pl.terms.p, pl.px.p, pl.py.p, pl.pz.p,
-                     tiles, pstride, part);
-  NKX_HIP_CHECK(hipGetLastError());
+  const int64_t step = max_workgroups(256) / (8 * nmg * nspin) * 8 * g;  // batches of a launch
+  for (int64_t b = b0; b < b1; b += step) {
+    const int64_t be = std::min(b + step, b1), ng = ((be - b + g - 1) / g + 7) / 8 * 8;
+    hipLaunchKernelGGL(gga ? density_fused_f64<true> : density_fused_f64<false>,
+                       dim3((unsigned)(ng * nmg * nspin)), dim3(256), 0, s, pl.tab(), pl.P_total,
+                       nspin, g, Pt, pl.b_off.p, pl.b_fbl.p, s0, b, be, nmg, narr, pl.funcs.p,
+                       pl.terms.p, pl.px.p, pl.py.p, pl.pz.p, tiles, pstride, part);
+    NKX_HIP_CHECK(hipGetLastError());
+  }
 }
 
 void vk_z_slots(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr, int nspin,

@@ -496,12 +496,14 @@ void vkg_basis(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
                const double *coef, bool accum, double *cpart, double *tpart, double *tpt) {
   if (b1 <= b0) return;
   const int nmg = (pl.max_mol_nfb + 1) / 2;
-  const int64_t nwg = (b1 - b0 + 7) / 8 * 8 * nmg;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "gradient grid too large");
-  hipLaunchKernelGGL(grad_basis_f64, dim3((unsigned)nwg), dim3(256), 0, s, pl.tab(), Pt, pl.b_off.p,
-                     pl.b_fbl.p, s0, b0, b1, nmg, narr, yarr, gga, tiles, coef, pl.funcs.p,
-                     pl.terms.p, pl.px.p, pl.py.p, pl.pz.p, cpart, tpart);
-  NKX_HIP_CHECK(hipGetLastError());
+  const int64_t step = max_workgroups(256) / (8 * nmg) * 8;  // batches of a launch
+  for (int64_t b = b0; b < b1; b += step) {
+    const int64_t be = std::min(b + step, b1), nwg = (be - b + 7) / 8 * 8 * nmg;
+    hipLaunchKernelGGL(grad_basis_f64, dim3((unsigned)nwg), dim3(256), 0, s, pl.tab(), Pt,
+                       pl.b_off.p, pl.b_fbl.p, s0, b, be, nmg, narr, yarr, gga, tiles, coef,
+                       pl.funcs.p, pl.terms.p, pl.px.p, pl.py.p, pl.pz.p, cpart, tpart);
+    NKX_HIP_CHECK(hipGetLastError());
+  }
   hipLaunchKernelGGL(grad_points_kernel, dim3((unsigned)(b1 - b0)), dim3(192), 0, s, s0, b0,
                      pl.b_off.p, tpart, accum ? 1 : 0, tpt);
   NKX_HIP_CHECK(hipGetLastError());

@@ -400,13 +400,13 @@ __global__ void __launch_bounds__(256) finish_kernel(
     VArgs va, double *const *__restrict__ Vmol, const double *__restrict__ en,
     double *__restrict__ enout) {
   __shared__ double sv[3][256];
-  const int64_t nv = (int64_t)npairs * nz * FB;
-  if ((int64_t)blockIdx.x >= nv) {
-    en_reduce(mt, (int)(blockIdx.x - nv), en, enout, sv);
+  const unsigned wg = blockIdx.y * gridDim.x + blockIdx.x, nv = (unsigned)npairs * nz * FB;
+  if (wg >= nv) {
+    if (en && (int)(wg - nv) < nmol) en_reduce(mt, (int)(wg - nv), en, enout, sv);
     return;
   }
-  const int mu = blockIdx.x & (FB - 1);
-  const int p = (int)(blockIdx.x / FB) % npairs, zs = (int)(blockIdx.x / FB) / npairs;
+  const int mu = wg & (FB - 1);
+  const int p = (int)(wg / FB) % npairs, zs = (int)(wg / FB) / npairs;
   const int I = pair_I[p], J = pair_J[p];
   const int mol = mt.blk_mol[I];
   const int nbf = mol_nbf[mol];
@@ -449,15 +449,16 @@ __global__ void __launch_bounds__(256) fill0_kernel(int64_t n, double *__restric
 __global__ void __launch_bounds__(256) gather_p_f64(GatherArgs a, int tr) {
   const GatherP g = a.g[blockIdx.y];
   const int nbf = g.nbf, nbf_pad = g.nfb * FB;
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)nbf_pad * nbf_pad) return;
-  const int i = (int)(e / nbf_pad), j = (int)(e % nbf_pad);
-  double v = 0.0;
-  if (i < nbf && j < nbf) {
-    const int fi = g.fperm[i], fj = g.fperm[j];
-    v = g.P[tr ? (int64_t)fj * nbf + fi : (int64_t)fi * nbf + fj];
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < (int64_t)nbf_pad * nbf_pad;
+       e += (int64_t)gridDim.x * 256) {
+    const int i = (int)(e / nbf_pad), j = (int)(e % nbf_pad);
+    double v = 0.0;
+    if (i < nbf && j < nbf) {
+      const int fi = g.fperm[i], fj = g.fperm[j];
+      v = g.P[tr ? (int64_t)fj * nbf + fi : (int64_t)fi * nbf + fj];
+    }
+    static_cast<double *>(g.out)[e] = v;
   }
-  static_cast<double *>(g.out)[e] = v;
 }
 
 // Z = (w/2) Phi for the overlap build (S = Phi W Phi^T through vgemm).
@@ -481,8 +482,10 @@ void vk_gather_p(hipStream_t s, const std::vector<GatherP> &g, bool transpose) {
       a.g[i] = g[k + i];
       e = std::max(e, (int64_t)FB * a.g[i].nfb * FB * a.g[i].nfb);
     }
-    hipLaunchKernelGGL(gather_p_f64, dim3((unsigned)((e + 255) / 256), (unsigned)n), dim3(256), 0,
-                       s, a, transpose ? 1 : 0);
+    // (1024 blocks need one workgroup more than a launch takes)
+    const int64_t nwg = std::min((e + 255) / 256, max_workgroups(256));
+    hipLaunchKernelGGL(gather_p_f64, dim3((unsigned)nwg, (unsigned)n), dim3(256), 0, s, a,
+                       transpose ? 1 : 0);
     NKX_HIP_CHECK(hipGetLastError());
   }
 }
@@ -508,7 +511,7 @@ void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
               int narr, int nz, bool first, const double *tiles, double *vpart) {
   if (b1 <= b0 || pl.nspairs == 0) return;
   const int64_t nwg = (int64_t)pl.nspairs * ((nsplit + 7) / 8 * 8) * nz;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "V contraction grid too large");
+  NKX_REQUIRE(nwg <= max_workgroups(512), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
   hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)nwg), dim3(512), 0, s, pl.nspairs, nsplit,
                      reinterpret_cast<const int4 *>(pl.sp_blk.p),
                      reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.npairs, pl.tile_slot.p,
@@ -524,7 +527,7 @@ void vk_finish(hipStream_t s, const Plan &pl, int nsplit, int nz, const double *
   NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "reduction grid too large");
   VArgs va{};
   if (!Vmol_dev) std::copy(V, V + (size_t)nz * pl.nmol, va.p);
-  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)nwg), dim3(256), 0, s, pl.npairs, nsplit, nz,
+  hipLaunchKernelGGL(finish_kernel, grid_2d(nwg, 256), dim3(256), 0, s, pl.npairs, nsplit, nz,
                      pl.pair_I.p, pl.pair_J.p, pl.fperm_d.p, pl.tab(), pl.nmol, pl.mol_nbf.p,
                      vpart, va, Vmol_dev, en, enout);
   NKX_HIP_CHECK(hipGetLastError());

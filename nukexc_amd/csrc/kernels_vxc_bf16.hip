@@ -454,12 +454,14 @@ void vkb_density(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, c
 void vkb_vgemm(hipStream_t s, int nprod, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
                int nsplit, int gga, bool first, const uint16_t *store, double *vpart) {
   if (b1 <= b0 || pl.npairs == 0) return;
+  const int64_t nwg = (int64_t)pl.npairs * nsplit;
+  NKX_REQUIRE(nwg <= max_workgroups(256), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
   if (nprod == 3)
-    hipLaunchKernelGGL(vgemm_mixed<3>, dim3((unsigned)(pl.npairs * nsplit)), dim3(256), 0, s,
+    hipLaunchKernelGGL(vgemm_mixed<3>, dim3((unsigned)nwg), dim3(256), 0, s,
                        pl.npairs, nsplit, pl.pair_I.p, pl.pair_J.p, pl.tile_slot.p, pl.nb, b0,
                        b1, s0, gga, first ? 1 : 0, store, vpart);
   else
-    hipLaunchKernelGGL(vgemm_mixed<6>, dim3((unsigned)(pl.npairs * nsplit)), dim3(256), 0, s,
+    hipLaunchKernelGGL(vgemm_mixed<6>, dim3((unsigned)nwg), dim3(256), 0, s,
                        pl.npairs, nsplit, pl.pair_I.p, pl.pair_J.p, pl.tile_slot.p, pl.nb, b0,
                        b1, s0, gga, first ? 1 : 0, store, vpart);
   NKX_HIP_CHECK(hipGetLastError());

@@ -1108,15 +1108,15 @@ template <int GBT>
 static void launch_density_x2_i8(hipStream_t s, int64_t b0, int64_t b1, int64_t s0,
                                  const Plan &pl, const signed char *Ps, int gga,
                                  const signed char *store, double *part) {
-  const int64_t ngroups = (b1 - b0 + GBT - 1) / GBT;
-  const int64_t ngq = (ngroups + 7) / 8;
   const int umax = std::min(pl.nfb, GBT * pl.max_mol_nfb);
   const int nmg = (umax + 1) / 2;
-  const int64_t nwg = ngq * 8 * nmg;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "density grid too large");
-  hipLaunchKernelGGL((density_x2_i8<GBT, false>), dim3((unsigned)nwg), dim3(256), 0, s,
-                     pl.tab(), pl.nfb, Ps, pl.b_off.p, pl.b_fbl.p, s0, b0, b1, nmg, 0, 0, gga,
-                     store, part);
+  const int64_t step = max_workgroups(256) / (8 * nmg) * 8 * GBT;  // batches of a launch
+  for (int64_t b = b0; b < b1; b += step) {
+    const int64_t be = std::min(b + step, b1), ngroups = (be - b + GBT - 1) / GBT;
+    hipLaunchKernelGGL((density_x2_i8<GBT, false>), dim3((unsigned)((ngroups + 7) / 8 * 8 * nmg)),
+                       dim3(256), 0, s, pl.tab(), pl.nfb, Ps, pl.b_off.p, pl.b_fbl.p, s0, b, be,
+                       nmg, 0, 0, gga, store, part);
+  }
 }
 
 // absolute block pairs in XCD tiles of tpn pairs x tbn batches
@@ -1124,12 +1124,16 @@ static void launch_density_x2a_i8(hipStream_t s, int64_t b0, int64_t b1, int64_t
                                   const Plan &pl, const signed char *Ps, int gga,
                                   const signed char *store, double *part, int tpn, int tbn) {
   const int npair = (pl.max_mol_nfb + 1) / 2;
-  const int64_t ntiles = (int64_t)((npair + tpn - 1) / tpn) * ((b1 - b0 + tbn - 1) / tbn);
-  const int64_t nwg = (ntiles + 7) / 8 * 8 * tpn * tbn;
-  NKX_REQUIRE(nwg < (int64_t)1 << 31, NKX_ERR_UNSUPPORTED, "density grid too large");
-  hipLaunchKernelGGL((density_x2_i8<1, true>), dim3((unsigned)nwg), dim3(256), 0, s, pl.tab(),
-                     pl.nfb, Ps, pl.b_off.p, pl.b_fbl.p, s0, b0, b1, npair, tpn, tbn, gga,
-                     store, part);
+  const int64_t row = (int64_t)((npair + tpn - 1) / tpn) * tpn;  // pairs, whole tiles
+  // batches of a launch, whole tiles (up to seven tiles come on top)
+  const int64_t step = (max_workgroups(256) - 7 * tpn * tbn) / row / tbn * tbn;
+  for (int64_t b = b0; b < b1; b += step) {
+    const int64_t be = std::min(b + step, b1), ntiles = row / tpn * ((be - b + tbn - 1) / tbn);
+    const int64_t nwg = (ntiles + 7) / 8 * 8 * tpn * tbn;
+    hipLaunchKernelGGL((density_x2_i8<1, true>), dim3((unsigned)nwg), dim3(256), 0, s, pl.tab(),
+                       pl.nfb, Ps, pl.b_off.p, pl.b_fbl.p, s0, b, be, npair, tpn, tbn, gga,
+                       store, part);
+  }
 }
 
 // shape: 65 / 66 one / two batches per workgroup, 71 / 72 one batch per
@@ -1216,8 +1220,9 @@ void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
   // all super-pairs of a split on one XCD where they fit its 32 CUs twice at
   // most: 32 waters (28 super-pairs) 19.1 -> 17.8 ms; 100 waters (210) lose by it
   const bool grouped = pl.nspairs <= 64;
-  const int64_t ns = grouped ? (nsplit + 7) / 8 * 8 : nsplit;
-  hipLaunchKernelGGL(vgemm_i8, dim3((unsigned)(pl.nspairs * ns)), dim3(512), 0, s, pl.nspairs,
+  const int64_t ns = grouped ? (nsplit + 7) / 8 * 8 : nsplit, nwg = pl.nspairs * ns;
+  NKX_REQUIRE(nwg <= max_workgroups(512), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
+  hipLaunchKernelGGL(vgemm_i8, dim3((unsigned)nwg), dim3(512), 0, s, pl.nspairs,
                      nsplit, grouped ? 1 : 0, reinterpret_cast<const int4 *>(pl.sp_blk.p),
                      reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.npairs, pl.tile_slot.p,
                      pl.tab(), b0, b1, s0, gga, store, zbase, zstride, first ? 1 : 0,

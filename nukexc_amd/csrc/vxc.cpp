@@ -431,8 +431,9 @@ void for_each_chunk(const Plan &pl, int64_t max_slots, F &&fn) {
   int64_t b0 = 0;
   while (b0 < pl.nb) {
     int64_t b1 = b0 + 1;
-    // grow while the slot range fits (at least one batch per chunk)
-    int64_t lo = b0 + 1, hi = pl.nb;
+    // grow while the slot range fits (at least one batch per chunk, and a
+    // workgroup of 256 per batch in one launch)
+    int64_t lo = b0 + 1, hi = std::min(pl.nb, b0 + max_workgroups(256));
     while (lo < hi) {
       const int64_t mid = (lo + hi + 1) / 2;
       if (pl.b_off_h[mid] - pl.b_off_h[b0] <= max_slots) lo = mid;
