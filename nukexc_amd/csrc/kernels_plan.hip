@@ -141,7 +141,8 @@ __device__ __forceinline__ bool reaches(const double *box, const double *fn, int
 }
 
 // One wave per batch: live[b * nfb + f], the number of live blocks and of
-// functions in them.
+// functions in them, of pairs of blocks (2a, 2a + 1) with a live one, and whether
+// the last block of an odd number is live.
 __global__ void __launch_bounds__(NT) plan_screen(int64_t nb, int nbf, int nfb,
                                                   const double *__restrict__ boxes,
                                                   const double *__restrict__ fn,
@@ -151,16 +152,19 @@ __global__ void __launch_bounds__(NT) plan_screen(int64_t nb, int nbf, int nfb,
   if (b >= nb) return;
   double box[6];
   for (int k = 0; k < 6; ++k) box[k] = boxes[6 * b + k];
-  int nblk = 0, nfun = 0;
+  int nblk = 0, nfun = 0, ntwo = 0;
+  bool even = false;  // of the even block before
   for (int f = 0; f < nfb; ++f) {
     const bool hit = reaches(box, fn, nbf, f);
+    if (f & 1) ntwo += hit || even;
+    else even = hit;
     if (hit) {
       ++nblk;
       nfun += min(nbf, (f + 1) * FB) - f * FB;
     }
     if ((threadIdx.x & 63) == 0) live[b * nfb + f] = hit ? 1 : 0;
   }
-  if ((threadIdx.x & 63) == 0) count[b] = make_int2(nblk, nfun);
+  if ((threadIdx.x & 63) == 0) count[b] = make_int2(plan_count(nblk, ntwo, (nfb & 1) && even), nfun);
 }
 
 // One wave per batch: its live blocks in ascending order from slot b_off[b],

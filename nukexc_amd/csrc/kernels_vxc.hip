@@ -92,6 +92,13 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
 // with each stage's slots looked up in LDS between its barrier and its copies).  One workgroup per
 // block pair, both products on the diagonal too, read four tiles for every two
 // products of them (58 GB on 16 waters): 9.9 ms, 737 us and 245 us.
+//
+// Where screening leaves few super-pairs whole (long chains, centres far apart) a
+// unit is a single pair (sp_blk NULL), two waves to 16 rows, each with half of a
+// stage's products: the work of a super-pair, 2.65 pairs, is the same with one
+// live tile as with four.  build_plan counts both.  A chain of 700 atoms (7000
+// functions, 21 of 110 blocks live in a batch) takes 247 ms and by super-pairs
+// 279, one of 240 atoms 76 and 85; 100 waters (34 of 40) 237 and 176.
 constexpr int VS = 16;             // points of a stage
 constexpr int VSEC = FB * VS;      // doubles of one block's stage
 
@@ -102,8 +109,9 @@ __device__ __forceinline__ v4d ld4(const double *p) { return *reinterpret_cast<c
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 __global__ void __launch_bounds__(512) vgemm_f64(
-    int nsp, int nsplit, const int4 *__restrict__ sp_blk, const int4 *__restrict__ sp_pidx,
-    int npairs, const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1, int64_t s0,
+    int nsp, int nsplit, int grouped, const int4 *__restrict__ sp_blk,
+    const int4 *__restrict__ sp_pidx, const int *__restrict__ pair_I,
+    const int *__restrict__ pair_J, int npairs, const int *__restrict__ tile_slot, MolTab mt, int64_t b0, int64_t b1, int64_t s0,
     int narr, int zbase, int first, const double *__restrict__ tiles,
     double *__restrict__ vpart) {
   // Z_J0, Z_J1, Phi_J0, Phi_J1 of a stage; two buffers, declared apart so that
@@ -112,21 +120,24 @@ __global__ void __launch_bounds__(512) vgemm_f64(
   __shared__ __attribute__((aligned(16))) double bufB[4][VSEC];
   __shared__ int ls[4][512];  // slots of I_0, I_1, J_0, J_1 per listed batch
   __shared__ int wcnt[8];
-  // workgroups are dealt to the eight XCDs in turn: the super-pairs of a split
-  // run on one XCD and share its L2 for the batches' tiles
-  const int xcd = blockIdx.x & 7, rr = blockIdx.x >> 3, nsg = (nsplit + 7) / 8;
-  const int sp = rr % nsp, split = (rr / nsp) % nsg * 8 + xcd, zs = rr / (nsp * nsg);
-  if (split >= nsplit) return;
+  // grouped: workgroups are dealt to the eight XCDs in turn, and the super-pairs of
+  // a split run on one XCD and share its L2 for the batches' tiles; else splits
+  // one after the other
+  const int xcd = grouped ? blockIdx.x & 7 : 0, rr = grouped ? blockIdx.x >> 3 : blockIdx.x;
+  const int nsg = grouped ? nsplit / 8 : nsplit;
+  const int sp = rr % nsp, split = (rr / nsp) % nsg * (grouped ? 8 : 1) + xcd,
+            zs = rr / (nsp * nsg);
   const int64_t zoff = (int64_t)(zbase + zs) * TILE;
   vpart += (int64_t)zs * nsplit * npairs * (FB * FB);
-  const int4 blk = sp_blk[sp], pix = sp_pidx[sp];
+  const int4 blk = sp_blk ? sp_blk[sp] : make_int4(pair_I[sp], -1, pair_J[sp], -1);
+  const int4 pix = sp_blk ? sp_pidx[sp] : make_int4(sp, -1, -1, -1);
   const bool diag = blk.x == blk.z;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, q = lane >> 4;
   // this wave's tile (wa, wb), rows row0 .. of I_wa, one or two groups of 16;
   // half: the half of a stage's products it forms (-1: all)
   const bool two = blk.w >= 0;           // two J blocks (then two I blocks)
-  const bool one = !two && blk.y < 0;    // one block in all
+  const bool one = !two && blk.y < 0;    // one block each side
   const int wa = one ? 0 : wv >> 2, wb = two ? wv & 1 : 0;
   const int row0 = two ? 32 * ((wv >> 1) & 1) : 16 * (wv & 3);
   const int half = one ? wv >> 2 : -1;
@@ -263,31 +274,31 @@ __global__ void __launch_bounds__(512) vgemm_f64(
     }
   }
 
-  if (diag) {
-    // through LDS, tile by tile: with one block the second halves' sums, then
-    // V(a, b) = Vbar(a, b) + Vbar(b, a)^T for (0, 0), (0, 1), (1, 1)
-    double(*t)[FB + 1] = reinterpret_cast<double(*)[FB + 1]>(&bufA[0][0]);
-    static_assert(sizeof(bufA) >= 32 * (FB + 1) * sizeof(double), "half a tile in a buffer");
-    const int ng = two ? 2 : 1;
-    if (one) {
+  double(*t)[FB + 1] = reinterpret_cast<double(*)[FB + 1]>(&bufA[0][0]);
+  static_assert(sizeof(bufA) >= 32 * (FB + 1) * sizeof(double), "half a tile in a buffer");
+  if (one) {  // the second halves' sums through LDS, 32 rows at a time
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {  // 32 rows at a time
-        __syncthreads();
-        if (half == 1 && (row0 >> 5) == h) {
+    for (int h = 0; h < 2; ++h) {
+      __syncthreads();
+      if (half == 1 && (row0 >> 5) == h) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) t[(row0 & 31) + 4 * r + q][16 * j + l16] = acc[0][j][r];
-        }
-        __syncthreads();
-        if (half == 0 && (row0 >> 5) == h) {
+          for (int r = 0; r < 4; ++r) t[(row0 & 31) + 4 * r + q][16 * j + l16] = acc[0][j][r];
+      }
+      __syncthreads();
+      if (half == 0 && (row0 >> 5) == h) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[0][j][r] += t[(row0 & 31) + 4 * r + q][16 * j + l16];
-        }
+          for (int r = 0; r < 4; ++r) acc[0][j][r] += t[(row0 & 31) + 4 * r + q][16 * j + l16];
       }
     }
+  }
+  if (diag) {
+    // through LDS, tile by tile:
+    // V(a, b) = Vbar(a, b) + Vbar(b, a)^T for (0, 0), (0, 1), (1, 1)
+    const int ng = two ? 2 : 1;
     const int ntile = two ? 3 : (one ? 1 : 2);
     for (int k = 0; k < ntile; ++k) {
       // target tile (ta, tb), from tile (tb, ta)
@@ -510,12 +521,16 @@ void vk_zoverlap(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr
 void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
               int narr, int nz, bool first, const double *tiles, double *vpart) {
   if (b1 <= b0 || pl.nspairs == 0) return;
-  const int64_t nwg = (int64_t)pl.nspairs * ((nsplit + 7) / 8 * 8) * nz;
+  const int nsp = pl.v_by_pair ? pl.npairs : pl.nspairs;
+  const int64_t nwg = (int64_t)nsp * nsplit * nz;
   NKX_REQUIRE(nwg <= max_workgroups(512), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
-  hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)nwg), dim3(512), 0, s, pl.nspairs, nsplit,
-                     reinterpret_cast<const int4 *>(pl.sp_blk.p),
-                     reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.npairs, pl.tile_slot.p,
-                     pl.tab(), b0, b1, s0, narr, narr - nz, first ? 1 : 0, tiles, vpart);
+  // other numbers of splits leave XCDs with fewer of them than others, or none
+  const int grouped = nsplit % 8 == 0;
+  hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)nwg), dim3(512), 0, s, nsp, nsplit, grouped,
+                     reinterpret_cast<const int4 *>(pl.v_by_pair ? nullptr : pl.sp_blk.p),
+                     reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.pair_I.p, pl.pair_J.p,
+                     pl.npairs, pl.tile_slot.p, pl.tab(), b0, b1, s0, narr, narr - nz,
+                     first ? 1 : 0, tiles, vpart);
   NKX_HIP_CHECK(hipGetLastError());
 }
 

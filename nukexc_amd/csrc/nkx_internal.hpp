@@ -203,10 +203,11 @@ struct Plan {
   bool pairs_full = false;        // every block pair of every molecule is kept
   std::vector<int> pair_I_h, pair_J_h;
   DevView<int> pair_I, pair_J;
-  // 2 x 2 super-pairs of blocks (one molecule) for the int8 V contraction:
+  // 2 x 2 super-pairs of blocks (one molecule) for the V contractions:
   // 4 ints each, blocks I0 I1 J0 J1 (-1: none) and the pair indices of the
   // tiles (I0,J0) (I0,J1) (I1,J0) (I1,J1) (-1: not a kept pair, or redundant)
   int nspairs = 0;
+  bool v_by_pair = false;         // FP64 V contraction by pairs, not super-pairs (vgemm_f64)
   int max_mol_nfb = 0;            // largest function-block count of one molecule
   DevView<int> sp_blk, sp_pidx;
   DevBuf<int> tile_slot;          // per molecule [block][batch] -> slot in the tile store or -1

@@ -212,6 +212,8 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
   sc.live.reserve(ts);
   sc.count.reserve(2 * nb);
   sc.pairs.reserve(pairs);
+  for (int m = 0; m < nmol; ++m)
+    NKX_REQUIRE(parts[m].nfb <= 0xffff, NKX_ERR_UNSUPPORTED, "more than 65535 function blocks");
   std::vector<double *> fn(nmol);
   TablePack fpack;
   for (int m = 0; m < nmol; ++m) fpack.add(fn[m], parts[m].fn.data(), parts[m].fn.size());
@@ -233,11 +235,14 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
   pl.b_off_h.resize(nb + 1);
   int64_t nslots = 0;
   double nb2g = 0, nbg = 0;
+  int64_t by_pair = 0, by_super = 0;
   for (int m = 0; m < nmol; ++m)
     for (int64_t b = 0; b < parts[m].nb; ++b) {
       const int64_t gb = pl.mol_b0_h[m] + b;
       pl.b_off_h[gb] = (int)nslots;
-      nslots += host[2 * gb];
+      const unsigned cnt = (unsigned)host[2 * gb];
+      const int64_t n = cnt & 0xffff, f = cnt >> 17, last = (cnt >> 16) & 1;
+      nslots += n;
       NKX_REQUIRE(nslots < (int64_t)INT32_MAX, NKX_ERR_UNSUPPORTED,
                   "too many live (block, batch) pairs for 32-bit slot numbers");
       // algorithmic work: true functions of the live blocks, true points
@@ -245,6 +250,11 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
       const double g = (double)std::min<int64_t>(PT, parts[m].npts - b * PT);
       nb2g += nfun * nfun * g;
       nbg += nfun * g;
+      // the FP64 V contraction's work in 1/200 of a pair of blocks: by pairs (on
+      // the diagonal 0.55), or by super-pairs (2.65, on the diagonal 1.5, beside an
+      // odd last block 1.7), whole where one block of each side is live
+      by_pair += n * (100 * (n - 1) + 110);
+      by_super += f * (265 * (f - 1) + 300) + last * (340 * f + 110);
     }
   pl.b_off_h[nb] = (int)nslots;
   pl.b_off.upload(pl.b_off_h.data(), pl.b_off_h.size(), s);
@@ -329,6 +339,7 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
   pl.npairs = (int)pl.pair_I_h.size();
   pl.pairs_full = pl.npairs == all_pairs;
   pl.nspairs = (int)(spb.size() / 4);
+  pl.v_by_pair = by_pair < by_super;
   pl.max_mol_nfb = 0;
   for (int m = 0; m < nmol; ++m) pl.max_mol_nfb = std::max(pl.max_mol_nfb, parts[m].nfb);
   pl.work_nb2g = nb2g;
@@ -401,26 +412,39 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
 }
 
 // Split count of the V contraction over batches, or the tuned value.  One
-// workgroup of a super-pair tile (bf16: of a pair) fits a CU at a time, so:
+// workgroup of a unit (super-pair; bf16, and FP64 where few super-pairs are whole:
+// pair) fits a CU at a time, so:
 //   one unit:  256 splits, one equal workgroup per CU (mixed benzene, 99 x 578
 //              points: 1536 us per build, 1617 with 320, 1608 with 335)
 //   a few:     512 splits each (16- and 24-atom molecules: within 1 % of the
 //              best of 32 .. 1024)
 //   many:      about 8192 workgroups (FP64: 4096), the tail of unequal units
 //              levelled by their number; every split costs a tile of partials
-//              per pair
+//              per pair.  By pairs 32768, as many partials as 8192 whole super-
+//              pairs have: a chain of 240 atoms takes 71.8 ms with 64 splits, 84.6
+//              with 8
 // and never less than four batches per split (mixed water: 146 us with 4 to 5,
 // 179 with 32), or in a molecule set 16 (FP64: 8) of an average molecule (8
-// molecules, mixed: 2782 us, 2893 with 4).
+// molecules, mixed: 2782 us, 2893 with 4).  FP64 with more workgroups than CUs: a
+// multiple of eight, which vgemm_f64 deals to the XCDs evenly, where its partials
+// stay below 1 GB (100 waters, 210 super-pairs: 176 ms with 24 splits, 179 with
+// 20; a chain of 700 atoms by super-pairs 279 ms with 8, 320 with 3).
 int choose_nsplit(const Plan &pl, int precision, int tuned = 0) {
   const bool f64 = precision == NKX_PREC_FP64;
-  const int64_t units = precision == NKX_PREC_MIXED_BF16 ? pl.npairs : pl.nspairs;
+  const bool by_pair = precision == NKX_PREC_MIXED_BF16 || (f64 && pl.v_by_pair);
+  const int64_t units = by_pair ? pl.npairs : pl.nspairs;
   if (units == 0) return 1;
   int64_t ns = tuned;
   if (tuned <= 0) {
     const int64_t per = pl.nmol > 1 ? (f64 ? 8 : 16) * (int64_t)pl.nmol : 4;
-    ns = std::min<int64_t>((f64 ? 4096 : 8192) / units + 1, units == 1 ? 256 : 512);
+    const int64_t target = !f64 ? 8192 : by_pair ? 32768 : 4096;
+    ns = std::min<int64_t>(target / units + 1, units == 1 ? 256 : 512);
     ns = std::min<int64_t>(ns, pl.nb / per);
+    if (f64 && units * ns > 256) {
+      const int64_t up = (ns + 7) / 8 * 8;
+      if (up * pl.npairs * FB * FB * (int64_t)sizeof(double) <= (int64_t)1 << 30) ns = up;
+      else if (ns > 8) ns = ns / 8 * 8;
+    }
   }
   ns = std::max<int64_t>(1, std::min<int64_t>(ns, pl.nb));
   return (int)ns;

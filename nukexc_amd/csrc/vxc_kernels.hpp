@@ -10,8 +10,14 @@ namespace nkx {
 void vk_plan_points(hipStream_t s, PlanScratch &sc, int64_t npts, const double *pts,
                     const double *w, double *px, double *py, double *pz, double *pw, int *pidx,
                     double *boxes);
-// live[batch][block] and per batch (live blocks, functions in them); fn:
-// centre and screening radius per sorted function
+// live[batch][block] and per batch (plan_count, functions in the live blocks); fn:
+// centre and screening radius per sorted function.  plan_count: the live blocks,
+// the pairs of blocks (2a, 2a + 1) with a live one, and whether the last block of
+// an odd number is live, of at most 65535 blocks in one word (the host reads two
+// words per batch that the device wrote: two more took 15 us of a geometry step).
+__host__ __device__ inline int plan_count(int blocks, int twos, bool last) {
+  return (int)((unsigned)twos << 17 | (unsigned)last << 16 | (unsigned)blocks);
+}
 void vk_plan_screen(hipStream_t s, int64_t nb, int nbf, int nfb, const double *boxes,
                     const double *fn, unsigned char *live, int *count);
 // slots of the molecule's batches b0 .. b0 + nb - 1 (b_off over all batches),
