@@ -155,6 +155,7 @@ __global__ void __launch_bounds__(512) vgemm_f64(
 #pragma unroll
   for (int u = 0; u < 4; ++u) tso[u] = bl[u] >= 0 ? (int64_t)mt.blk_local[bl[u]] * mnb : -1;
   const int64_t lo = b0 > mb0 ? b0 : mb0, hi = b1 < mb0 + mnb ? b1 : mb0 + mnb;
+  if (!first && lo + split >= hi) return;  // nothing to add
 
   struct AFrag {
     v4d f[2], z[2];  // rows of Phi_I, Z_I per row group

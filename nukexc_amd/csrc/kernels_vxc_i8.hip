@@ -1058,6 +1058,11 @@ __global__ void __launch_bounds__(512) vgemm_i8(
     split = rr / nsp * 8 + (blockIdx.x & 7);
   }
   const int4 blk = sp_blk[sp], pix = sp_pidx[sp];
+  if (!first) {  // a later chunk without batches of this split adds nothing
+    const int mol = mt.blk_mol[blk.x];
+    const int64_t mb0 = mt.b0[mol], mb1 = mb0 + mt.nb[mol];
+    if ((b0 > mb0 ? b0 : mb0) + split >= (b1 < mb1 ? b1 : mb1)) return;
+  }
 #define NKX_VTILE(NG, NJ)                                                                       \
   vgemm_i8_tile<NG, NJ>(blk, pix, split, nsplit, npairs, tile_slot, mt, b0, b1, s0, gga, store, \
                         zbase, zstride, first, vpart, bufA, bufB, ls, wcnt)

@@ -429,7 +429,18 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
 // multiple of eight, which vgemm_f64 deals to the XCDs evenly, where its partials
 // stay below 1 GB (100 waters, 210 super-pairs: 176 ms with 24 splits, 179 with
 // 20; a chain of 700 atoms by super-pairs 279 ms with 8, 320 with 3).
-int choose_nsplit(const Plan &pl, int precision, int tuned = 0) {
+//
+// In chunks (max_slots slots each), every split reads and writes its partials
+// again in each: as many workgroups per chunk as CUs (by pairs, a quarter of the
+// work and of the partials each, four times as many), or, where a chunk is long,
+// that times the root of its share of work (units times batches over 1743, from
+// 4.7 us per batch of a super-pair and 16 us for the partials of 256, and up to
+// three times that where few chunks hold all; a set's chunk holds a share of its
+// units).  V contraction, mixed, ms: 32 waters in chunks of 8 GB 16.8 with 96 to
+// 192 splits, 19.4 with 512, in two of 48 GB 17.4 with 203, 16.6 with 293; 24
+// waters in chunks of 64 MB 3.1 with 16, 49 with 512; 60 waters in chunks of 64 MB
+// 26 with 2 to 4, 230 with 106, of 1 GB 16 with 8 to 32, 25 with 106.
+int choose_nsplit(const Plan &pl, int precision, int64_t max_slots, int tuned = 0) {
   const bool f64 = precision == NKX_PREC_FP64;
   const bool by_pair = precision == NKX_PREC_MIXED_BF16 || (f64 && pl.v_by_pair);
   const int64_t units = by_pair ? pl.npairs : pl.nspairs;
@@ -440,9 +451,18 @@ int choose_nsplit(const Plan &pl, int precision, int tuned = 0) {
     const int64_t target = !f64 ? 8192 : by_pair ? 32768 : 4096;
     ns = std::min<int64_t>(target / units + 1, units == 1 ? 256 : 512);
     ns = std::min<int64_t>(ns, pl.nb / per);
+    if (max_slots < pl.nslots) {
+      const double share = (double)max_slots / pl.nslots;
+      const double u = pl.nmol > 1 ? std::max(1.0, units * share) : (double)units;
+      const double waves =
+          std::max(1.0, (1.0 + 2.0 * share) * std::sqrt(u * share * pl.nb / 1743.0));
+      ns = std::min<int64_t>(ns, (int64_t)((by_pair ? 1024.0 : 256.0) * waves / u));
+    }
     if (f64 && units * ns > 256) {
       const int64_t up = (ns + 7) / 8 * 8;
-      if (up * pl.npairs * FB * FB * (int64_t)sizeof(double) <= (int64_t)1 << 30) ns = up;
+      if (max_slots >= pl.nslots &&
+          up * pl.npairs * FB * FB * (int64_t)sizeof(double) <= (int64_t)1 << 30)
+        ns = up;
       else if (ns > 8) ns = ns / 8 * 8;
     }
   }
@@ -494,7 +514,6 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   b.gga = gga;
   const int nmol = pl.nmol;
   b.narr = 1 + nspin;  // Phi, Z per spin
-  b.nsplit = choose_nsplit(pl, precision, tuned_split);
   b.bf16 = precision == NKX_PREC_MIXED_BF16;
   b.mixed = precision == NKX_PREC_MIXED || b.bf16;
   NKX_REQUIRE(!b.bf16 || nspin == 1, NKX_ERR_UNSUPPORTED,
@@ -515,6 +534,7 @@ BuildSetup prepare_build(Workspace &ws, const Plan &pl, int nspin, bool gga, int
   for (int64_t bb = 0; bb < pl.nb; ++bb)
     max_slots = std::max<int64_t>(max_slots, pl.b_off_h[bb + 1] - pl.b_off_h[bb]);
   b.slots_alloc = std::min<int64_t>(max_slots, std::max<int64_t>(pl.nslots, 1));
+  b.nsplit = choose_nsplit(pl, precision, b.slots_alloc, tuned_split);
   if (b.mixed) {
     ws.mstore.reserve((size_t)b.slots_alloc * slot_bytes);
     if (!b.bf16 && nspin == 2)
@@ -672,9 +692,10 @@ namespace {
 // Times each candidate on plan pl (build() runs one build with the ctx
 // options): first the density shape, then the V split count; keeps the
 // fastest pair in the ctx options and returns its build time.
-double autotune_on(Ctx &c, const Plan &pl, int precision, const std::function<void()> &build,
+double autotune_on(Ctx &c, const Plan &pl, int precision, bool gga,
+                   const std::function<void()> &build,
                    int *best_split, int *best_group) {
-  const int base = choose_nsplit(pl, precision);
+  const int base = prepare_build(c.ws, pl, 1, gga, precision, 0, 0, c.opt.mem_budget).nsplit;
   std::vector<int> splits;
   for (int k : {base / 4, base / 2, base, 2 * base, 4 * base}) {
     const int v = std::max(1, std::min<int>(k, (int)std::max<int64_t>(pl.nb, 1)));
@@ -757,7 +778,7 @@ double autotune(Ctx &c, const double *P, const XcList &xl, bool gga, int precisi
   ensure_plan(c);
   double E, N;
   return autotune_on(
-      c, c.plan, precision, [&]() { vxc_build(c, P, xl, gga, precision, &E, &N, V); },
+      c, c.plan, precision, gga, [&]() { vxc_build(c, P, xl, gga, precision, &E, &N, V); },
       best_split, best_group);
 }
 
@@ -766,7 +787,7 @@ double molset_autotune(Ctx &c, const double *const *P, const XcList &xl, bool gg
   NKX_REQUIRE(c.mplan.nmol > 0, NKX_ERR_STATE, "no molecule set: call nkx_molset_create");
   std::vector<double> E(c.mplan.nmol), N(c.mplan.nmol);
   return autotune_on(
-      c, c.mplan, precision,
+      c, c.mplan, precision, gga,
       [&]() { build_on_plan(c, c.mplan, 1, P, xl, gga, precision, E.data(), N.data(), V); },
       best_split, best_group);
 }
@@ -1105,13 +1126,13 @@ void overlap_build(Ctx &c, double *S) {
   Workspace &ws = c.ws;
   hipStream_t s = c.stream;
   const int narr = 2;
-  const int nsplit = choose_nsplit(pl, NKX_PREC_FP64);
   int64_t max_slots =
       chunk_slot_budget((size_t)narr * FB * PT * sizeof(double), c.opt.mem_budget);
   for (int64_t b = 0; b < pl.nb; ++b)
     max_slots = std::max<int64_t>(max_slots, pl.b_off_h[b + 1] - pl.b_off_h[b]);
   const int64_t slots_alloc = std::min<int64_t>(max_slots, std::max<int64_t>(pl.nslots, 1));
   ws.tiles64.reserve((size_t)slots_alloc * narr * FB * PT);
+  const int nsplit = choose_nsplit(pl, NKX_PREC_FP64, slots_alloc);
   const size_t vsz = (size_t)nsplit * std::max(pl.npairs, 1) * FB * FB;
   ws.vpart.reserve(vsz);
   vk_fill0(s, S, (int64_t)pl.nbf * pl.nbf);
