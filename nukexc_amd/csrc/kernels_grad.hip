@@ -495,7 +495,7 @@ void vkg_basis(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
                const double *Pt, int narr, int yarr, int gga, const double *tiles,
                const double *coef, bool accum, double *cpart, double *tpart, double *tpt) {
   if (b1 <= b0) return;
-  const int nmg = (pl.max_mol_nfb + 1) / 2;
+  const int nmg = std::max(1, (pl.max_live + 1) / 2);  // of the fullest batch
   const int64_t step = max_workgroups(256) / (8 * nmg) * 8;  // batches of a launch
   for (int64_t b = b0; b < b1; b += step) {
     const int64_t be = std::min(b + step, b1), nwg = (be - b + 7) / 8 * 8 * nmg;

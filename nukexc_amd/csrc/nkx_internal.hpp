@@ -209,6 +209,7 @@ struct Plan {
   int nspairs = 0;
   bool v_by_pair = false;         // FP64 V contraction by pairs, not super-pairs (vgemm_f64)
   int max_mol_nfb = 0;            // largest function-block count of one molecule
+  int max_live = 0;               // most live blocks of a batch
   DevView<int> sp_blk, sp_pidx;
   DevBuf<int> tile_slot;          // per molecule [block][batch] -> slot in the tile store or -1
   int64_t nslots = 0;

@@ -235,7 +235,7 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
   pl.b_off_h.resize(nb + 1);
   int64_t nslots = 0;
   double nb2g = 0, nbg = 0;
-  int64_t by_pair = 0, by_super = 0;
+  int64_t by_pair = 0, by_super = 0, max_live = 0;
   for (int m = 0; m < nmol; ++m)
     for (int64_t b = 0; b < parts[m].nb; ++b) {
       const int64_t gb = pl.mol_b0_h[m] + b;
@@ -243,6 +243,7 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
       const unsigned cnt = (unsigned)host[2 * gb];
       const int64_t n = cnt & 0xffff, f = cnt >> 17, last = (cnt >> 16) & 1;
       nslots += n;
+      max_live = std::max(max_live, n);
       NKX_REQUIRE(nslots < (int64_t)INT32_MAX, NKX_ERR_UNSUPPORTED,
                   "too many live (block, batch) pairs for 32-bit slot numbers");
       // algorithmic work: true functions of the live blocks, true points
@@ -340,6 +341,7 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
   pl.pairs_full = pl.npairs == all_pairs;
   pl.nspairs = (int)(spb.size() / 4);
   pl.v_by_pair = by_pair < by_super;
+  pl.max_live = (int)max_live;
   pl.max_mol_nfb = 0;
   for (int m = 0; m < nmol; ++m) pl.max_mol_nfb = std::max(pl.max_mol_nfb, parts[m].nfb);
   pl.work_nb2g = nb2g;
