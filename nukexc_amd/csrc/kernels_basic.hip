@@ -386,15 +386,18 @@ void launch_collocation_ref(hipStream_t s, int nbf, const FuncRec *f, const Harm
     return;
   }
   const int64_t nwg = (npts + 63) / 64;
-  // Small outputs: narrow tiles (FW 4, 2 below one workgroup per CU), each a
-  // workgroup of its own, for shorter chains and more waves in flight; the lines
-  // that two tiles share meet in the last-level cache (256 MB, shared with what
-  // else is held).  Larger ones: those lines would go to memory twice, so one
-  // workgroup writes all tiles of its points, 32 functions wide.  Both calls
-  // (FW 8 in a loop / FW 4 each its own): 9 MB of output 72.3 / 69.6 us, 71 MB
-  // 96 / 83, 0.5 GB 269 / 308, 2.2 GB 799 / 1246; FW 2 at 4 MB 64.5 for 67.2.
+  // Small outputs, or few points: narrow tiles (FW 4, 2 below one workgroup per
+  // CU), each a workgroup of its own, for shorter chains and more waves in flight;
+  // the lines that two tiles share meet in the last-level cache (256 MB, shared
+  // with what else is held).  Larger ones: those lines would go to memory twice, so
+  // one workgroup writes all tiles of its points, 32 functions wide, where there
+  // are points for twelve workgroups a CU.  Both calls, us (FW 8 in a loop / FW 4
+  // each its own): 9 MB of output 72.3 / 69.6, 71 MB 96 / 83, 0.5 GB 269 / 308, 2.2
+  // GB 799 / 1246; the gradients of 3120 functions at 5 000 points 754 / 173, 1040
+  // at 40 000 377 / 264, 120 at 130 000 143 / 140, at 260 000 254 / 260, at 340 000
+  // 318 / 375; FW 2 at 4 MB 64.5 for 67.2.
   const int64_t bytes = (int64_t)8 * nbf * npts * ((phi ? 1 : 0) + (gx ? 3 : 0));
-  const int fw = bytes > ((int64_t)1 << 26) ? 8 : nwg < 256 ? 2 : 4;
+  const int fw = bytes <= ((int64_t)1 << 26) ? (nwg < 256 ? 2 : 4) : (nwg < 12 * 256 ? 4 : 8);
   const unsigned ny = fw == 8 ? 1 : (unsigned)((nbf + 4 * fw - 1) / (4 * fw));
 #define NKX_COLLOC_FW(V, G, W)                                                              \
   hipLaunchKernelGGL((colloc_ref_kernel<V, G, W>), dim3((unsigned)nwg, ny), dim3(256), 0, s, \
