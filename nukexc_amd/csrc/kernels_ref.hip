@@ -10,6 +10,7 @@
 //                split-K contraction Vbar = Phi Z^T on FP64 MFMA
 //   finish_ref   sum of the split partials, and E (mirror_ref: V = Vbar +
 //                Vbar^T where zv_ref did not form it)
+//   density_few  rho, grad rho, sigma of up to eight functions
 //
 // The four matrices are read twice per call (once per contraction) and nothing
 // of their size is written.
@@ -262,6 +263,50 @@ __global__ void __launch_bounds__(256, MAXT == 1 ? 3 : 2) density_mo(
     }
     for (int o = 32; o > 0; o >>= 1) e += __shfl_down(e, o);
     if (lane == 0) epart[blockIdx.x] = e;
+  }
+}
+
+// rho, grad rho and sigma of a basis of NB functions, a point per thread: the
+// point's rows are read once, into registers.  Taken to eight functions, where
+// density_mo spends more on a workgroup's set-up, exchange and barrier than on its
+// 64 points (with the gradient nine take 188 us in both, values gain up to twelve).
+// Two million points, call times in us, here and there: 1 function 25 and 75, with
+// the gradient 49 and 156; 3 functions 30 and 76, 68 and 162; 8 functions 41 and
+// 77, 140 and 195, with 40 orbitals 58 and 180, 151 and 501; 100 000 points 22 and
+// 26, 32 and 39.
+template <int NARR, int NB>
+__global__ void __launch_bounds__(256) density_few(int64_t npts, RefGrads in, int nocc,
+                                                   const double *__restrict__ C,
+                                                   const double *__restrict__ f, RhoOut out) {
+  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (g >= npts) return;
+  double x[NARR][NB], v[NARR];
+#pragma unroll
+  for (int a = 0; a < NARR; ++a) {
+    v[a] = 0.0;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) x[a][k] = in.a[a][g * NB + k];
+  }
+  for (int i = 0; i < nocc; ++i) {
+    double psi[NARR];
+#pragma unroll
+    for (int a = 0; a < NARR; ++a) {
+      psi[a] = 0.0;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) psi[a] = fma(C[i * NB + k], x[a][k], psi[a]);
+    }
+    const double fp = f[i] * psi[0];
+#pragma unroll
+    for (int a = 0; a < NARR; ++a) v[a] = fma(fp, psi[a], v[a]);
+  }
+  out.rho[g] = v[0];
+  if constexpr (NARR == 4) {
+    if (out.gx) {
+      out.gx[g] = 2.0 * v[1];
+      out.gy[g] = 2.0 * v[2];
+      out.gz[g] = 2.0 * v[3];
+    }
+    if (out.sigma) out.sigma[g] = 4.0 * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]);
   }
 }
 
@@ -599,6 +644,23 @@ void launch_density_mo(hipStream_t s, int nbf, int64_t npts, const RefGrads &in,
 #undef NKX_MO
 }
 
+// density_few where nbf is its NB; false: another size
+template <int NARR, int NB>
+bool launch_density_few(hipStream_t s, int nbf, int64_t npts, const RefGrads &in,
+                        const MoSpin &mo, const RhoOut &out) {
+  if constexpr (NB == 0) {
+    return false;
+  } else {
+    if (nbf != NB) return launch_density_few<NARR, NB - 1>(s, nbf, npts, in, mo, out);
+    const int64_t nwg = (npts + 255) / 256;
+    NKX_REQUIRE(nwg <= max_workgroups(256), NKX_ERR_UNSUPPORTED, "too many points");
+    hipLaunchKernelGGL((density_few<NARR, NB>), dim3((unsigned)nwg), dim3(256), 0, s, npts, in,
+                       mo.nocc, mo.C, mo.f, out);
+    NKX_HIP_CHECK(hipGetLastError());
+    return true;
+  }
+}
+
 template <int NARR, int NS>
 void launch_zv(hipStream_t s, int nbf, int64_t npts, int64_t kchunk, int nsplit,
                const RefGrads &in, const double *coef, double *part) {
@@ -688,6 +750,9 @@ void launch_density_ref(hipStream_t s, int nbf, int64_t npts, const double *phi,
   const MoSpin mo{nocc, C, f};
   const RhoOut out{rho, grx, gry, grz, sigma};
   const XcList none{};
+  if (gx ? launch_density_few<4, 8>(s, nbf, npts, in, mo, out)
+         : launch_density_few<1, 8>(s, nbf, npts, in, mo, out))
+    return;
   if (gx)
     launch_density_mo<4, kMoDensity>(s, nbf, npts, in, mo, mo, out, none, nullptr, nullptr, nullptr);
   else
