@@ -228,7 +228,9 @@ struct Plan {
   }
 };
 
-// Scratch of a plan's construction, kept by the ctx.
+// Scratch of a plan's construction, kept by the ctx up to kPlanScratchBytes (a plan
+// of about 4 M points) and given back after larger ones.
+constexpr size_t kPlanScratchBytes = (size_t)160 << 20;
 struct PlanScratch {
   DevBuf<double> part, boxes;      // box of the points; box per batch
   DevBuf<uint64_t> key;            // Morton codes, unsorted and sorted
@@ -237,6 +239,25 @@ struct PlanScratch {
   DevBuf<unsigned char> live;      // per molecule [batch][block]
   DevBuf<char> fn;                 // screening centres and radii
   PinBuf pin_fn, pin_tab, pin_cnt;
+  void trim() {
+    const size_t held = (part.n + boxes.n + key.n) * 8 + (idx.n + count.n + pairs.n) * 4 + tmp.n +
+                        live.n + fn.n;
+    if (held <= kPlanScratchBytes) return;
+    part.release();
+    boxes.release();
+    key.release();
+    idx.release();
+    count.release();
+    pairs.release();
+    tmp.release();
+    live.release();
+    fn.release();
+  }
+  // gives it back at the end of a scope, whichever way it ends
+  struct Scope {
+    PlanScratch &s;
+    ~Scope() { s.trim(); }
+  };
 };
 
 // Scratch of the grid build, kept between builds of up to kGridScratchPoints

@@ -162,6 +162,7 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
                 const std::vector<const BasisHost *> &bases, double tol) {
   hipStream_t s = c.stream;
   PlanScratch &sc = c.plan_ws;
+  PlanScratch::Scope scope{sc};
   const int nmol = (int)mols.size();
   std::vector<PlanPart> parts;
   for (int m = 0; m < nmol; ++m) parts.push_back(make_part(mols[m].npts, *bases[m], tol));
