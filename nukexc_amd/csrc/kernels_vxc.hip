@@ -97,8 +97,8 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
 // unit is a single pair (sp_blk NULL), two waves to 16 rows, each with half of a
 // stage's products: the work of a super-pair, 2.65 pairs, is the same with one
 // live tile as with four.  build_plan counts both.  A chain of 700 atoms (7000
-// functions, 21 of 110 blocks live in a batch) takes 247 ms and by super-pairs
-// 279, one of 240 atoms 76 and 85; 100 waters (34 of 40) 237 and 176.
+// functions, 21 of 110 blocks live in a batch) takes 231 ms and by super-pairs
+// 279, one of 240 atoms 71 and 85; 100 waters (34 of 40) 237 and 176.
 constexpr int VS = 16;             // points of a stage
 constexpr int VSEC = FB * VS;      // doubles of one block's stage
 

@@ -423,15 +423,16 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
 //              best of 32 .. 1024)
 //   many:      about 8192 workgroups (FP64: 4096), the tail of unequal units
 //              levelled by their number; every split costs a tile of partials
-//              per pair.  By pairs 32768, as many partials as 8192 whole super-
-//              pairs have: a chain of 240 atoms takes 71.8 ms with 64 splits, 84.6
-//              with 8
+//              per pair.  By pairs 65536, of which one takes a quarter of the
+//              partials: V of a chain of 240 atoms 71.4 ms with 128 splits, 73.5 with
+//              64, 86.5 with 8
 // and never less than four batches per split (mixed water: 146 us with 4 to 5,
 // 179 with 32), or in a molecule set 16 (FP64: 8) of an average molecule (8
 // molecules, mixed: 2782 us, 2893 with 4).  FP64 with more workgroups than CUs: a
 // multiple of eight, which vgemm_f64 deals to the XCDs evenly, where its partials
-// stay below 1 GB (100 waters, 210 super-pairs: 176 ms with 24 splits, 179 with
-// 20; a chain of 700 atoms by super-pairs 279 ms with 8, 320 with 3).
+// stay below 1 GB (by pairs 2 GB; 100 waters, 210 super-pairs: 176 ms with 24
+// splits, 179 with 20; a chain of 700 atoms by super-pairs 279 ms with 8, 320 with
+// 3, by pairs 235 with 8, 227 with 16).
 //
 // In chunks (max_slots slots each), every split reads and writes its partials
 // again in each: as many workgroups per chunk as CUs (by pairs, a quarter of the
@@ -451,7 +452,7 @@ int choose_nsplit(const Plan &pl, int precision, int64_t max_slots, int tuned = 
   int64_t ns = tuned;
   if (tuned <= 0) {
     const int64_t per = pl.nmol > 1 ? (f64 ? 8 : 16) * (int64_t)pl.nmol : 4;
-    const int64_t target = !f64 ? 8192 : by_pair ? 32768 : 4096;
+    const int64_t target = !f64 ? 8192 : by_pair ? 65536 : 4096;
     ns = std::min<int64_t>(target / units + 1, units == 1 ? 256 : 512);
     ns = std::min<int64_t>(ns, pl.nb / per);
     if (max_slots < pl.nslots) {
@@ -464,7 +465,7 @@ int choose_nsplit(const Plan &pl, int precision, int64_t max_slots, int tuned = 
     if (f64 && units * ns > 256) {
       const int64_t up = (ns + 7) / 8 * 8;
       if (max_slots >= pl.nslots &&
-          up * pl.npairs * FB * FB * (int64_t)sizeof(double) <= (int64_t)1 << 30)
+          up * pl.npairs * FB * FB * (int64_t)sizeof(double) <= (int64_t)(by_pair ? 2 : 1) << 30)
         ns = up;
       else if (ns > 8) ns = ns / 8 * 8;
     }
