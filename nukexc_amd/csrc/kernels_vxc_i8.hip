@@ -1223,8 +1223,10 @@ void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
   const signed char *zbase = zstore_b ? zstore_b : store + OFF_Z;
   const int64_t zstride = zstore_b ? (int64_t)SEC : slot_bytes_i8(gga);
   // all super-pairs of a split on one XCD where they fit its 32 CUs twice at
-  // most: 32 waters (28 super-pairs) 19.1 -> 17.8 ms; 100 waters (210) lose by it
-  const bool grouped = pl.nspairs <= 64;
+  // most: 32 waters (28 super-pairs) 19.1 -> 17.8 ms; 100 waters (210) lose by it;
+  // and only where every XCD gets its share (a chain of 100 atoms, 36 super-pairs,
+  // whole builds with 3 splits: 15.2 ms in plain order, 20.3 on three XCDs)
+  const bool grouped = pl.nspairs <= 64 && (nsplit % 8 == 0 || nsplit >= 64);
   const int64_t ns = grouped ? (nsplit + 7) / 8 * 8 : nsplit, nwg = pl.nspairs * ns;
   NKX_REQUIRE(nwg <= max_workgroups(512), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
   hipLaunchKernelGGL(vgemm_i8, dim3((unsigned)nwg), dim3(512), 0, s, pl.nspairs,
