@@ -1,25 +1,25 @@
 // Batched V_xc build on MI355X (gfx950), FP64 form.
 //
 // Data layout in HBM (one chunk of point batches at a time):
-//   tile store   [slot][array][64 functions][PT points], array = Phi, dPhi/dx,
-//                dPhi/dy, dPhi/dz, Z (GGA) or Phi, Z (LDA); spin-polarised
-//                builds carry Z_alpha, Z_beta in place of Z.  A slot is one
-//                (function block, point batch) pair that survived screening.
+//   tile store   [slot][array][64 functions][64 points], array = Phi, then Z (of
+//                each spin).  A slot is one (function block, point batch) pair
+//                that survived screening.  No gradient is stored: it is formed
+//                again where it is used.
 //   Pd           transpose of the permuted, zero-padded density matrix.
 //   vpart        split-K partial V tiles [split][pair][64][64].
 //
 // Kernels per chunk:
-//   colloc_tiles     Phi and grad Phi for every live slot (HBM-write bound).
-//   density_x        X = P Phi on MFMA over the batch's live function blocks and
-//                    the column sums of Phi X and grad Phi X
-//                    (kernels_density.hip); density_f: the functional per
-//                    batch; z_slots: Z = w (v_rho/2 Phi + 2 v_sigma grad rho .
-//                    grad Phi) written back to the tile store.
-//   vgemm            one workgroup per (2 x 2 super-pair of blocks, split):
-//                    acc += Phi_I Z_J^T + Z_I Phi_J^T over the batches where
-//                    both blocks are live (MFMA-bound).
-// and once per build: finish (split sum + un-permute + mirror, and the FP64
-// energy / electron-count sums).
+//   colloc_tiles_f64   Phi of every live slot.
+//   density_fused_f64  X = P Phi on MFMA over the batch's live function blocks
+//                      and the column sums of Phi X and grad Phi X, then density_f
+//                      (density_fp), the functional per batch, and z_slots_f64, Z =
+//                      w (v_rho / 2 Phi + 2 v_sigma grad rho . grad Phi) into the
+//                      tile store (kernels_density.hip, kernels_vxc_i8.hip).
+//   vgemm_f64          one workgroup per (2 x 2 super-pair of blocks, or pair;
+//                      split): V += Phi_I Z_J^T + Z_I Phi_J^T over the batches
+//                      where both blocks are live.
+// and once per build finish_kernel: split sum, un-permutation and mirror image, and
+// the energy and electron-count sums.
 #include <algorithm>
 
 #include "nkx_internal.hpp"
