@@ -7,6 +7,7 @@
 // (0.19 ms for the whole plan of 121 k points, 6.6 ms in host loops).
 #include <hipcub/hipcub.hpp>
 
+#include "morton.hpp"
 #include "nkx_internal.hpp"
 #include "vxc_kernels.hpp"
 
@@ -14,79 +15,9 @@ namespace nkx {
 
 namespace {
 
-constexpr int NT = 256;
+constexpr int NT = kBoxThreads;
 constexpr int PT = 64;
 constexpr int FB = 64;
-
-__device__ __forceinline__ uint64_t spread21(uint64_t v) {
-  v &= 0x1fffff;
-  v = (v | v << 32) & 0x1f00000000ffffull;
-  v = (v | v << 16) & 0x1f0000ff0000ffull;
-  v = (v | v << 8) & 0x100f00f00f00f00full;
-  v = (v | v << 4) & 0x10c30c30c30c30c3ull;
-  v = (v | v << 2) & 0x1249249249249249ull;
-  return v;
-}
-
-// Minimum and maximum of six values per thread over the workgroup (lo xyz, hi
-// xyz); thread k < 6 returns value k.
-__device__ __forceinline__ double box_reduce(double v[6], double (*s)[NT]) {
-  for (int k = 0; k < 6; ++k) s[k][threadIdx.x] = v[k];
-  __syncthreads();
-  for (int h = NT / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h)
-      for (int k = 0; k < 6; ++k) {
-        const double o = s[k][threadIdx.x + h];
-        s[k][threadIdx.x] = k < 3 ? fmin(s[k][threadIdx.x], o) : fmax(s[k][threadIdx.x], o);
-      }
-    __syncthreads();
-  }
-  return threadIdx.x < 6 ? s[threadIdx.x][0] : 0.0;
-}
-
-// box of the points, per workgroup
-__global__ void __launch_bounds__(NT) plan_bbox(int64_t n, const double *__restrict__ pts,
-                                                double *__restrict__ part) {
-  __shared__ double s[6][NT];
-  double v[6] = {HUGE_VAL, HUGE_VAL, HUGE_VAL, -HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT)
-    for (int d = 0; d < 3; ++d) {
-      const double x = pts[3 * i + d];
-      v[d] = fmin(v[d], x);
-      v[3 + d] = fmax(v[3 + d], x);
-    }
-  const double r = box_reduce(v, s);
-  if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = r;
-}
-
-// 63-bit Morton code of each point's place in the box (the nparts partial
-// boxes are reduced by every workgroup again: at most 64 of them), x in the
-// lowest bit of each triple
-__global__ void __launch_bounds__(NT) plan_keys(int64_t n, int nparts,
-                                                const double *__restrict__ pts,
-                                                const double *__restrict__ part,
-                                                uint64_t *__restrict__ key,
-                                                int *__restrict__ idx) {
-#pragma clang fp contract(off)
-  __shared__ double bb[6];
-  if (threadIdx.x < 6) {
-    double r = part[threadIdx.x];
-    for (int i = 1; i < nparts; ++i)
-      r = threadIdx.x < 3 ? fmin(r, part[6 * i + threadIdx.x]) : fmax(r, part[6 * i + threadIdx.x]);
-    bb[threadIdx.x] = r;
-  }
-  __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (i >= n) return;
-  uint64_t code = 0;
-  for (int d = 0; d < 3; ++d) {
-    const double ext = fmax(bb[3 + d] - bb[d], 1e-12);
-    const double t = fmin(fmax((pts[3 * i + d] - bb[d]) / ext, 0.0), 1.0);
-    code |= spread21((uint64_t)(t * 2097151.0)) << d;
-  }
-  key[i] = code;
-  idx[i] = (int)i;
-}
 
 // One wave per batch: its 64 points in sorted order (past the end: copies of
 // the last one, weight 0, index -1) and their box.
@@ -214,20 +145,20 @@ void vk_plan_points(hipStream_t s, PlanScratch &sc, int64_t npts, const double *
                     double *boxes) {
   NKX_REQUIRE(npts > 0 && npts < INT32_MAX, NKX_ERR_UNSUPPORTED,
               "a molecule's plan takes 1 .. 2^31 - 2 points");
-  const int nparts = (int)std::min<int64_t>(64, (npts + NT - 1) / NT);
+  const int nparts = (int)std::min<int64_t>(kBoxParts, (npts + NT - 1) / NT);
   size_t bytes = 0;
   NKX_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, (uint64_t *)nullptr,
                                                    (uint64_t *)nullptr, (int *)nullptr,
                                                    (int *)nullptr, (int)npts, 0, 63, s));
-  sc.part.reserve((size_t)6 * 64);
+  sc.part.reserve((size_t)6 * kBoxParts);
   sc.key.reserve((size_t)2 * npts);
   sc.idx.reserve((size_t)2 * npts);
   sc.tmp.reserve(bytes);
   uint64_t *k0 = sc.key.p, *k1 = k0 + npts;
   int *i0 = sc.idx.p, *i1 = i0 + npts;
-  hipLaunchKernelGGL(plan_bbox, dim3(nparts), dim3(NT), 0, s, npts, pts, sc.part.p);
-  hipLaunchKernelGGL(plan_keys, dim3(nblocks(npts)), dim3(NT), 0, s, npts, nparts, pts, sc.part.p,
-                     k0, i0);
+  hipLaunchKernelGGL(points_box, dim3(nparts), dim3(NT), 0, s, npts, pts, sc.part.p);
+  hipLaunchKernelGGL(points_keys<false>, dim3(nblocks(npts)), dim3(NT), 0, s, npts, nparts, pts,
+                     sc.part.p, k0, i0);
   NKX_HIP_CHECK(hipGetLastError());
   // stable: points with equal codes stay in the grid's order
   NKX_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(sc.tmp.p, bytes, k0, k1, i0, i1, (int)npts, 0,

@@ -5,6 +5,7 @@
 // own screening on 64-point batches and does not need these lists.
 #include <hipcub/hipcub.hpp>
 
+#include "morton.hpp"
 #include "nkx_internal.hpp"
 #include "vxc_kernels.hpp"
 
@@ -12,79 +13,7 @@ namespace nkx {
 
 namespace {
 
-constexpr int NT = 256;
-
-__device__ __forceinline__ uint64_t spread21(uint64_t v) {
-  v &= 0x1fffff;
-  v = (v | v << 32) & 0x1f00000000ffffull;
-  v = (v | v << 16) & 0x1f0000ff0000ffull;
-  v = (v | v << 8) & 0x100f00f00f00f00full;
-  v = (v | v << 4) & 0x10c30c30c30c30c3ull;
-  v = (v | v << 2) & 0x1249249249249249ull;
-  return v;
-}
-
-// Per-workgroup minimum and maximum of the points: part[6 g + (lo xyz, hi xyz)].
-__global__ void __launch_bounds__(NT) bbox_partial(int64_t n, const double *__restrict__ pts,
-                                                   double *__restrict__ part) {
-  __shared__ double s[6][NT];
-  double v[6] = {HUGE_VAL, HUGE_VAL, HUGE_VAL, -HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
-  for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * NT)
-    for (int d = 0; d < 3; ++d) {
-      const double x = pts[3 * i + d];
-      v[d] = fmin(v[d], x);
-      v[3 + d] = fmax(v[3 + d], x);
-    }
-  for (int k = 0; k < 6; ++k) s[k][threadIdx.x] = v[k];
-  __syncthreads();
-  for (int h = NT / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h)
-      for (int k = 0; k < 6; ++k) {
-        const double o = s[k][threadIdx.x + h];
-        s[k][threadIdx.x] = k < 3 ? fmin(s[k][threadIdx.x], o) : fmax(s[k][threadIdx.x], o);
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
-}
-
-// Reduces nparts partial boxes (one workgroup).
-__global__ void __launch_bounds__(NT) bbox_final(int nparts, const double *__restrict__ part,
-                                                 double *__restrict__ bb) {
-  __shared__ double s[6][NT];
-  double v[6] = {HUGE_VAL, HUGE_VAL, HUGE_VAL, -HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
-  for (int i = threadIdx.x; i < nparts; i += NT)
-    for (int k = 0; k < 6; ++k)
-      v[k] = k < 3 ? fmin(v[k], part[6 * i + k]) : fmax(v[k], part[6 * i + k]);
-  for (int k = 0; k < 6; ++k) s[k][threadIdx.x] = v[k];
-  __syncthreads();
-  for (int h = NT / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h)
-      for (int k = 0; k < 6; ++k) {
-        const double o = s[k][threadIdx.x + h];
-        s[k][threadIdx.x] = k < 3 ? fmin(s[k][threadIdx.x], o) : fmax(s[k][threadIdx.x], o);
-      }
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) bb[threadIdx.x] = s[threadIdx.x][0];
-}
-
-// 63-bit Morton code of each point: 21 bits per axis of its position in the
-// bounding box, x in the highest bit of each triple.
-__global__ void __launch_bounds__(NT) morton_keys(int64_t n, const double *__restrict__ pts,
-                                                  const double *__restrict__ bb,
-                                                  uint64_t *__restrict__ key, int *__restrict__ idx) {
-  const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (i >= n) return;
-  uint64_t code = 0;
-  for (int d = 0; d < 3; ++d) {
-    const double ext = fmax(bb[3 + d] - bb[d], 1e-12);
-    const double t = fmin(fmax((pts[3 * i + d] - bb[d]) / ext, 0.0), 1.0);
-    code |= spread21((uint64_t)(t * 2097151.0)) << (2 - d);
-  }
-  key[i] = code;
-  idx[i] = (int)i;
-}
+constexpr int NT = kBoxThreads;
 
 __global__ void __launch_bounds__(NT) permute_points(
     int64_t n, const int *__restrict__ perm, const double *__restrict__ pts,
@@ -234,9 +163,9 @@ void sparse_bounding_boxes(hipStream_t s, int64_t npts, double *pts, double *w, 
   if (npts <= 0) return;
   NKX_REQUIRE(npts < INT32_MAX && per > 0, NKX_ERR_INVALID_ARGUMENT,
               "bounding boxes: 0 < npts < 2^31 - 1 and max_points_per_box > 0");
-  const int nparts = (int)std::min<int64_t>(1024, (npts + NT - 1) / NT);
-  // scratch: partial boxes, the box, keys (2), indices (2), permuted copies
-  const size_t b_part = (size_t)6 * nparts * sizeof(double), b_bb = 6 * sizeof(double);
+  const int nparts = (int)std::min<int64_t>(kBoxParts, (npts + NT - 1) / NT);
+  // scratch: partial boxes, keys (2), indices (2), permuted copies
+  const size_t b_part = (size_t)6 * nparts * sizeof(double);
   const size_t b_key = (size_t)npts * sizeof(uint64_t), b_idx = (size_t)npts * sizeof(int);
   const size_t b_pts = (size_t)3 * npts * sizeof(double), b_w = (size_t)npts * sizeof(double);
   size_t b_tmp = 0;
@@ -244,7 +173,7 @@ void sparse_bounding_boxes(hipStream_t s, int64_t npts, double *pts, double *w, 
                                                    (uint64_t *)nullptr, (int *)nullptr,
                                                    (int *)nullptr, (int)npts, 0, 63, s));
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
-  const size_t total = up(b_part) + up(b_bb) + 2 * up(b_key) + 2 * up(b_idx) + up(b_pts) +
+  const size_t total = up(b_part) + 2 * up(b_key) + 2 * up(b_idx) + up(b_pts) +
                        up(b_w) + up(b_idx) + up(b_tmp);
   Scratch sc;
   NKX_HIP_CHECK(hipMalloc(&sc.p, total));
@@ -254,15 +183,16 @@ void sparse_bounding_boxes(hipStream_t s, int64_t npts, double *pts, double *w, 
     q += up(x);
     return r;
   };
-  double *part = (double *)take(b_part), *bb = (double *)take(b_bb);
+  double *part = (double *)take(b_part);
   uint64_t *k0 = (uint64_t *)take(b_key), *k1 = (uint64_t *)take(b_key);
   int *i0 = (int *)take(b_idx), *i1 = (int *)take(b_idx);
   double *pts2 = (double *)take(b_pts), *w2 = (double *)take(b_w);
   int *own2 = (int *)take(b_idx);
   void *tmp = take(b_tmp);
-  hipLaunchKernelGGL(bbox_partial, dim3(nparts), dim3(NT), 0, s, npts, pts, part);
-  hipLaunchKernelGGL(bbox_final, dim3(1), dim3(NT), 0, s, nparts, part, bb);
-  hipLaunchKernelGGL(morton_keys, dim3(nblocks(npts)), dim3(NT), 0, s, npts, pts, bb, k0, i0);
+  hipLaunchKernelGGL(points_box, dim3(nparts), dim3(NT), 0, s, npts, pts, part);
+  // x in the highest bit of each triple
+  hipLaunchKernelGGL(points_keys<true>, dim3(nblocks(npts)), dim3(NT), 0, s, npts, nparts, pts,
+                     part, k0, i0);
   NKX_HIP_CHECK(
       hipcub::DeviceRadixSort::SortPairs(tmp, b_tmp, k0, k1, i0, i1, (int)npts, 0, 63, s));
   hipLaunchKernelGGL(permute_points, dim3(nblocks(npts)), dim3(NT), 0, s, npts, i1, pts, w,

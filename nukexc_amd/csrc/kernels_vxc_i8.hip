@@ -1167,11 +1167,10 @@ void vkm_density(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_t s0, c
 
 // Second half of the density stage: per-batch functional from the slot
 // partial sums, then the Z slices of every slot.
-void vkm_density_finish(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_t s0,
+void vkm_density_finish(hipStream_t s, int64_t b0, int64_t b1, int64_t s0,
                         const Plan &pl, int gga, signed char *store, const XcList &xl,
                         double *coef, double *blockEN, const double *part) {
   if (b1 <= b0) return;
-  (void)shape;
   hipLaunchKernelGGL(density_f, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, s0, b0,
                      pl.b_off.p, gga, part, pl.pw.p, xl, coef, blockEN, nullptr, nullptr);
   NKX_HIP_CHECK(hipGetLastError());
@@ -1223,8 +1222,10 @@ void vkm_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl
   const signed char *zbase = zstore_b ? zstore_b : store + OFF_Z;
   const int64_t zstride = zstore_b ? (int64_t)SEC : slot_bytes_i8(gga);
   // all super-pairs of a split on one XCD where they fit its 32 CUs twice at
-  // most: 32 waters (28 super-pairs) 19.1 -> 17.8 ms; 100 waters (210) lose by it;
-  // and only where every XCD gets its share (a chain of 100 atoms, 36 super-pairs,
+  // most: 32 waters (28 super-pairs) 19.1 -> 17.8 ms.  On both sides of the line,
+  // grouped and not: 45 super-pairs (44 waters) 7.85 and 8.0 ms, 55 (50 waters)
+  // 10.9 and 10.7, 66 (56 waters) 14.8 and 14.9, 78 (61 waters) 19.7 and 18.0, 210
+  // (100 waters) 59.7 and 57.8.  And only where every XCD gets its share (a chain of 100 atoms, 36 super-pairs,
   // whole builds with 3 splits: 15.2 ms in plain order, 20.3 on three XCDs)
   const bool grouped = pl.nspairs <= 64 && (nsplit % 8 == 0 || nsplit >= 64);
   const int64_t ns = grouped ? (nsplit + 7) / 8 * 8 : nsplit, nwg = pl.nspairs * ns;

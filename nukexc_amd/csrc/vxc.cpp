@@ -20,6 +20,7 @@
 #include <numeric>
 #include <string>
 
+#include "morton.hpp"
 #include "nkx_internal.hpp"
 #include "vxc_kernels.hpp"
 
@@ -27,30 +28,9 @@ namespace nkx {
 
 namespace {
 
-uint64_t spread21(uint64_t v) {
-  v &= 0x1fffff;
-  v = (v | v << 32) & 0x1f00000000ffffull;
-  v = (v | v << 16) & 0x1f0000ff0000ffull;
-  v = (v | v << 8) & 0x100f00f00f00f00full;
-  v = (v | v << 4) & 0x10c30c30c30c30c3ull;
-  v = (v | v << 2) & 0x1249249249249249ull;
-  return v;
-}
-
 struct Box {
   double lo[3], hi[3];
 };
-
-uint64_t morton(const double *p, const Box &bb) {
-  uint64_t code = 0;
-  for (int d = 0; d < 3; ++d) {
-    const double ext = std::max(bb.hi[d] - bb.lo[d], 1e-12);
-    double t = (p[d] - bb.lo[d]) / ext;
-    t = std::min(std::max(t, 0.0), 1.0);
-    code |= spread21((uint64_t)(t * 2097151.0)) << d;
-  }
-  return code;
-}
 
 constexpr int FB = 64;
 constexpr int PT = 64;
@@ -67,7 +47,6 @@ struct PlanPart {
   std::vector<FuncRec> fr;
   std::vector<HarmTerm> terms;
   std::vector<double> fn;  // centre and screening radius per sorted function
-  std::vector<int> pair_I, pair_J;
 };
 
 // Functions of basis B in plan order, their records and screening radii.
@@ -108,7 +87,7 @@ PlanPart make_part(int64_t npts, const BasisHost &B, double tol) {
   for (int i = 0; i < nbf; ++i) {
     const double ctr[3] = {B.cx[i], B.cy[i], B.cz[i]};
     const int cls = (int)std::floor(2.0 * std::log2(std::max(rad[i], 0.25)));
-    fkey[i] = std::make_tuple(cls, morton(ctr, cb), i);
+    fkey[i] = std::make_tuple(cls, morton_code<false>(ctr, cb.lo, cb.hi), i);
   }
   std::sort(fkey.begin(), fkey.end());
   pt.fperm.resize(nbf);
@@ -418,7 +397,9 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
 // workgroup of a unit (super-pair; bf16, and FP64 where few super-pairs are whole:
 // pair) fits a CU at a time, so:
 //   one unit:  256 splits, one equal workgroup per CU (mixed benzene, 99 x 578
-//              points: 1536 us per build, 1617 with 320, 1608 with 335)
+//              points: 1536 us per build, 1617 with 320, 1608 with 335; FP64, V
+//              alone: benzene 179 us, 310 with 128, 190 with 512, a 12-atom
+//              molecule with two spins 155, 143 and 178)
 //   a few:     512 splits each (16- and 24-atom molecules: within 1 % of the
 //              best of 32 .. 1024)
 //   many:      about 8192 workgroups (FP64: 4096), the tail of unequal units
@@ -428,7 +409,8 @@ int64_t chunk_slot_budget(size_t slot_bytes, size_t cap) {
 //              64, 86.5 with 8
 // and never less than four batches per split (mixed water: 146 us with 4 to 5,
 // 179 with 32), or in a molecule set 16 (FP64: 8) of an average molecule (8
-// molecules, mixed: 2782 us, 2893 with 4).  FP64 with more workgroups than CUs: a
+// molecules, mixed: 2782 us, 2893 with 4; sets of 8, 64 and 20 molecules of 2 to 30
+// atoms are within 1, 2 and 1 % of the best of 1 .. 64, mixed 1, 4 and 1 %).  FP64 with more workgroups than CUs: a
 // multiple of eight, which vgemm_f64 deals to the XCDs evenly, where its partials
 // stay below 1 GB (by pairs 2 GB; 100 waters, 210 super-pairs: 176 ms with 24
 // splits, 179 with 20; a chain of 700 atoms by super-pairs 279 ms with 8, 320 with
@@ -572,8 +554,8 @@ static void fp64_functional(hipStream_t s, int nspin, int64_t b0, int64_t b1, in
                            epoint);
 }
 
-// Every launch of one build, stream-ordered, ending with the copy of the
-// (E, N_alpha, N_beta) triples of all molecules into en_dst (host).  No
+// Every launch of one build, stream-ordered; the last one writes the (E, N_alpha,
+// N_beta) triples of all molecules into en_dst (page-locked).  No
 // allocation, no memset, no synchronisation: the sequence can be captured.
 void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
                    const double *const *P, const XcList &xl, double *const *V,
@@ -642,7 +624,7 @@ void enqueue_build(Ctx &c, Workspace &ws, const Plan &pl, const BuildSetup &b,
                                ws.coef.p, ws.coef.p + (size_t)4 * pl.npts_pad, ws.blockEN.p,
                                ws.dpart.p, ws.dpart.p + (size_t)b.slots_alloc * 4 * PT);
       else
-        vkm_density_finish(s, b.group, b0, b1, s0, pl, ig, ws.mstore.p, xl, ws.coef.p,
+        vkm_density_finish(s, b0, b1, s0, pl, ig, ws.mstore.p, xl, ws.coef.p,
                            ws.blockEN.p, ws.dpart.p);
       tm.end(tt, s);
     }

@@ -103,7 +103,7 @@ bool mixed_density_shape_ok(int shape);
 void vkm_density(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_t s0, const Plan &pl,
                  const signed char *Ps, int gga, signed char *store, const XcList &xl,
                  double *coef, double *blockEN, double *part);
-void vkm_density_finish(hipStream_t s, int shape, int64_t b0, int64_t b1, int64_t s0,
+void vkm_density_finish(hipStream_t s, int64_t b0, int64_t b1, int64_t s0,
                         const Plan &pl, int gga, signed char *store, const XcList &xl,
                         double *coef, double *blockEN, const double *part);
 // per-batch reduction of part and the functional only (no Z slices), both
