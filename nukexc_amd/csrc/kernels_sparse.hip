@@ -163,9 +163,9 @@ void sparse_bounding_boxes(hipStream_t s, int64_t npts, double *pts, double *w, 
   if (npts <= 0) return;
   NKX_REQUIRE(npts < INT32_MAX && per > 0, NKX_ERR_INVALID_ARGUMENT,
               "bounding boxes: 0 < npts < 2^31 - 1 and max_points_per_box > 0");
-  const int nparts = (int)std::min<int64_t>(kBoxParts, (npts + NT - 1) / NT);
-  // scratch: partial boxes, keys (2), indices (2), permuted copies
-  const size_t b_part = (size_t)6 * nparts * sizeof(double);
+  const int nparts = (int)std::min<int64_t>(1024, (npts + NT - 1) / NT);
+  // scratch: partial boxes and the box, keys (2), indices (2), permuted copies
+  const size_t b_part = (size_t)6 * (nparts + 1) * sizeof(double);
   const size_t b_key = (size_t)npts * sizeof(uint64_t), b_idx = (size_t)npts * sizeof(int);
   const size_t b_pts = (size_t)3 * npts * sizeof(double), b_w = (size_t)npts * sizeof(double);
   size_t b_tmp = 0;
@@ -183,16 +183,17 @@ void sparse_bounding_boxes(hipStream_t s, int64_t npts, double *pts, double *w, 
     q += up(x);
     return r;
   };
-  double *part = (double *)take(b_part);
+  double *part = (double *)take(b_part), *bb = part + 6 * nparts;
   uint64_t *k0 = (uint64_t *)take(b_key), *k1 = (uint64_t *)take(b_key);
   int *i0 = (int *)take(b_idx), *i1 = (int *)take(b_idx);
   double *pts2 = (double *)take(b_pts), *w2 = (double *)take(b_w);
   int *own2 = (int *)take(b_idx);
   void *tmp = take(b_tmp);
   hipLaunchKernelGGL(points_box, dim3(nparts), dim3(NT), 0, s, npts, pts, part);
+  hipLaunchKernelGGL(points_box_final, dim3(1), dim3(NT), 0, s, nparts, part, bb);
   // x in the highest bit of each triple
-  hipLaunchKernelGGL(points_keys<true>, dim3(nblocks(npts)), dim3(NT), 0, s, npts, nparts, pts,
-                     part, k0, i0);
+  hipLaunchKernelGGL(points_keys<true>, dim3(nblocks(npts)), dim3(NT), 0, s, npts, 1, pts, bb, k0,
+                     i0);
   NKX_HIP_CHECK(
       hipcub::DeviceRadixSort::SortPairs(tmp, b_tmp, k0, k1, i0, i1, (int)npts, 0, 63, s));
   hipLaunchKernelGGL(permute_points, dim3(nblocks(npts)), dim3(NT), 0, s, npts, i1, pts, w,
