@@ -386,19 +386,23 @@ void launch_collocation_ref(hipStream_t s, int nbf, const FuncRec *f, const Harm
     return;
   }
   const int64_t nwg = (npts + 63) / 64;
-  // Small outputs, or few points: narrow tiles (FW 4, 2 below one workgroup per
-  // CU), each a workgroup of its own, for shorter chains and more waves in flight;
-  // the lines that two tiles share meet in the last-level cache (256 MB, shared
-  // with what else is held).  Larger ones: those lines would go to memory twice, so
-  // one workgroup writes all tiles of its points, 32 functions wide, where there
-  // are points for twelve workgroups a CU.  Both calls, us (FW 8 in a loop / FW 4
-  // each its own): 9 MB of output 72.3 / 69.6, 71 MB 96 / 83, 0.5 GB 269 / 308, 2.2
-  // GB 799 / 1246; the gradients of 3120 functions at 5 000 points 754 / 173, 1040
-  // at 40 000 377 / 264, 120 at 130 000 143 / 140, at 260 000 254 / 260, at 340 000
-  // 318 / 375; FW 2 at 4 MB 64.5 for 67.2.
+  // Small outputs: narrow tiles (FW 4, 2 below one workgroup per CU), each a
+  // workgroup of its own, for shorter chains and more waves in flight; the lines
+  // that two tiles share meet in the last-level cache (256 MB, shared with what
+  // else is held).  Larger ones: those lines would go to memory twice, so tiles are
+  // 32 functions wide and one workgroup writes all of its points' tiles, or where
+  // that makes fewer than 2048 workgroups (eight a CU) every ny-th of them.  Both
+  // calls, us (FW 8 in a loop / FW 4 each its own): 9 MB of output 72.3 / 69.6, 71
+  // MB 96 / 83, 0.5 GB 269 / 308, 2.2 GB 799 / 1246; FW 2 at 4 MB 64.5 for 67.2.
+  // Values and gradients, us (one workgroup / ny by 2048 / a workgroup each tile / FW
+  // 4 each its own): 1200 functions at 3 840 points 585 / 213 / 206 / 191, 400 at 28
+  // 800 262 / 197 / 183 / 168, 110 at 62 370 155 / 150 / 154 / 168, 110 at 176 418
+  // 319 / 320 / 338 / 398.
   const int64_t bytes = (int64_t)8 * nbf * npts * ((phi ? 1 : 0) + (gx ? 3 : 0));
-  const int fw = bytes <= ((int64_t)1 << 26) ? (nwg < 256 ? 2 : 4) : (nwg < 12 * 256 ? 4 : 8);
-  const unsigned ny = fw == 8 ? 1 : (unsigned)((nbf + 4 * fw - 1) / (4 * fw));
+  const int fw = bytes > ((int64_t)1 << 26) ? 8 : nwg < 256 ? 2 : 4;
+  const int64_t tiles = (nbf + 4 * fw - 1) / (4 * fw);
+  const unsigned ny =
+      (unsigned)(fw == 8 ? std::min<int64_t>(tiles, std::max<int64_t>(1, 2048 / nwg)) : tiles);
 #define NKX_COLLOC_FW(V, G, W)                                                              \
   hipLaunchKernelGGL((colloc_ref_kernel<V, G, W>), dim3((unsigned)nwg, ny), dim3(256), 0, s, \
                      nbf, f, t, npts, pts, phi, gx, gy, gz)

@@ -86,8 +86,8 @@ __global__ void __launch_bounds__(256) colloc_tiles_f64(
 // pieces of an LDS row are exchanged by bits 1 .. 3 of the row, so that sixteen
 // rows fall on sixteen different bank groups.
 //
-// Bound by the FP64 MFMA rate (busy 70 % of the cycles; the rest is the wait at
-// a stage's start, one workgroup per CU): 16 waters take 7.9 ms, 52 TFLOP/s,
+// Bound by the FP64 MFMA rate (busy 67 % of the cycles on 100 waters; the rest is
+// the wait at a stage's start, one workgroup per CU): 16 waters take 7.9 ms, 52 TFLOP/s,
 // a 12-atom molecule with two spins 341 us, water 24 us (8.5 ms, 361 us and 27 us
 // with each stage's slots looked up in LDS between its barrier and its copies).  One workgroup per
 // block pair, both products on the diagonal too, read four tiles for every two

@@ -1,7 +1,7 @@
 """Reference-shaped collocation on both sides of the borders between its tile
-shapes (64 MB of output, 256 and 3072 groups of 64 points), values and
-gradients, against the same points in pieces of 4 000, which take the narrowest
-tiles: the same bits."""
+shapes (64 MB of output, 256 groups of 64 points) and between numbers of
+workgroups to a group (2048 over the groups), values and gradients, against the
+same points in pieces of 4 000, which take the narrowest tiles: the same bits."""
 import numpy as np
 import pytest
 
@@ -11,8 +11,9 @@ pytestmark = pytest.mark.gpu
 import nukexc_amd as nk  # noqa: E402
 
 
-@pytest.mark.parametrize("nbf,npts", [(3100, 4100), (1037, 10000), (1037, 8000), (120, 196544),
-                                      (120, 196608), (120, 196609), (61, 150000), (45, 200001)])
+@pytest.mark.parametrize("nbf,npts", [(3100, 4100), (1037, 10000), (1037, 8000), (120, 65536),
+                                      (120, 65537), (120, 131072), (120, 131073), (61, 150000),
+                                      (45, 200001)])
 def test_pieces(nbf, npts):
     rng = np.random.default_rng(nbf)
     f = []
