@@ -224,8 +224,6 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
       const int64_t n = cnt & 0xffff, f = cnt >> 17, last = (cnt >> 16) & 1;
       nslots += n;
       max_live = std::max(max_live, n);
-      NKX_REQUIRE(nslots < (int64_t)INT32_MAX, NKX_ERR_UNSUPPORTED,
-                  "too many live (block, batch) pairs for 32-bit slot numbers");
       // algorithmic work: true functions of the live blocks, true points
       const double nfun = host[2 * gb + 1];
       const double g = (double)std::min<int64_t>(PT, parts[m].npts - b * PT);
@@ -237,6 +235,8 @@ void build_plan(Ctx &c, Plan &pl, const std::vector<MolPoints> &mols,
       by_pair += n * (100 * (n - 1) + 110);
       by_super += f * (265 * (f - 1) + 300) + last * (340 * f + 110);
     }
+  NKX_REQUIRE(nslots < (int64_t)INT32_MAX, NKX_ERR_UNSUPPORTED,
+              "too many live (block, batch) pairs for 32-bit slot numbers");
   pl.b_off_h[nb] = (int)nslots;
   pl.b_off.upload(pl.b_off_h.data(), pl.b_off_h.size(), s);
   pl.b_fbl.reserve(std::max<int64_t>(nslots, 1));
