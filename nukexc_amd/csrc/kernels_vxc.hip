@@ -522,13 +522,22 @@ void vk_zoverlap(hipStream_t s, int64_t s0, int64_t s1, const Plan &pl, int narr
 void vk_vgemm(hipStream_t s, int64_t b0, int64_t b1, int64_t s0, const Plan &pl, int nsplit,
               int narr, int nz, bool first, const double *tiles, double *vpart) {
   if (b1 <= b0 || pl.nspairs == 0) return;
-  const int nsp = pl.v_by_pair ? pl.npairs : pl.nspairs;
+  // Where the super-pairs do not fill the CUs once, pairs that take fewer rounds for
+  // their size (a super-pair 2.65 pairs, 1.5 on the diagonal, 1.7 beside a single
+  // block): 40 atoms (10 super-pairs, 28 pairs) with 8 splits 2.8 ms by pairs and 7.2
+  // by super-pairs, with 16 2.9 and 3.6, with 24 2.8 and 2.4; benzene (1 and 3) with
+  // 64 464 us and 579, with 96 465 and 401.
+  bool by_pair = pl.v_by_pair;
+  const int64_t ks = (int64_t)pl.nspairs * nsplit * nz, kp = (int64_t)pl.npairs * nsplit * nz;
+  if (!by_pair && pl.npairs > pl.nspairs && ks <= 256)
+    by_pair = (kp + 255) / 256 < (pl.max_mol_nfb <= 2 ? 1.5 : pl.max_mol_nfb == 3 ? 1.7 : 2.65);
+  const int nsp = by_pair ? pl.npairs : pl.nspairs;
   const int64_t nwg = (int64_t)nsp * nsplit * nz;
   NKX_REQUIRE(nwg <= max_workgroups(512), NKX_ERR_UNSUPPORTED, "V contraction grid too large");
   // other numbers of splits leave XCDs with fewer of them than others, or none
   const int grouped = nsplit % 8 == 0;
   hipLaunchKernelGGL(vgemm_f64, dim3((unsigned)nwg), dim3(512), 0, s, nsp, nsplit, grouped,
-                     reinterpret_cast<const int4 *>(pl.v_by_pair ? nullptr : pl.sp_blk.p),
+                     reinterpret_cast<const int4 *>(by_pair ? nullptr : pl.sp_blk.p),
                      reinterpret_cast<const int4 *>(pl.sp_pidx.p), pl.pair_I.p, pl.pair_J.p,
                      pl.npairs, pl.tile_slot.p, pl.tab(), b0, b1, s0, narr, narr - nz,
                      first ? 1 : 0, tiles, vpart);

@@ -47,7 +47,7 @@ def _near(V, ref):
 
 
 @pytest.mark.parametrize("budget", [0, 64 << 20])
-@pytest.mark.parametrize("split", [0, 1, 3, 8, 13, 64])
+@pytest.mark.parametrize("split", [0, 1, 3, 8, 13, 25, 64])
 def test_split_counts(case, split, budget):
     c, P, closed, opened = case
     print(f"split {split}, budget {budget}, {c.plan_stats()}", flush=True)
